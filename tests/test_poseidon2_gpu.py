@@ -176,3 +176,47 @@ def test_bad_arguments(ba, rc):
     finally:
         v.free()
         r.free()
+
+
+# Up to 65536 digests run on quads of threads, more on one thread each; 64 quads or 256 threads a block.
+@pytest.mark.parametrize("count", [63, 64, 65, 65535, 65536, 65537, 65536 + 257])
+def test_nodes_either_side_of_the_quad_rule(ba, rc, count):
+    rng = np.random.default_rng(count)
+    values = raw_u64(rng, 8 * count)
+    edges = np.array([0, 1, 0xFFFFFFFF, 0x100000000, gl_oracle.P - 1, gl_oracle.P, 2**64 - 1], dtype=np.uint64)
+    values[:: 3] = rng.choice(edges, values[:: 3].size)
+    want = gl_oracle.poseidon2_nodes(values, count, rc)
+    d_v, d_r = ba.DeviceAllocation.from_host(values), ba.DeviceAllocation(4 * count)
+    try:
+        log(f"poseidon2 nodes count={count}")
+        ba.poseidon2.compute_node_hashes(d_v, d_r)
+        ba.synchronize()
+        assert np.array_equal(d_r.to_host(), want)
+    finally:
+        d_v.free()
+        d_r.free()
+
+
+@pytest.mark.parametrize("log_rows,cols,count", [(0, 11, 65537), (1, 6, 66000), (2, 2, 70001), (2, 3, 61), (3, 3, 65)])
+def test_leaves_either_side_of_the_quad_rule(ba, rc, log_rows, cols, count):
+    """Both kernels' absorption, with the first columns' capacity stored and loaded again."""
+    rows = 1 << log_rows
+    values = raw_u64(np.random.default_rng(cols), rows * cols * count)
+    want = gl_oracle.poseidon2_leaves(values, rows, cols, count, rc)
+    d_v, d_r = ba.DeviceAllocation.from_host(values), ba.DeviceAllocation(4 * count)
+    try:
+        log(f"poseidon2 leaves rows={rows} cols={cols} count={count}")
+        ba.poseidon2.compute_leaf_hashes(d_v, d_r, log_rows)
+        ba.synchronize()
+        assert np.array_equal(d_r.to_host(), want)
+        first = max(1, 8 // rows)  # the columns of the first chunk
+        if first < cols and rows * first % 8 == 0:
+            head = d_v.sub(0, first * rows * count)
+            tail = d_v.sub(first * rows * count, (cols - first) * rows * count)
+            ba.poseidon2.compute_leaf_hashes(head, d_r, log_rows, store_intermediate=True)
+            ba.poseidon2.compute_leaf_hashes(tail, d_r, log_rows, load_intermediate=True)
+            ba.synchronize()
+            assert np.array_equal(d_r.to_host(), want)
+    finally:
+        d_v.free()
+        d_r.free()

@@ -132,6 +132,13 @@ __device__ __forceinline__ u64 minus_eps(u32 x0, u32 x1, u64 m) {
   return pack(r0, subb0(x1, m & ~k));
 }
 
+// 1 in the lanes of m, else 0
+__device__ __forceinline__ u32 one_if(u64 m) {
+  u32 r;
+  asm("v_cndmask_b32_e64 %0, 0, 1, %1" : "=v"(r) : "s"(m));
+  return r;
+}
+
 }  // namespace isa
 
 // a, b < p: canonical a + b.  s = a + b with carry c; when c, s + EPS (= a + b - p < p); when
@@ -222,6 +229,35 @@ __device__ __forceinline__ u64 mul(u64 a, u64 b) {
   const u32 r2 = addc(lo(w), hi(y), k1, k2);
   const u32 r3 = addc0(hi(w), k2, dead);
   return reduce3b(pack(lo(z), r1), r2, r3, cy);
+}
+
+// a, b any u64; result a lazy residue (any u64).  The words r0..r3 and cy as in mul:
+//   t = [r0, r1] - r3 - cy; a borrow selects t - EPS (t > 2^64 - 2^32, no wrap);
+//   R = r2 EPS + t; a carry selects R + EPS (R < r2 EPS <= (2^32 - 1)^2, no wrap).
+// 14 VALU, and two scalar mask operations where mul has six.
+__device__ __forceinline__ u64 mul_lazy(u64 a, u64 b) {
+  using namespace isa;
+  u64 cy, k1, k2, b1, bw, c, dead;
+  const u64 z = (u64)lo(a) * lo(b);
+  const u64 x = (u64)hi(a) * lo(b);
+  const u64 y = mad(lo(a), hi(b), x, cy);
+  const u64 w = (u64)hi(a) * hi(b);
+  const u32 r1 = add_co(hi(z), lo(y), k1);
+  const u32 r2 = addc(lo(w), hi(y), k1, k2);
+  const u32 r3 = addc0(hi(w), k2, dead);
+  const u32 t0 = subb(lo(z), r3, cy, b1);
+  const u32 t1 = subb0(r1, b1, bw);
+  const u64 R = mad_eps(r2, minus_eps(t0, t1, bw), c);
+  return (u64)one_if(c) * (u32)EPS + R;
+}
+
+// a any u64, b < p; lazy a + b: a carry selects s + EPS (s < p - 1 then, no wrap).  4 VALU.
+__device__ __forceinline__ u64 add_lazy(u64 a, u64 b) {
+  using namespace isa;
+  u64 c, c2, dead;
+  const u32 s0 = add_co(lo(a), lo(b), c);
+  const u32 s1 = addc(hi(a), hi(b), c, c2);
+  return mad_eps(one_if(c2), pack(s0, s1), dead);
 }
 
 __device__ __forceinline__ u64 sqr(u64 a) { return mul(a, a); }
