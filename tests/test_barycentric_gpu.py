@@ -128,3 +128,45 @@ def test_bad_arguments(ba):
             ba.barycentric.batch_eval_temp_elems(3, 16, 1)
     finally:
         d.free()
+
+
+# The evaluation kernel's column groups (1, 2, 4 and 8 columns a workgroup, with a shorter last group)
+# on one and on several chunks of 4096 rows, and short columns whose lanes run past the end.
+@pytest.mark.parametrize("kind", [0, 1, 2])
+@pytest.mark.parametrize("log_count,num_polys", [(9, 11), (12, 1200), (13, 500), (14, 259), (16, 100), (16, 301)])
+def test_batch_eval_column_groups(ba, kind, log_count, num_polys):
+    if kind == 2:
+        num_polys = num_polys // 2 + 1
+    rng = np.random.default_rng(100 * kind + log_count)
+    count, ext = 1 << log_count, kind != 0
+    # any coefficients: the largest words, whose products carry everywhere, among random ones
+    coeffs = raw_u64(rng, count * (2 if ext else 1)) % np.uint64(P)
+    ys = raw_u64(rng, count * num_polys * (2 if kind == 2 else 1))
+    coeffs[: count // 2] = P - 1
+    ys[::2] = P - 1
+    want = gl_oracle.barycentric_eval(kind, ys, count, num_polys, coeffs)
+    temp_n = ba.barycentric.batch_eval_temp_elems(kind, count, num_polys)
+    d_ys, d_l = ba.DeviceAllocation.from_host(ys), ba.DeviceAllocation.from_host(coeffs)
+    d_t, d_e = ba.DeviceAllocation(temp_n), ba.DeviceAllocation(len(want))
+    try:
+        log(f"batch_eval kind={kind} log_count={log_count} polys={num_polys}")
+        ba.barycentric.batch_eval(kind, d_ys, count, num_polys, d_l, d_t, d_e)
+        ba.synchronize()
+        assert np.array_equal(d_e.to_host(), want)
+    finally:
+        for t in (d_ys, d_l, d_t, d_e):
+            t.free()
+
+
+@pytest.mark.parametrize("ext", [False, True])
+@pytest.mark.parametrize("log_count", [0, 7, 8, 9, 10, 12])
+def test_coeffs_at_edge_points(ba, ext, log_count):
+    """X = 0, 1 and -1, X on the domain (common factor 0, so every coefficient is 0), several shifts."""
+    count, w = 1 << log_count, pow(0x7E9BD009B86A0845, 1 << (30 - log_count), P)
+    for coset in (1, 7, P - 1):
+        for x0 in (0, 1, P - 1, coset, coset * pow(w, count // 3, P) % P):
+            for x1 in ((0, 5) if ext else (None,)):
+                x = (x0, x1) if ext else x0
+                for bitrev in (False, True):
+                    want = gl_oracle.barycentric_coeffs(x, coset, count, bitrev, ext=ext)
+                    assert np.array_equal(gpu_coeffs(ba, x, coset, count, bitrev, ext), want), (coset, x, bitrev)

@@ -10,19 +10,19 @@
 // 2 k count; extension results are interleaved (c0, c1) per polynomial.
 //
 // Kernels:
-//  * coefficients: each lane takes 8 elements (grid-strided), forms X w^-i - c from the inverse
-//    power table and inverts the 8 at once (one field inversion and 3 multiplies per element,
-//    Montgomery's trick), as the reference batches its inversions per thread;
-//  * batch evaluation: a grid over (row chunks of 4096, column groups), each lane 16 rows of a
-//    column, coefficients kept in registers across the columns of its group, a wave-level
-//    reduction through LDS, one partial sum per (chunk, column); a second kernel sums the chunks.
-// Both are HBM-bound for base-field data (8 B per element read once) and VALU-bound for
-// extension-field products.
+//  * coefficients: each lane takes up to 8 elements, forms the denominators from the inverse power
+//    table and inverts their 8 base-field norms at once (one field inversion and 3 multiplies per
+//    element, Montgomery's trick), writing natural or bit-reversed order directly;
+//  * batch evaluation: a grid over (row chunks of 4096, column groups), each lane 8 rows of a column
+//    with their coefficients in registers across the columns of its group, exact sums of products
+//    reduced once per column, one partial sum per (chunk, column); a second kernel, one wave per
+//    column, sums the chunks.
 #include <algorithm>
 #include <mutex>
 #include <vector>
 
 #include "api_internal.h"
+#include "gl_host.h"
 
 namespace {
 
@@ -32,212 +32,276 @@ using gl::u64;
 struct Ext {
   u64 a, b;
 };
-__device__ __forceinline__ Ext ext_add(const Ext &x, const Ext &y) { return {gl::add(x.a, y.a), gl::add(x.b, y.b)}; }
-__device__ __forceinline__ Ext ext_sub(const Ext &x, const Ext &y) { return {gl::sub(x.a, y.a), gl::sub(x.b, y.b)}; }
-__device__ __forceinline__ Ext ext_mul(const Ext &x, const Ext &y) {
-  const u64 ac = gl::mul(x.a, y.a), bd = gl::mul(x.b, y.b);
-  const u64 ad = gl::mul(x.a, y.b), bc = gl::mul(x.b, y.a);
-  return {gl::add(ac, gl::mul(bd, 7)), gl::add(ad, bc)};
-}
-__device__ __forceinline__ Ext ext_scale(const Ext &x, u64 s) { return {gl::mul(x.a, s), gl::mul(x.b, s)}; }
-__device__ __forceinline__ Ext ext_pow(Ext x, u64 e) {
-  Ext r{1, 0};
-  while (e) {
-    if (e & 1) r = ext_mul(r, x);
-    e >>= 1;
-    if (e) x = ext_mul(x, x);
-  }
-  return r;
-}
-// (a + b u)^-1 = (a - b u) / (a^2 - 7 b^2); 0 maps to 0
-__device__ __forceinline__ Ext ext_inv(const Ext &x) {
-  const u64 norm = gl::sub(gl::sqr(x.a), gl::mul(gl::sqr(x.b), 7));
-  const u64 ni = gl::inv(norm);
-  return {gl::mul(x.a, ni), gl::neg(gl::mul(x.b, ni))};
-}
-
-// Field traits: base field (u64) or extension (Ext) element operations
-template <bool EXT>
-struct F;
-template <>
-struct F<false> {
-  typedef u64 T;
-  static __device__ __forceinline__ T one() { return 1; }
-  static __device__ __forceinline__ T zero() { return 0; }
-  static __device__ __forceinline__ T mul(const T &x, const T &y) { return gl::mul(x, y); }
-  static __device__ __forceinline__ T add(const T &x, const T &y) { return gl::add(x, y); }
-  static __device__ __forceinline__ T sub(const T &x, const T &y) { return gl::sub(x, y); }
-  static __device__ __forceinline__ T scale(const T &x, u64 s) { return gl::mul(x, s); }
-  static __device__ __forceinline__ T inv(const T &x) { return gl::inv(x); }
-  static __device__ __forceinline__ T pow(const T &x, u64 e) { return gl::pow_u64(x, e); }
-  static __device__ __forceinline__ T from_base(u64 c) { return c; }
-  static __device__ __forceinline__ T load(const u64 *p, u64 i, u64) { return gl::canon(p[i]); }
-  static __device__ __forceinline__ void store(u64 *p, u64 i, u64, const T &v) { p[i] = v; }
-};
-template <>
-struct F<true> {
-  typedef Ext T;
-  static __device__ __forceinline__ T one() { return {1, 0}; }
-  static __device__ __forceinline__ T zero() { return {0, 0}; }
-  static __device__ __forceinline__ T mul(const T &x, const T &y) { return ext_mul(x, y); }
-  static __device__ __forceinline__ T add(const T &x, const T &y) { return ext_add(x, y); }
-  static __device__ __forceinline__ T sub(const T &x, const T &y) { return ext_sub(x, y); }
-  static __device__ __forceinline__ T scale(const T &x, u64 s) { return ext_scale(x, s); }
-  static __device__ __forceinline__ T inv(const T &x) { return ext_inv(x); }
-  static __device__ __forceinline__ T pow(const T &x, u64 e) { return ext_pow(x, e); }
-  static __device__ __forceinline__ T from_base(u64 c) { return {c, 0}; }
-  // element i of a two-plane vector whose planes are `plane` apart
-  static __device__ __forceinline__ T load(const u64 *p, u64 i, u64 plane) {
-    return {gl::canon(p[i]), gl::canon(p[i + plane])};
-  }
-  static __device__ __forceinline__ void store(u64 *p, u64 i, u64 plane, const T &v) {
-    p[i] = v.a;
-    p[i + plane] = v.b;
-  }
-};
-
-// common = c (X^N - c^N) / (N c^N)   (one lane)
-template <bool EXT>
-__global__ void common_factor_kernel(const u64 *x_ptr, u64 *common, u64 coset, u32 count) {
-  typedef F<EXT> Fx;
-  if (blockIdx.x | threadIdx.x) return;
-  const typename Fx::T x = Fx::load(x_ptr, 0, 1);
-  const u64 c = gl::canon(coset);
-  const u64 cn = gl::pow_u64(c, count);
-  const typename Fx::T num = Fx::scale(Fx::sub(Fx::pow(x, count), Fx::from_base(cn)), c);
-  const u64 den_inv = gl::inv(gl::mul(count % gl::P, cn));
-  Fx::store(common, 0, 1, Fx::scale(num, den_inv));
-}
 
 constexpr u32 kThreads = 256;
-constexpr int kInvBatch = 8;
+constexpr u32 kLogInvBatch = 3;
 
-// L_i = common / (X w^-i - c): each lane takes kInvBatch elements i = lane + k * stride and
-// inverts their product once
+// Coefficients L_i = common / (X w^-i - c), common = (X^N - c^N) scale with scale = c / (N c^N) from
+// the host; lane t of 2^log_t takes the 2^log_k elements at positions t + m 2^log_t.  The lane's
+// natural indices are an arithmetic progression in both orders (bit-reversed: the low log_k bits of
+// the index are the reversed m), so one table read and a constant step give all its powers of w.
+// At an extension point X = a + b u the norm of X w^-i - c = (a w - c) + b w u (w short for w^-i) is
+// w (w (a^2 - 7 b^2) - 2 a c) + c^2, in the base field: only norms are inverted, and
+//   L_i = (w A - B + (w C - D) u) / norm,  A = e a - 7 f b, B = e c, C = f a - e b, D = f c,  common = e + f u.
+// (A zero norm needs X on the domain, and then common = 0.)
+// What bounds it: VALU issue, per lane ~170 instructions per extension element, ~1.0 k for the
+// inversion and ~1.1 k for X^N.  One launch: 2^20 extension coefficients in bit-reversed order take
+// 33 us, base-field ones 16 us; a one-lane kernel for the common factor, extension-field inversions
+// and a separate bit reverse took 83 and 59 us.
 template <bool EXT>
-__global__ __launch_bounds__(kThreads) void coeffs_kernel(gl::Tables tab, const u64 *x_ptr, const u64 *common_ptr,
-                                                          u64 coset, u32 log_count, u64 *coeffs) {
-  typedef F<EXT> Fx;
-  typedef typename Fx::T T;
-  const u64 count = 1ull << log_count;
-  const u64 stride = (u64)gridDim.x * kThreads;
-  const u64 i0 = (u64)blockIdx.x * kThreads + threadIdx.x;
-  if (i0 >= count) return;
-  const T x = Fx::load(x_ptr, 0, 1);
-  const T common = Fx::load(common_ptr, 0, 1);
-  const u64 c = gl::canon(coset);
+__global__ __launch_bounds__(kThreads) void coeffs_kernel(gl::Tables tab, const u64 *x_ptr, u64 *common_ptr, u64 c,
+                                                          u64 cn, u64 scale, u32 log_count, u32 log_k,
+                                                          bool bit_reverse, u64 *coeffs) {
+  constexpr int K = 1 << kLogInvBatch;
+  const u32 log_t = log_count - log_k;
+  const u32 t = blockIdx.x * kThreads + threadIdx.x;
+  if (t >> log_t) return;
+  const u64 a = gl::canon(x_ptr[0]), b = EXT ? gl::canon(x_ptr[1]) : 0;
+  // the lane's first index and index step
   const u32 shift = gl::OMEGA_LOG_ORDER - log_count;
-  T den[kInvBatch], pre[kInvBatch];
-  T run = Fx::one();
-  int n = 0;
-  for (int k = 0; k < kInvBatch; k++) {
-    const u64 i = i0 + k * stride;
-    if (i >= count) break;
-    const u64 w_inv = gl::pow_w(tab, (u32)i << shift, true);
-    den[k] = Fx::sub(Fx::scale(x, w_inv), Fx::from_base(c));
-    pre[k] = run;  // product of den[0..k)
-    run = Fx::mul(run, den[k]);
-    n = k + 1;
+  const u32 i0 = bit_reverse ? gl::ntt::bitrev32(t, log_t) << log_k : t;
+  const u64 step = gl::pow_w(tab, (bit_reverse ? 1u : 1u << log_t) << shift, true);
+  u64 w[K], den[K], pre[K];
+  w[0] = gl::pow_w(tab, i0 << shift, true);
+  u64 alpha = 0, beta = 0, gamma = 0;
+  if constexpr (EXT) {
+    alpha = gl::sub(gl::sqr(a), gl::mul(gl::sqr(b), 7));
+    beta = gl::mul(gl::add(a, a), c);
+    gamma = gl::sqr(c);
   }
-  T inv = Fx::mul(Fx::inv(run), common);  // common / prod
-  for (int k = n - 1; k >= 0; k--) {
-    Fx::store(coeffs, i0 + k * stride, count, Fx::mul(inv, pre[k]));  // common / den[k]
-    inv = Fx::mul(inv, den[k]);
+  u64 run = 1;
+#pragma unroll
+  for (int j = 0; j < K; j++) {
+    if (j >> log_k) break;
+    if (j) w[j] = gl::mul_lazy(w[j ? j - 1 : 0], step);
+    // lazy: a lazy value minus, or plus, a canonical one stays a u64 residue
+    den[j] = EXT ? gl::add_lazy(gl::mul_lazy(w[j], gl::sub(gl::mul_lazy(w[j], alpha), beta)), gamma)
+                 : gl::sub(gl::mul_lazy(a, w[j]), c);
+    pre[j] = run;  // product of den[0..j)
+    run = gl::mul_lazy(run, den[j]);
+  }
+  u64 inv = gl::inv(run);
+  // X^N and the common factor
+  u64 e = a, f = b;
+#pragma unroll 1
+  for (u32 k = 0; k < log_count; k++) {
+    if constexpr (EXT) {  // (e^2 + 7 f^2, 2 e f) on the words of the products
+      using namespace gl::isa;
+      const u64 ee = gl::mul_lazy(e, e), ff = gl::mul_lazy(f, f), ef = gl::mul_lazy(e, f);
+      e = gl::fold_words((u64)lo(ff) * 7 + lo(ee), (u64)hi(ff) * 7 + hi(ee));
+      f = gl::fold_words((u64)lo(ef) * 2, (u64)hi(ef) * 2);
+    } else {
+      e = gl::mul_lazy(e, e);
+    }
+  }
+  e = gl::mul(gl::sub(gl::reduce1(e), cn), scale);
+  f = gl::mul(f, scale);
+  if (t == 0) {
+    common_ptr[0] = e;
+    if (EXT) common_ptr[1] = f;
+  }
+  u64 A = 0, B = 0, C = 0, D = 0;
+  if constexpr (EXT) {
+    A = gl::sub(gl::mul(e, a), gl::mul(gl::mul(f, b), 7));
+    B = gl::mul(e, c);
+    C = gl::sub(gl::mul(f, a), gl::mul(e, b));
+    D = gl::mul(f, c);
+  } else {
+    inv = gl::mul(inv, e);
+  }
+#pragma unroll
+  for (int j = K - 1; j >= 0; j--) {
+    if (j >> log_k) continue;
+    // 1 / den[j] (times common at a base point)
+    const u64 v = EXT ? gl::mul_lazy(inv, pre[j]) : gl::mul(inv, pre[j]);
+    const u32 m = bit_reverse ? gl::ntt::bitrev32(j, log_k) : j;
+    u64 *out = coeffs + (t + (m << log_t));
+    if constexpr (EXT) {
+      out[0] = gl::mul(gl::sub(gl::mul_lazy(w[j], A), B), v);
+      out[1ull << log_count] = gl::mul(gl::sub(gl::mul_lazy(w[j], C), D), v);
+    } else {
+      out[0] = v;
+    }
+    inv = gl::mul_lazy(inv, den[j]);
   }
 }
 
-constexpr int kRows = 16;                        // rows per lane per column
-constexpr u32 kChunk = kThreads * kRows;         // rows per workgroup
-constexpr u32 kColsPerGroup = 8;                 // columns a workgroup visits
+// ---------------------------------------------------------------- batch evaluation
+constexpr u32 kEvalThreads = 512;
+constexpr int kRows = 8;                           // rows per lane per column
+constexpr u32 kChunk = kEvalThreads * kRows;       // rows per workgroup
+constexpr u32 kColsPerGroup = 8;                   // most columns a workgroup visits
 
-// partial[chunk, col] = sum over the chunk's rows of L_row * y[row, col]
+// An exact sum of up to 2^16 products of u64 values: the partial products of equal weight (1, 2^32,
+// 2^64) are summed in 64 bits with a count of the carries.  8 VALU per product, where a reduced
+// product and a field addition take 20.
+struct ProductSum {
+  u64 z = 0, m = 0, w = 0;
+  u32 cz = 0, cm = 0, cw = 0;
+  __device__ __forceinline__ void add(u64 x, u64 y) {
+    using namespace gl::isa;
+    u64 c;
+    z = mad(lo(x), lo(y), z, c);
+    cz = addc0(cz, c);
+    m = mad(hi(x), lo(y), m, c);
+    cm = addc0(cm, c);
+    m = mad(lo(x), hi(y), m, c);
+    cm = addc0(cm, c);
+    w = mad(hi(x), hi(y), w, c);
+    cw = addc0(cw, c);
+  }
+  // The sum as a lazy residue: words r0..r4 with r4 < 2^17, reduced as [r0, r1] - [r3, r4] + r2 EPS
+  // (2^64 = EPS, 2^96 = -1, 2^128 = -2^32); the borrow selects t - EPS (t > 2^64 - 2^50, no wrap),
+  // the carry R + EPS (R < r2 EPS, no wrap).
+  __device__ __forceinline__ u64 value() const {
+    using namespace gl::isa;
+    u64 k, b, c, dead;
+    const u32 r1 = add_co(hi(z), lo(m), k);
+    u32 r2 = addc(lo(w), hi(m), k, k);
+    u32 r3 = addc0(hi(w), k, k);
+    u32 r4 = addc0(cw, k);
+    r2 = add_co(r2, cz, k);
+    r3 = addc(r3, cm, k, k);
+    r4 = addc0(r4, k);
+    const u32 t0 = sub_co(lo(z), r3, b);
+    const u32 t1 = subb(r1, r4, b, b);
+    const u64 r = mad_eps(r2, minus_eps(t0, t1, b), c);
+    return mad_eps(one_if(c), r, dead);
+  }
+};
+
+// A residue cut into limbs of 22, 22 and 20 bits, so that sums over lanes are plain 32-bit additions.
+struct Limbs {
+  u32 l[3];
+};
+__device__ __forceinline__ Limbs limbs_of(u64 x) {
+  return {{(u32)x & 0x3FFFFFu, (u32)(x >> 22) & 0x3FFFFFu, (u32)(x >> 44)}};
+}
+// l0 + l1 2^22 + l2 2^44, canonical
+__device__ __forceinline__ u64 joined(const Limbs &v) {
+  return gl::reduce1(gl::fold_words(v.l[0] + ((u64)v.l[1] << 22), (u64)v.l[2] << 12));
+}
+
+// lane 63 holds the sum of the wave's 64 values (six row shifts and broadcasts; the other lanes hold
+// partial sums)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ u32 plus_dpp(u32 x) {
+  return x + (u32)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xF, true);
+}
+__device__ __forceinline__ u32 wave_sum(u32 x) {
+  x = plus_dpp<0x111, 0xF>(x);  // row_shr:1, 2, 4, 8
+  x = plus_dpp<0x112, 0xF>(x);
+  x = plus_dpp<0x114, 0xF>(x);
+  x = plus_dpp<0x118, 0xF>(x);
+  x = plus_dpp<0x142, 0xA>(x);  // row_bcast:15 into rows 1 and 3
+  x = plus_dpp<0x143, 0xC>(x);  // row_bcast:31 into rows 2 and 3
+  return x;
+}
+__device__ __forceinline__ Limbs wave_sum(const Limbs &v) { return {{wave_sum(v.l[0]), wave_sum(v.l[1]), wave_sum(v.l[2])}}; }
+
+// partial[chunk, col] = sum over the chunk's rows of L_row * y[row, col], for the chunk's rows and
+// `cols_per_group` columns; with a single chunk, the evaluations themselves (`partial` = evals).
+// XE: extension coefficients; YE: extension values.
+// What bounds it: HBM (8 B per base value read once), with 32 KB of the next column in flight per
+// workgroup.  64 x 2^20 base values at an extension point take 103 us with the sum over the chunks
+// (5.2 TB/s), at a base point 94 us; reducing every product took 278 and 164 us, 52 of them in a
+// final kernel with one lane per column.
 template <bool XE, bool YE>
-__global__ __launch_bounds__(kThreads) void partial_kernel(const u64 *ys, const u64 *coeffs, u32 log_count,
-                                                           u32 num_polys, u64 *partial, u32 chunks) {
-  typedef F<XE> Fx;
-  typedef typename Fx::T T;
+__global__ __launch_bounds__(kEvalThreads) void partial_kernel(const u64 *ys, const u64 *coeffs, u32 log_count,
+                                                               u32 num_polys, u32 cols_per_group, u64 *partial,
+                                                               u32 chunks) {
+  constexpr int PL = XE ? 2 : 1, PY = YE ? 2 : 1;  // planes of a coefficient, of a value
+  constexpr int WAVES = kEvalThreads / 64;
   const u64 count = 1ull << log_count;
   const u32 chunk = blockIdx.x;
-  const u64 r0 = (u64)chunk * kChunk;
   const u32 t = threadIdx.x;
-  T l[kRows];
+  // rows past the end of a short column read row 0 with coefficient zero
+  u32 row[kRows];
+  u64 l[PL][kRows];
+#pragma unroll
   for (int k = 0; k < kRows; k++) {
-    const u64 r = r0 + t + (u64)k * kThreads;
-    l[k] = r < count ? Fx::load(coeffs, r, count) : Fx::zero();
+    const u32 r = chunk * kChunk + t + k * kEvalThreads;
+    const bool in = !(r >> log_count);
+    row[k] = in ? r : 0;
+#pragma unroll
+    for (int p = 0; p < PL; p++) {
+      const u64 x = coeffs[row[k] + p * count];
+      l[p][k] = in ? x : 0;
+    }
   }
-  __shared__ T red[kThreads / 64];
-  const u32 col_end = min(num_polys, (blockIdx.y + 1) * kColsPerGroup);
-  // base-field values: the next column's are loaded while the current column is accumulated
-  // (rows past the end of a short column read as zero and contribute nothing); extension values
-  // are read in the loop (two registers each would leave one wave per SIMD)
-  u64 nxt[YE ? 1 : kRows];
+  __shared__ u64 sums[kColsPerGroup][PL][WAVES];
+  const u32 col0 = blockIdx.y * cols_per_group;
+  const u32 cols = min(num_polys - col0, cols_per_group);
+  // the next column's values are loaded while the current column is accumulated
+  u64 nxt[PY][kRows];
   auto fetch = [&](u32 col) {
-    if constexpr (!YE) {
+    const u64 *y = ys + (u64)col * PY * count;
 #pragma unroll
-      for (int k = 0; k < kRows; k++) {
-        const u64 r = r0 + t + (u64)k * kThreads;
-        nxt[k] = r < count ? ys[(u64)col * count + r] : 0;
-      }
-    }
+    for (int k = 0; k < kRows; k++)
+#pragma unroll
+      for (int p = 0; p < PY; p++) nxt[p][k] = y[row[k] + p * count];
   };
-  u32 col = blockIdx.y * kColsPerGroup;
-  if (col < col_end) fetch(col);
-  for (; col < col_end; col++) {
-    T acc = Fx::zero();
-    if constexpr (YE) {
+  fetch(col0);
+  for (u32 i = 0; i < cols; i++) {
+    u64 cur[PY][kRows];
+#pragma unroll
+    for (int k = 0; k < kRows; k++)
+#pragma unroll
+      for (int p = 0; p < PY; p++) cur[p][k] = nxt[p][k];
+    if (i + 1 < cols) fetch(col0 + i + 1);
+    Limbs out[PL];
+    if constexpr (YE) {  // (l0 + l1 u)(y0 + y1 u) = l0 y0 + 7 l1 y1 + (l0 y1 + l1 y0) u
+      ProductSum s00, s11, s01;
+#pragma unroll
       for (int k = 0; k < kRows; k++) {
-        const u64 r = r0 + t + (u64)k * kThreads;
-        if (r >= count) break;
-        const Ext y = F<true>::load(ys + (u64)col * 2 * count, r, count);
-        acc = Fx::add(acc, Fx::mul(l[k], T(y)));
+        s00.add(l[0][k], cur[0][k]);
+        s11.add(l[1][k], cur[1][k]);
+        s01.add(l[0][k], cur[1][k]);
+        s01.add(l[1][k], cur[0][k]);
       }
+      const Limbs p = limbs_of(s00.value()), q = limbs_of(s11.value());
+#pragma unroll
+      for (int j = 0; j < 3; j++) out[0].l[j] = p.l[j] + 7 * q.l[j];  // < 2^25, < 2^31 over a wave
+      out[1] = limbs_of(s01.value());
     } else {
-      u64 cur[kRows];
 #pragma unroll
-      for (int k = 0; k < kRows; k++) cur[k] = nxt[k];
-      if (col + 1 < col_end) fetch(col + 1);
+      for (int p = 0; p < PL; p++) {
+        ProductSum s;
 #pragma unroll
-      for (int k = 0; k < kRows; k++) acc = Fx::add(acc, Fx::scale(l[k], gl::canon(cur[k])));
-    }
-    // wave reduction through shuffles, then across the 4 waves through LDS
-    for (int off = 32; off > 0; off >>= 1) {
-      T o;
-      if constexpr (XE) {
-        o.a = __shfl_xor(acc.a, off);
-        o.b = __shfl_xor(acc.b, off);
-      } else {
-        o = __shfl_xor(acc, off);
+        for (int k = 0; k < kRows; k++) s.add(l[p][k], cur[0][k]);
+        out[p] = limbs_of(s.value());
       }
-      acc = Fx::add(acc, o);
     }
-    if ((t & 63) == 0) red[t >> 6] = acc;
-    __syncthreads();
-    if (t == 0) {
-      T s = red[0];
-      for (u32 w = 1; w < kThreads / 64; w++) s = Fx::add(s, red[w]);
-      // partial sums: column `col` holds `chunks` values (two planes for the extension)
-      Fx::store(partial + (u64)col * chunks * (XE ? 2 : 1), chunk, chunks, s);
+#pragma unroll
+    for (int p = 0; p < PL; p++) {
+      const u64 v = joined(wave_sum(out[p]));
+      if ((t & 63) == 63) sums[i][p][t >> 6] = v;
     }
-    __syncthreads();
+  }
+  __syncthreads();
+  // one lane per (column, plane) adds the waves' sums
+  if (t < cols * PL) {
+    const u32 i = t / PL, p = t % PL;
+    u64 s = sums[i][p][0];
+#pragma unroll
+    for (int w = 1; w < WAVES; w++) s = gl::add(s, sums[i][p][w]);
+    // partial sums: a column holds `chunks` values per plane; a single chunk's are its evaluations
+    partial[((u64)(col0 + i) * PL + p) * chunks + chunk] = s;
   }
 }
 
-// evals[col] = sum over chunks of partial[chunk, col]; extension results interleaved (c0, c1)
-template <bool XE>
-__global__ __launch_bounds__(kThreads) void final_kernel(const u64 *partial, u32 chunks, u32 num_polys, u64 *evals) {
-  typedef F<XE> Fx;
-  typedef typename Fx::T T;
-  const u32 col = blockIdx.x * kThreads + threadIdx.x;
-  if (col >= num_polys) return;
-  const u64 *p = partial + (u64)col * chunks * (XE ? 2 : 1);
-  T s = Fx::zero();
-  for (u32 k = 0; k < chunks; k++) s = Fx::add(s, Fx::load(p, k, chunks));
-  if constexpr (XE) {
-    evals[2 * (u64)col] = s.a;
-    evals[2 * (u64)col + 1] = s.b;
-  } else {
-    evals[col] = s;
+// evals[col] = sum over chunks of partial[chunk, col], one wave per (column, plane); extension results
+// interleaved (c0, c1).  A lane sums the words of its chunks in 64 bits (at most 2^18 chunks).
+__global__ __launch_bounds__(64) void final_kernel(const u64 *partial, u32 chunks, u64 *evals) {
+  const u64 *p = partial + (u64)blockIdx.x * chunks;
+  u64 l = 0, h = 0;
+  for (u32 k = threadIdx.x; k < chunks; k += 64) {
+    const u64 x = p[k];
+    l += gl::isa::lo(x);
+    h += gl::isa::hi(x);
   }
+  const u64 s = joined(wave_sum(limbs_of(gl::fold_words(l, h))));
+  if (threadIdx.x == 63) evals[blockIdx.x] = s;
 }
 
 bool pow2(u64 x) { return x && !(x & (x - 1)); }
@@ -258,22 +322,15 @@ extern "C" int ba_barycentric_precompute_lagrange_coeffs(int ext, const uint64_t
   const ba_context *ctx = ba_context_for_current_device();
   if (!ctx) return BA_ERROR_NOT_INITIALIZED;
   hipStream_t s = (hipStream_t)stream;
-  const u32 grid = (u32)std::max<u64>(1, ((u64)count + (u64)kThreads * kInvBatch - 1) / ((u64)kThreads * kInvBatch));
-  if (ext) {
-    hipLaunchKernelGGL(common_factor_kernel<true>, dim3(1), dim3(64), 0, s, x, common_factor, coset, count);
-    hipLaunchKernelGGL(coeffs_kernel<true>, dim3(grid), dim3(kThreads), 0, s, ctx->tab, x,
-                       (const u64 *)common_factor, coset, log_count, lagrange_coeffs);
-  } else {
-    hipLaunchKernelGGL(common_factor_kernel<false>, dim3(1), dim3(64), 0, s, x, common_factor, coset, count);
-    hipLaunchKernelGGL(coeffs_kernel<false>, dim3(grid), dim3(kThreads), 0, s, ctx->tab, x,
-                       (const u64 *)common_factor, coset, log_count, lagrange_coeffs);
-  }
-  hipError_t err = hipGetLastError();
-  if (err != hipSuccess) return (int)err;
-  // bit-reversed order, as the reference's bit_reverse_in_place epilogue (barycentric.rs:118-124):
-  // the extension planes are two columns of count
-  if (bit_reverse) return ba_bit_reverse_in_place(lagrange_coeffs, count, log_count, ext ? 2 : 1, stream);
-  return BA_SUCCESS;
+  // 8 elements per lane once a workgroup's lanes have at least one each
+  const u32 log_k = log_count > 8 ? std::min(kLogInvBatch, log_count - 8) : 0;
+  const u32 grid = std::max(1u, (count >> log_k) / kThreads);
+  const u64 c = gl::canon(coset), cn = gl_host::pow(c, count);
+  const u64 scale = gl_host::mul(c, gl_host::inv(gl_host::mul(count, cn)));
+  const auto kernel = ext ? coeffs_kernel<true> : coeffs_kernel<false>;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), 0, s, ctx->tab, x, common_factor, c, cn, scale, log_count,
+                     log_k, bit_reverse != 0, lagrange_coeffs);
+  return (int)hipGetLastError();
 }
 
 extern "C" int ba_barycentric_batch_eval_temp_elems(int kind, uint32_t count, uint32_t num_polys, uint64_t *elems) {
@@ -293,26 +350,25 @@ extern "C" int ba_barycentric_batch_eval(int kind, const uint64_t *ys, uint32_t 
   const u32 log_count = log2u(count);
   const u32 chunks = (u32)(((u64)count + kChunk - 1) / kChunk);
   hipStream_t s = (hipStream_t)stream;
-  const dim3 grid(chunks, (num_polys + kColsPerGroup - 1) / kColsPerGroup);
-  const dim3 fgrid((num_polys + kThreads - 1) / kThreads);
-  if (grid.y > 65535) return BA_ERROR_INVALID_VALUE;
-  switch (kind) {
-    case 0:  // base-field evaluations at a base-field point
-      hipLaunchKernelGGL((partial_kernel<false, false>), grid, dim3(kThreads), 0, s, ys, lagrange_coeffs, log_count,
-                         num_polys, temp, chunks);
-      hipLaunchKernelGGL(final_kernel<false>, fgrid, dim3(kThreads), 0, s, (const u64 *)temp, chunks, num_polys, evals);
-      break;
-    case 1:  // base-field evaluations at an extension point
-      hipLaunchKernelGGL((partial_kernel<true, false>), grid, dim3(kThreads), 0, s, ys, lagrange_coeffs, log_count,
-                         num_polys, temp, chunks);
-      hipLaunchKernelGGL(final_kernel<true>, fgrid, dim3(kThreads), 0, s, (const u64 *)temp, chunks, num_polys, evals);
-      break;
-    default:  // extension evaluations at an extension point
-      hipLaunchKernelGGL((partial_kernel<true, true>), grid, dim3(kThreads), 0, s, ys, lagrange_coeffs, log_count,
-                         num_polys, temp, chunks);
-      hipLaunchKernelGGL(final_kernel<true>, fgrid, dim3(kThreads), 0, s, (const u64 *)temp, chunks, num_polys, evals);
-      break;
-  }
+  if ((num_polys + kColsPerGroup - 1) / kColsPerGroup > 65535) return BA_ERROR_INVALID_VALUE;
+  // Columns per workgroup: as many as give most CUs a workgroup.  Eight columns read the
+  // coefficients once for all of them; with fewer workgroups than that, idle CUs cost more than
+  // reading them again: 100 x 2^12 takes 5.6 us on 100 workgroups and 12.0 on 13, 100 x 2^16 17.1 us
+  // on 800 and 15.8 on 208.
+  u32 cols = kColsPerGroup;
+  while (cols > 1 && (u64)chunks * ((num_polys + cols - 1) / cols) < 192) cols /= 2;
+  const dim3 grid(chunks, (num_polys + cols - 1) / cols);
+  u64 *sums = chunks == 1 ? evals : temp;
+  // 0: base-field evaluations at a base-field point; 1: base-field evaluations at an extension point;
+  // 2: extension evaluations at an extension point
+  const auto kernel = kind == 0   ? partial_kernel<false, false>
+                      : kind == 1 ? partial_kernel<true, false>
+                                  : partial_kernel<true, true>;
+  hipLaunchKernelGGL(kernel, grid, dim3(kEvalThreads), 0, s, ys, lagrange_coeffs, log_count, num_polys, cols, sums,
+                     chunks);
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess || chunks == 1) return (int)err;
+  hipLaunchKernelGGL(final_kernel, dim3(num_polys * (kind ? 2 : 1)), dim3(64), 0, s, (const u64 *)temp, chunks, evals);
   return (int)hipGetLastError();
 }
 

@@ -322,7 +322,34 @@ __device__ __forceinline__ u64 pow_u64(u64 a, u64 e) {
   return r;
 }
 
-// a^-1 = a^(p-2) (0 maps to 0)
-__device__ __forceinline__ u64 inv(u64 a) { return pow_u64(a, P - 2); }
+// a^(2^K), lazy
+template <int K>
+__device__ __forceinline__ u64 sqr_times(u64 a) {
+#pragma unroll 1
+  for (int i = 0; i < K; i++) a = mul_lazy(a, a);
+  return a;
+}
+
+// a^-1 = a^(p-2) (0 maps to 0), a any u64; result canonical.  With e_k = a^(2^k - 1):
+// p - 2 = (2^31 - 1) 2^33 + 2^32 - 1, so the inverse is e_31^(2^33) e_32: 64 squarings and 9
+// products (126 by binary exponentiation).
+__device__ __forceinline__ u64 inv(u64 a) {
+  const u64 e2 = mul_lazy(mul_lazy(a, a), a), e3 = mul_lazy(mul_lazy(e2, e2), a);
+  const u64 e6 = mul_lazy(sqr_times<3>(e3), e3), e12 = mul_lazy(sqr_times<6>(e6), e6);
+  const u64 e24 = mul_lazy(sqr_times<12>(e12), e12), e30 = mul_lazy(sqr_times<6>(e24), e6);
+  const u64 e31 = mul_lazy(mul_lazy(e30, e30), a), e32 = mul_lazy(mul_lazy(e31, e31), a);
+  return mul(sqr_times<33>(e31), e32);
+}
+
+// l + h 2^32 as a lazy residue, for l, h < 2^62: with h = h0 + h1 2^32 the value is
+// l + h0 2^32 + h1 EPS < 2^64 + 2^63, so it overflows at most once, and adding EPS for that
+// overflow does not wrap.  4 VALU.
+__device__ __forceinline__ u64 fold_words(u64 l, u64 h) {
+  using namespace isa;
+  u64 c1, c2, dead;
+  const u32 s = add_co(hi(l), lo(h), c1);
+  const u64 r = mad_eps(hi(h), pack(lo(l), s), c2);
+  return mad_eps(one_if(c1 | c2), r, dead);
+}
 
 }  // namespace gl

@@ -84,16 +84,7 @@ __device__ __forceinline__ u64 shl_add(u64 a, u64 b) {
 __device__ __forceinline__ Planes operator+(const Planes &a, const Planes &b) {
   return {shl_add<0>(a.l, b.l), shl_add<0>(a.h, b.h)};
 }
-// l + h 2^32 as a lazy residue, for l, h < 2^62: with h = h0 + h1 2^32 the value is
-// l + h0 2^32 + h1 EPS < 2^64 + 2^63, so it overflows at most once, and adding EPS for that
-// overflow does not wrap.  4 VALU.
-__device__ __forceinline__ u64 folded(const Planes &v) {
-  using namespace gl::isa;
-  u64 c1, c2, dead;
-  const u32 s = add_co(hi(v.l), lo(v.h), c1);
-  const u64 r = mad_eps(hi(v.h), pack(lo(v.l), s), c2);
-  return mad_eps(one_if(c1 | c2), r, dead);
-}
+__device__ __forceinline__ u64 folded(const Planes &v) { return gl::fold_words(v.l, v.h); }
 
 // M4 of Appendix B, [[5,7,1,3],[4,6,1,1],[1,3,5,7],[1,1,4,6]], as an addition chain on one plane
 __device__ __forceinline__ void m4(u64 (&x)[4]) {
