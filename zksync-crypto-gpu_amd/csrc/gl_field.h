@@ -118,25 +118,22 @@ __device__ __forceinline__ u64 ge_p(u64 x) {
   asm("v_cmp_ge_u64_e64 %0, %1, %2" : "=s"(m) : "v"(x), "s"(P));
   return m;
 }
-// x + EPS in the lanes of m (x + 2^32 - 1: low word - 1, high word + 1 unless the low word
-// borrowed); wraps mod 2^64 where the sum overflows
-__device__ __forceinline__ u64 plus_eps(u32 x0, u32 x1, u64 m) {
-  u64 k;
-  const u32 r0 = subb0(x0, m, k);
-  return pack(r0, addc0(x1, m & ~k));
-}
-// x - EPS in the lanes of m (low word + 1, high word - 1 unless the low word carried)
-__device__ __forceinline__ u64 minus_eps(u32 x0, u32 x1, u64 m) {
-  u64 k;
-  const u32 r0 = addc0(x0, m, k);
-  return pack(r0, subb0(x1, m & ~k));
-}
-
 // 1 in the lanes of m, else 0
 __device__ __forceinline__ u32 one_if(u64 m) {
   u32 r;
   asm("v_cndmask_b32_e64 %0, 0, 1, %1" : "=v"(r) : "s"(m));
   return r;
+}
+
+// x + EPS in the lanes of m, wrapping mod 2^64.  2 VALU and no mask logic: a form with a borrowing
+// subtract and a carrying add is as many VALU instructions, but puts a scalar mask operation and
+// three wait states into the chain (12-bit contiguous NTT pass 5 % slower).
+__device__ __forceinline__ u64 add_eps(u64 x, u64 m) { return (u64)one_if(m) * (u32)EPS + x; }
+// x - EPS in the lanes of m (low word + 1, high word - 1 unless the low word carried)
+__device__ __forceinline__ u64 minus_eps(u32 x0, u32 x1, u64 m) {
+  u64 k;
+  const u32 r0 = addc0(x0, m, k);
+  return pack(r0, subb0(x1, m & ~k));
 }
 
 }  // namespace isa
@@ -148,7 +145,7 @@ __device__ __forceinline__ u64 add(u64 a, u64 b) {
   u64 c, c2;
   const u32 s0 = add_co(lo(a), lo(b), c);
   const u32 s1 = addc(hi(a), hi(b), c, c2);
-  return plus_eps(s0, s1, c2 | ge_p(pack(s0, s1)));
+  return add_eps(pack(s0, s1), c2 | ge_p(pack(s0, s1)));
 }
 
 // a < p, b < p: canonical a - b.  d = a - b with borrow; a borrow selects d - EPS (= a - b + p,
@@ -165,42 +162,32 @@ __device__ __forceinline__ u64 sub(u64 a, u64 b) {
 // Canonical form of any u64: x >= p selects x + EPS (wrapping to x - p).  3 VALU.
 __device__ __forceinline__ u64 reduce1(u64 x) {
   using namespace isa;
-  return plus_eps(lo(x), hi(x), ge_p(x));
+  return add_eps(x, ge_p(x));
 }
 
 __device__ __forceinline__ u64 neg(u64 a) { return a ? P - a : 0; }
 
-// Canonical residue of lo + hl (2^32 - 1) - hh - bi (lo < 2^64; hl, hh < 2^32; bi a 0/1 lane
-// mask), i.e. of lo + (hl + (hh + bi) 2^32) 2^64 by 2^64 = 2^32 - 1 and 2^96 = -1.
-//   R = hl EPS + lo with carry c (one v_mad_u64_u32), D = R - hh - bi with borrow b; the value is
-//   V = D + (c - b) 2^64, in (-2^33, 2^64 + 2^64), and
-//     b & !c:  V < 0,           the residue is D - EPS (D >= 2^64 - 2^33, no wrap);
-//     c & !b:  V > p,           the residue is D + EPS (D < hl EPS, no wrap, result < p);
-//     else     V = D in [0, 2^64): D >= p selects D + EPS (wrapping to D - p).
-// 8 VALU.
+// Canonical residue of lo + hl (2^32 - 1) - hh - bi (lo < 2^64; hl, hh < 2^32, hh + bi < 2^32; bi a
+// 0/1 lane mask), i.e. of lo + (hl + (hh + bi) 2^32) 2^64 by 2^64 = 2^32 - 1 and 2^96 = -1.
+//   t = lo - hh - bi; a borrow selects t - EPS (t > 2^64 - 2^32 then, no wrap);
+//   R = hl EPS + t with carry c (one v_mad_u64_u32); a carry selects R + EPS, canonical since
+//   R < hl EPS <= (2^32 - 1)^2; without one, R >= p selects R + EPS (wrapping to R - p).
+// 8 VALU, 2 scalar mask operations.
 __device__ __forceinline__ u64 reduce3b(u64 lo_, u32 hl, u32 hh, u64 bi) {
   using namespace isa;
   u64 c, b1, b;
-  const u64 R = mad_eps(hl, lo_, c);
-  const u32 d0 = subb(lo(R), hh, bi, b1);
-  const u32 d1 = subb0(hi(R), b1, b);
-  const u64 ge = ge_p(pack(d0, d1));
-  const u64 m_sub = b & ~c;
-  const u64 m_add = (c & ~b) | (ge & ~(c ^ b));
-  const u64 e = minus_eps(d0, d1, m_sub);
-  return plus_eps(lo(e), hi(e), m_add);
+  const u32 t0 = subb(lo(lo_), hh, bi, b1);
+  const u32 t1 = subb0(hi(lo_), b1, b);
+  const u64 R = mad_eps(hl, minus_eps(t0, t1, b), c);
+  return add_eps(R, c | ge_p(R));
 }
 __device__ __forceinline__ u64 reduce3(u64 lo_, u32 hl, u32 hh) {
   using namespace isa;
   u64 c, b1, b;
-  const u64 R = mad_eps(hl, lo_, c);
-  const u32 d0 = sub_co(lo(R), hh, b1);
-  const u32 d1 = subb0(hi(R), b1, b);
-  const u64 ge = ge_p(pack(d0, d1));
-  const u64 m_sub = b & ~c;
-  const u64 m_add = (c & ~b) | (ge & ~(c ^ b));
-  const u64 e = minus_eps(d0, d1, m_sub);
-  return plus_eps(lo(e), hi(e), m_add);
+  const u32 t0 = sub_co(lo(lo_), hh, b1);
+  const u32 t1 = subb0(hi(lo_), b1, b);
+  const u64 R = mad_eps(hl, minus_eps(t0, t1, b), c);
+  return add_eps(R, c | ge_p(R));
 }
 
 // Canonical residue of lo + hl (2^32 - 1) (lo < 2^64, hl < 2^32): R = hl EPS + lo with carry c;
@@ -209,7 +196,7 @@ __device__ __forceinline__ u64 reduce2(u64 lo_, u32 hl) {
   using namespace isa;
   u64 c;
   const u64 R = mad_eps(hl, lo_, c);
-  return plus_eps(lo(R), hi(R), c | ge_p(R));
+  return add_eps(R, c | ge_p(R));
 }
 
 // Reduces lo + hi * 2^64 (any 128-bit value) to a canonical residue.

@@ -36,10 +36,10 @@ __device__ __forceinline__ void sfor(F &&f) {
 // ---------------------------------------------------------------- product (canonical result)
 struct Mul {
   u64 a, b, r;
-  u64 z, y, w, R, cy, k1, k2, c, b1, bb, msub, madd, k;
-  u32 r1, r2, r3, d0, d1, e0, e1, f0;
+  u64 z, y, w, R, cy, k1, k2, c, b1, bw, m, k;
+  u32 r1, r2, r3, t0, t1, one;
 };
-constexpr int MUL_PHASES = 13;
+constexpr int MUL_PHASES = 12;
 
 // phase P of gl::mul(s.a, s.b) -> s.r
 template <int P>
@@ -58,23 +58,19 @@ __device__ __forceinline__ void mul_phase(Mul &s) {
   } else if constexpr (P == 4) {
     s.r3 = addc0(hi(s.w), s.k2);
   } else if constexpr (P == 5) {
-    s.R = mad_eps(s.r2, pack(lo(s.z), s.r1), s.c);
+    s.t0 = subb(lo(s.z), s.r3, s.cy, s.b1);
   } else if constexpr (P == 6) {
-    s.d0 = subb(lo(s.R), s.r3, s.cy, s.b1);
+    s.t1 = subb0(s.r1, s.b1, s.bw);
   } else if constexpr (P == 7) {
-    s.d1 = subb0(hi(s.R), s.b1, s.bb);
+    s.t0 = addc0(s.t0, s.bw, s.k);
   } else if constexpr (P == 8) {
-    const u64 ge = ge_p(pack(s.d0, s.d1));
-    s.msub = s.bb & ~s.c;
-    s.madd = (s.c & ~s.bb) | (ge & ~(s.c ^ s.bb));
+    s.t1 = subb0(s.t1, s.bw & ~s.k);
   } else if constexpr (P == 9) {
-    s.e0 = addc0(s.d0, s.msub, s.k);
+    s.R = mad_eps(s.r2, pack(s.t0, s.t1), s.c);
   } else if constexpr (P == 10) {
-    s.e1 = subb0(s.d1, s.msub & ~s.k);
+    s.one = one_if(s.c | ge_p(s.R));
   } else if constexpr (P == 11) {
-    s.f0 = subb0(s.e0, s.madd, s.k);
-  } else if constexpr (P == 12) {
-    s.r = pack(s.f0, addc0(s.e1, s.madd & ~s.k));
+    s.r = (u64)s.one * (u32)EPS + s.R;
   }
 }
 
@@ -104,15 +100,15 @@ __device__ __forceinline__ void mul_batch(X &&x, Y &&y) {
 
 // ---------------------------------------------------------------- shift by 2^F, canonical result
 // The three forms of gl::shl / gl::shr (x any u64):
-//   F in (0, 32]:  x << F = lo + hl 2^64 -> reduce2                          5 phases
-//   F in (32, 64): x << F = lo + (hl + hh 2^32) 2^64 -> reduce3              9 phases
+//   F in (0, 32]:  x << F = lo + hl 2^64 -> reduce2                          4 phases
+//   F in (32, 64): x << F = lo + (hl + hh 2^32) 2^64 -> reduce3              8 phases
 //   F in [64, 96): 2^F = -2^-(96-F): x 2^-M = q - r 2^(32-M) EPS, M = 96 - F  6 phases
-constexpr int shift_phases(int F) { return F == 0 ? 0 : F <= 32 ? 5 : F < 64 ? 9 : 6; }
+constexpr int shift_phases(int F) { return F == 0 ? 0 : F <= 32 ? 4 : F < 64 ? 8 : 6; }
 
 struct Shift {
   u64 x, t;  // in, out
-  u64 lo, R, c, b1, bb, m, k, msub, madd, q, u, bw;
-  u32 hl, hh, d0, d1, e0, e1, t0, r;
+  u64 lo, R, c, b1, bw, k, q, u;
+  u32 hl, hh, d0, d1, t0, r, one;
 };
 
 template <int F, int P>
@@ -127,11 +123,9 @@ __device__ __forceinline__ void shift_phase(Shift &s) {
     } else if constexpr (P == 1) {
       s.R = mad_eps(s.hl, s.lo, s.c);
     } else if constexpr (P == 2) {
-      s.m = s.c | ge_p(s.R);
+      s.one = one_if(s.c | ge_p(s.R));
     } else if constexpr (P == 3) {
-      s.t0 = subb0(lo(s.R), s.m, s.k);
-    } else if constexpr (P == 4) {
-      s.t = pack(s.t0, addc0(hi(s.R), s.m & ~s.k));
+      s.t = (u64)s.one * (u32)EPS + s.R;
     }
   } else if constexpr (F < 64) {
     if constexpr (P == 0) {
@@ -140,23 +134,19 @@ __device__ __forceinline__ void shift_phase(Shift &s) {
       s.hl = (u32)h;
       s.hh = (u32)(h >> 32);
     } else if constexpr (P == 1) {
-      s.R = mad_eps(s.hl, s.lo, s.c);
+      s.d0 = sub_co(isa::lo(s.lo), s.hh, s.b1);
     } else if constexpr (P == 2) {
-      s.d0 = sub_co(lo(s.R), s.hh, s.b1);
+      s.d1 = subb0(isa::hi(s.lo), s.b1, s.bw);
     } else if constexpr (P == 3) {
-      s.d1 = subb0(hi(s.R), s.b1, s.bb);
+      s.d0 = addc0(s.d0, s.bw, s.k);
     } else if constexpr (P == 4) {
-      const u64 ge = ge_p(pack(s.d0, s.d1));
-      s.msub = s.bb & ~s.c;
-      s.madd = (s.c & ~s.bb) | (ge & ~(s.c ^ s.bb));
+      s.d1 = subb0(s.d1, s.bw & ~s.k);
     } else if constexpr (P == 5) {
-      s.e0 = addc0(s.d0, s.msub, s.k);
+      s.R = mad_eps(s.hl, pack(s.d0, s.d1), s.c);
     } else if constexpr (P == 6) {
-      s.e1 = subb0(s.d1, s.msub & ~s.k);
+      s.one = one_if(s.c | ge_p(s.R));
     } else if constexpr (P == 7) {
-      s.t0 = subb0(s.e0, s.madd, s.k);
-    } else if constexpr (P == 8) {
-      s.t = pack(s.t0, addc0(s.e1, s.madd & ~s.k));
+      s.t = (u64)s.one * (u32)EPS + s.R;
     }
   } else {
     constexpr int M = 96 - F;
@@ -178,13 +168,13 @@ __device__ __forceinline__ void shift_phase(Shift &s) {
 }
 
 // ---------------------------------------------------------------- add and subtract
-// (s, d) = (a + b, a - b), canonical, from canonical a, b: 5 phases.
+// (s, d) = (a + b, a - b), canonical, from canonical a, b: 4 phases.
 struct AddSub {
   u64 a, b, s, d;
-  u64 cs, c2, cd, bw, m, k, kd;
-  u32 s0, s1, d0, d1;
+  u64 cs, c2, cd, bw, kd;
+  u32 s0, s1, d0, d1, one;
 };
-constexpr int ADDSUB_PHASES = 5;
+constexpr int ADDSUB_PHASES = 4;
 
 template <int P>
 __device__ __forceinline__ void addsub_phase(AddSub &s) {
@@ -196,12 +186,10 @@ __device__ __forceinline__ void addsub_phase(AddSub &s) {
     s.s1 = addc(hi(s.a), hi(s.b), s.cs, s.c2);
     s.d1 = subb(hi(s.a), hi(s.b), s.cd, s.bw);
   } else if constexpr (P == 2) {
-    s.m = s.c2 | ge_p(pack(s.s0, s.s1));
-  } else if constexpr (P == 3) {
-    s.s0 = subb0(s.s0, s.m, s.k);
+    s.one = one_if(s.c2 | ge_p(pack(s.s0, s.s1)));
     s.d0 = addc0(s.d0, s.bw, s.kd);
-  } else if constexpr (P == 4) {
-    s.s = pack(s.s0, addc0(s.s1, s.m & ~s.k));
+  } else if constexpr (P == 3) {
+    s.s = (u64)s.one * (u32)EPS + pack(s.s0, s.s1);
     s.d = pack(s.d0, subb0(s.d1, s.bw & ~s.kd));
   }
 }
