@@ -321,3 +321,65 @@ def test_lde_coset_plans_bit_exact(ba, log_n, bits):
             assert np.array_equal(got, gl_oracle.lde(x, log_n, cols, lb, nthreads=8)), (bits, lb)
     finally:
         ba.tune.set_plan(ba._test_ctx, log_n, ba.tune.LDE_COSETS, None)
+
+
+# The contiguous pass in every layout it can take: each width with its exchanges inside waves (S <= 10)
+# and across them (11, 12), whole 4096-element tiles of longer columns and short columns with a partial
+# last tile, both input orders and directions, the fused scales, both builds, one and several tiles per
+# workgroup.
+@pytest.mark.parametrize("log_n,bits,waves", [(k, [k], 0) for k in range(4, 9)] +
+                         [(k, [k], w) for k in range(9, 13) for w in (3, 4)] +
+                         [(k, [k - 4, 4], w) for k in range(13, 17) for w in (3, 4)])
+def test_contiguous_pass_layouts(ba, log_n, bits, waves):
+    n = 1 << log_n
+    per_tile = max(1, 4096 >> log_n)
+    rng = np.random.default_rng(log_n)
+    ctx = ba.Context.create(12, 12)
+    try:
+        for cols, reps in ((1, 1), (2 * per_tile + 1, 1), (5 * per_tile + max(1, per_tile // 2), 4)):
+            stride = n + 8
+            x = raw_u64(rng, cols * stride)
+            d_in, d_out = ba.DeviceAllocation.from_host(x), ba.DeviceAllocation.from_host(x)
+            try:
+                for bitrev in (False, True):
+                    ba.tune.set_plan(ctx, log_n, bitrev, bits, [reps] * len(bits), waves, 12)
+                    for inverse, lext, coset in ((False, 0, 0), (True, 0, 0), (False, 2, 3), (True, 1, 1)):
+                        log(f"contig log_n={log_n} cols={cols} reps={reps} bitrev={bitrev} inv={inverse} lext={lext}")
+                        ba.ntt.batch_ntt_ctx(ctx, d_in.ptr, d_out.ptr, log_n, cols, stride, stride, bitrev, inverse,
+                                             lext, coset)
+                        ba.synchronize()
+                        got = d_out.to_host().reshape(cols, stride)
+                        want = gl_oracle.batch_ntt(x, log_n, cols, stride, stride, bitrev, inverse, lext, coset)
+                        assert np.array_equal(got[:, :n], np.asarray(want).reshape(cols, stride)[:, :n])
+                        assert np.array_equal(got[:, n:], x.reshape(cols, stride)[:, n:])  # nothing past a column
+            finally:
+                d_in.free()
+                d_out.free()
+    finally:
+        ctx.destroy()
+
+
+@pytest.mark.parametrize("log_n,waves", [(k, 0) for k in range(4, 9)] + [(k, w) for k in range(9, 13) for w in (3, 4)])
+def test_contiguous_pass_gathers_short_lde_columns(ba, log_n, waves):
+    """A column of at most 4096 elements is one contiguous pass, whose coset NTTs read the monomials
+    bit-reversed through LDS."""
+    n, lb = 1 << log_n, 2
+    ctx = ba.Context.create(12, 12)
+    try:
+        for cols, reps in ((1, 1), (3 * max(1, 4096 >> log_n) + 1, 2)):
+            for kind in (0, ba.tune.LDE_COSETS):
+                ba.tune.set_plan(ctx, log_n, kind, [log_n], [reps], waves)
+            ev = raw_u64(np.random.default_rng(log_n), n * cols)
+            d_ev, d_mono = ba.DeviceAllocation.from_host(ev), ba.DeviceAllocation(n * cols)
+            d_out = ba.DeviceAllocation((n << lb) * cols)
+            try:
+                log(f"short lde log_n={log_n} cols={cols} waves={waves}")
+                ba.lde.lde_batch(ctx, d_ev, log_n, cols, lb, d_out, monomials=d_mono)
+                ba.synchronize()
+                want = gl_oracle.lde(ev, log_n, cols, lb)
+                assert np.array_equal(d_out.to_host(), want if isinstance(want, np.ndarray) else want[0])
+            finally:
+                for d in (d_ev, d_mono, d_out):
+                    d.free()
+    finally:
+        ctx.destroy()

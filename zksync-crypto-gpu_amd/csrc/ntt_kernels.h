@@ -541,6 +541,14 @@ __device__ __forceinline__ void strided_body(const PassArgs &a, const u32 bid) {
   }
 }
 
+// Orders LDS accesses of lanes of one wave: its LDS instructions execute in issue order, so only the
+// compiler has to keep that order.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // SC: fused forward pre-scale (INV = false) or inverse post-scale (INV = true): 0 none,
 // 1 one factor for every element (n^-1 of an inverse without coset), 2 per-element coset factors.
 // WHOLE: columns of >= 4096 elements (a tile is one contiguous block of one column); otherwise
@@ -548,6 +556,19 @@ __device__ __forceinline__ void strided_body(const PassArgs &a, const u32 bid) {
 // PREFETCH: the next tile is loaded into registers while the current one is transformed (the
 // three-waves-per-SIMD variant); otherwise each tile is loaded when its transform starts (the
 // four-waves variant, which fits 128 registers).
+//
+// Exchanges between rounds go through LDS within a wave wherever the layouts allow it, so that waves
+// need not run in step.  Thread t = (c, q) holds tile elements (c << S) | window_a<WB>(q, m); in
+// every layout but the top window's (WB = S - 4) of S >= 11 its wave holds exactly elements
+// [1024 w, 1024 w + 1024) of the tile, w = t / 64.  So only the exchange with that top window
+// crosses waves and takes workgroup barriers (one before its writes, for the region's readers of
+// the tile before, one after); passes of S <= 10 have none in their loop.  The global side of a tile
+// is either the top window itself (S >= 8: runs of >= 128 B per 2^(S-4) lanes, straight between
+// global memory and registers) or the wave's own block of 1024 elements, 64 consecutive ones per
+// instruction, staged through LDS within the wave: n2b loads the former and stores the latter, b2n
+// the other way round.  With workgroup barriers and tile-wide staging around every exchange the
+// 12-bit pass over 2^26 elements took 352 us b2n and 329 n2b; it takes 338 and 325, and moves 5
+// LDS words per element either way (7 before for b2n).
 template <int S, bool N2B, bool INV, int SC, bool WHOLE, bool PREFETCH>
 __device__ __forceinline__ void contig_body(const PassArgs &a, const u32 bid) {
   constexpr bool SCALE = SC == 2;
@@ -634,22 +655,54 @@ __device__ __forceinline__ void contig_body(const PassArgs &a, const u32 bid) {
     }
   };
 
-  // the next tile's elements are loaded while the current one is transformed
+  const u32 lane = t & 63, block0 = (t >> 6) << 10;  // the wave's block of 1024 tile elements
+  constexpr bool DIRECT = S >= 8;     // global memory <-> the top window's registers
+  constexpr bool CROSS = S >= 11;     // the exchange with the top window crosses waves
+  constexpr int WBT = S - 4;          // the top window
+  const u32 top0 = (c << S) + window_a<WBT>(q, 0);
+  // LDS slot of register m in a round's layout: for WB >= 4 the padding advances by 2^(WB-4) per step
+  // of m, for WB = 0 (u0 a multiple of 16) not at all; windows at WB = 1..3 (S = 5..7) are padded per
+  // element
+  auto slot_in = [&](auto wb_, int m) -> u32 {
+    constexpr int WB = decltype(wb_)::value;
+    const u32 u0 = (c << S) + window_a<WB>(q, 0);
+    if constexpr (WB == 0 || WB >= 4) {
+      constexpr u32 STEP = (1u << WB) + (WB >= 4 ? (1u << (WB >= 4 ? WB - 4 : 0)) : 0);
+      return lds_pad(u0) + m * STEP;
+    } else {
+      return lds_pad(u0 + ((u32)m << WB));
+    }
+  };
+  // LDS slot of block element lane + 64 k: lds_pad(block0 + lane) + 68 k
+  const u32 bslot = lds_pad(block0 + lane);
+  auto block_slot = [&](int k) -> u32 { return bslot + 68u * k; };
+  // a bit-reversed input (single n2b pass) is a permutation inside each column, applied on the way
+  // through LDS
+  const bool gather = N2B && a.in_bitrev;
+  const bool direct_in = DIRECT && N2B && !gather;
+  const u32 in0 = direct_in ? top0 : block0 + lane, in_step = direct_in ? WBT : 6;
+
   u64 nxt[VALS];
   auto fetch = [&](u64 tile) {
     if constexpr (whole) {
-      const u64 col = tile >> a.log_tile_stride;
-      const u64 *in = col_in(a, col) + tile_in_col;
+      const u64 *in = col_in(a, tile >> a.log_tile_stride) + tile_in_col;
       static_for<VALS>([&](auto k_) {
         constexpr int k = decltype(k_)::value;
-        nxt[k] = gload(at(in + THREADS * k, t * 8u));
+        nxt[k] = gload(at(in + (k << in_step), in0 * 8u));
+      });
+    } else if (direct_in) {
+      const u64 g = (tile << LOG_C) + c;
+      const bool valid = g < total_chunks;
+      const u64 *in = col_in(a, valid ? g : 0) + window_a<WBT>(q, 0);
+      static_for<VALS>([&](auto m_) {
+        constexpr int m = decltype(m_)::value;
+        nxt[m] = valid ? gload(in + (m << WBT)) : 0;
       });
     } else {
-      const u64 g0 = tile << LOG_C;
       static_for<VALS>([&](auto k_) {
         constexpr int k = decltype(k_)::value;
-        const u32 e = t + THREADS * k;
-        const u64 g = g0 + (e >> S);
+        const u32 e = block0 + lane + 64 * k;
+        const u64 g = (tile << LOG_C) + (e >> S);
         nxt[k] = g < total_chunks ? gload(col_in(a, g) + (e & ((1u << S) - 1))) : 0;
       });
     }
@@ -658,66 +711,75 @@ __device__ __forceinline__ void contig_body(const PassArgs &a, const u32 bid) {
       tile0 < a.tile_count
           ? (u32)min((u64)a.reps, (a.tile_count - tile0 + (1ull << a.log_tile_stride) - 1) >> a.log_tile_stride)
           : 0;
-  // An n2b pass over whole 4096-element tiles starts with the window of the top 4 bits, whose 16
-  // elements per thread (t + 256 m) are the ones the thread loaded: they go straight into
-  // registers, with no LDS staging and its barrier (unless the load is a bit-reversed gather).
-  // The twiddle table's fill then needs a barrier of its own before the first round reads it.
-  const bool direct0 = N2B && S == TILE_LOG && WHOLE && !a.in_bitrev;
-  if (direct0) __syncthreads();
+  __syncthreads();  // the twiddle tables
   if (PREFETCH && reps) fetch(tile0);
   for (u32 i = 0; i < reps; i++) {
     const u64 tile = tile0 + ((u64)i << a.log_tile_stride);
-    const u64 g0 = tile << LOG_C;
     if constexpr (!PREFETCH) fetch(tile);
     // keeps the 16 factors from being hoisted out of the loop (into 32 live registers)
     if constexpr (SCALE && AT_USE) asm volatile("" : "+v"(fbase));
     u64 v[VALS];
-    auto stage = [&](auto reduce_) {
-      static_for<VALS>([&](auto k_) {
-        constexpr int k = decltype(k_)::value;
-        const u32 e = t + THREADS * k;
-        // lds_pad(t + 256 k) = lds_pad(t) + 272 k; a bit-reversed input (single pass) is a
-        // permutation inside each column
-        u32 slot = lds_pad(t) + (THREADS + THREADS / 16) * k;
-        if (N2B && a.in_bitrev) slot = lds_pad(((e >> S) << S) + bitrev32(e & ((1u << S) - 1), L));
-        lds[slot] = decltype(reduce_)::value ? canon(nxt[k]) : nxt[k];
-      });
-    };
-    if (direct0) {
-      if (a.in_canonical) {
+    auto load = [&](auto reduce_) {
+      constexpr bool RED = decltype(reduce_)::value;
+      if (direct_in) {
         static_for<VALS>([&](auto m_) {
           constexpr int m = decltype(m_)::value;
-          v[m] = nxt[m];
+          v[m] = RED ? canon(nxt[m]) : nxt[m];
         });
       } else {
+        // the first round's window is the top one (n2b) or 0 (b2n); LDS is free once every wave has
+        // read the tile before, which only the top window's exchange lets another wave do
+        if constexpr (CROSS) __syncthreads();
+        if (gather) {
+          u32 e0 = block0 + lane;
+          asm volatile("" : "+v"(e0));  // keeps the 16 slots from being hoisted out of the loop
+          static_for<VALS>([&](auto k_) {
+            constexpr int k = decltype(k_)::value;
+            const u32 e = e0 + 64 * k;
+            lds[lds_pad(((e >> S) << S) + bitrev32(e & ((1u << S) - 1), L))] = RED ? canon(nxt[k]) : nxt[k];
+          });
+        } else {
+          static_for<VALS>([&](auto k_) {
+            constexpr int k = decltype(k_)::value;
+            lds[block_slot(k)] = RED ? canon(nxt[k]) : nxt[k];
+          });
+        }
+        if constexpr (CROSS && N2B)
+          __syncthreads();
+        else
+          wave_sync();
         static_for<VALS>([&](auto m_) {
           constexpr int m = decltype(m_)::value;
-          v[m] = canon(nxt[m]);
+          v[m] = lds[slot_in(std::integral_constant<int, Sh::WB(0)>{}, m)];
         });
+        wave_sync();
       }
-    } else if (a.in_canonical) {
-      stage(std::false_type{});
-    } else {
-      stage(std::true_type{});
-    }
+    };
+    if (a.in_canonical)
+      load(std::false_type{});
+    else
+      load(std::true_type{});
     if (PREFETCH && i + 1 < reps) fetch(tile + (1ull << a.log_tile_stride));
-    if (!direct0) __syncthreads();
     static_for<R>([&](auto r_) {
       constexpr int r = decltype(r_)::value;
       constexpr int WB = Sh::WB(r);
-      const u32 u0 = (c << S) + window_a<WB>(q, 0);
-      const u32 l0 = lds_pad(u0);
-      // for WB >= 4 the padding advances by 2^(WB-4) per step of m, for WB = 0 (u0 a multiple
-      // of 16) not at all; partial windows at WB = 1..3 (S = 5..7) are padded per element
-      constexpr bool LINEAR = WB == 0 || WB >= 4;
-      constexpr u32 STEP = (1u << WB) + (WB >= 4 ? (1u << (WB >= 4 ? WB - 4 : 0)) : 0);
-      auto slot = [&](int m) { return LINEAR ? l0 + m * STEP : lds_pad(u0 + ((u32)m << WB)); };
-      if (r != 0 || !direct0) {
+      if constexpr (r > 0) {
+        constexpr int WBP = Sh::WB(r - 1);
+        constexpr bool cross = CROSS && (WB == WBT || WBP == WBT);
+        if constexpr (cross) __syncthreads();
         static_for<VALS>([&](auto m_) {
           constexpr int m = decltype(m_)::value;
-          v[m] = lds[slot(m)];
+          lds[slot_in(std::integral_constant<int, WBP>{}, m)] = v[m];
         });
-        __syncthreads();
+        if constexpr (cross)
+          __syncthreads();
+        else
+          wave_sync();
+        static_for<VALS>([&](auto m_) {
+          constexpr int m = decltype(m_)::value;
+          v[m] = lds[slot_in(std::integral_constant<int, WB>{}, m)];
+        });
+        wave_sync();
       }
       if (SC != 0 && !INV && r == 0) scale_all(v);
       if constexpr (WB >= 4) {
@@ -737,28 +799,46 @@ __device__ __forceinline__ void contig_body(const PassArgs &a, const u32 bid) {
         do_round<Sh::K(r), N2B, INV, false>(v, tw[r], !(top && r == Sh::TOP));
       }
       if (SC != 0 && INV && r == R - 1 && !FOLD) scale_all(v);
+    });
+    if constexpr (DIRECT && !N2B) {  // the last window is the top one
+      if constexpr (whole) {
+        u64 *out = col_out(a, tile >> a.log_tile_stride) + tile_in_col;
+        static_for<VALS>([&](auto m_) {
+          constexpr int m = decltype(m_)::value;
+          gstore(at(out + (m << WBT), top0 * 8u), v[m]);
+        });
+      } else {
+        const u64 g = (tile << LOG_C) + c;
+        if (g < total_chunks) {
+          u64 *out = col_out(a, g) + window_a<WBT>(q, 0);
+          static_for<VALS>([&](auto m_) {
+            constexpr int m = decltype(m_)::value;
+            gstore(out + (m << WBT), v[m]);
+          });
+        }
+      }
+    } else {
       static_for<VALS>([&](auto m_) {
         constexpr int m = decltype(m_)::value;
-        lds[slot(m)] = v[m];
+        lds[slot_in(std::integral_constant<int, Sh::WB(R - 1)>{}, m)] = v[m];
       });
-      __syncthreads();
-    });
-    if constexpr (whole) {
-      const u64 col = tile >> a.log_tile_stride;
-      u64 *out = col_out(a, col) + tile_in_col;
-      static_for<VALS>([&](auto k_) {
-        constexpr int k = decltype(k_)::value;
-        gstore(at(out + THREADS * k, t * 8u), lds[lds_pad(t) + (THREADS + THREADS / 16) * k]);
-      });
-    } else {
-      static_for<VALS>([&](auto k_) {
-        constexpr int k = decltype(k_)::value;
-        const u32 e = t + THREADS * k;
-        const u64 g = g0 + (e >> S);
-        if (g < total_chunks) gstore(col_out(a, g) + (e & ((1u << S) - 1)), lds[lds_pad(e)]);
-      });
+      wave_sync();
+      if constexpr (whole) {
+        u64 *out = col_out(a, tile >> a.log_tile_stride) + tile_in_col;
+        static_for<VALS>([&](auto k_) {
+          constexpr int k = decltype(k_)::value;
+          gstore(at(out + 64 * k, (block0 + lane) * 8u), lds[block_slot(k)]);
+        });
+      } else {
+        static_for<VALS>([&](auto k_) {
+          constexpr int k = decltype(k_)::value;
+          const u32 e = block0 + lane + 64 * k;
+          const u64 g = (tile << LOG_C) + (e >> S);
+          if (g < total_chunks) gstore(col_out(a, g) + (e & ((1u << S) - 1)), lds[block_slot(k)]);
+        });
+      }
+      wave_sync();
     }
-    __syncthreads();
   }
 }
 
