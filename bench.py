@@ -61,9 +61,8 @@ def parse():
     ap.add_argument("--only-single", action="store_true",
                     help="run only the single 2^16 NTT leg (one call per transform) and print its JSON line")
     ap.add_argument("--serial-cosets", action="store_true",
-                    help="run every LDE's coset NTTs in order on the caller's stream (sets "
-                         "BOOJUM_AMD_LDE_SERIAL=1), so that a profiler's per-kernel durations are each "
-                         "launch's own rather than overlapping the other cosets'")
+                    help="launch every LDE's coset NTTs one by one (sets BOOJUM_AMD_LDE_SERIAL=1) instead of "
+                         "merged over the cosets, so that a profiler's per-kernel figures are one transform's")
     return ap.parse_args()
 
 
@@ -782,7 +781,7 @@ def main():
         "config": {"workload": f"batched coset LDE, {cols} columns x 2^{log_n}, blowup {B}, shift 7, "
                                f"bit-reversed output, one hipGraph per step",
                    "columns": cols, "log_n": log_n, "blowup": B, "parallelism": "single GPU",
-                   "cosets": "serial, one stream" if args.serial_cosets else "concurrent, auxiliary streams"},
+                   "cosets": "serial, one stream" if args.serial_cosets else "merged, one launch per pass"},
         "lde_roofline": {"alg_bytes_per_step": lde_alg_bytes,
                          "achieved_GBs": round(lde_alg_bytes / (ms_per_step / 1e3) / 1e9, 1),
                          "frac": round(lde_alg_bytes / (ms_per_step / 1e3) / 1e9 / HBM_PEAK_GBS, 4)},

@@ -148,13 +148,9 @@ int ba_bit_reverse_in_place(uint64_t *values, uint64_t stride, uint32_t log_rows
  * when it is non-null, else they replace the evaluations in place (as into_monomials consumes
  * its storage, storage.rs:155).  Preconditions: 1 <= log_n, 1 <= log_blowup,
  * log_n + log_blowup <= 30, strides >= n, out distinct from evals / monomials, the context's
- * device current.  Cosets after the first run on auxiliary streams of the context, forked from
- * `stream` after the inverse NTT and joined back into it before the call returns (a graph
- * captured from `stream` holds the same fork and join; under ba_profile_begin, or with
- * BOOJUM_AMD_LDE_SERIAL=1 in the environment, every launch stays on `stream`, in order); calls
- * on one context are serialised
- * while they enqueue, and no call on the context may run in another thread while a stream
- * capture holding one of its LDEs is still open. */
+ * device current.  Every launch is on `stream`, in order: the inverse NTT's passes, then each pass
+ * of the coset NTTs as one launch over up to 8 cosets (under ba_profile_begin, or with
+ * BOOJUM_AMD_LDE_SERIAL=1 in the environment, one launch per coset). */
 int ba_lde_batch(ba_context_t ctx, uint64_t *evals, uint64_t in_stride, uint64_t *monomials,
                  uint64_t *out, uint64_t out_col_stride, uint64_t out_coset_stride, uint32_t log_n,
                  uint32_t num_cols, uint32_t log_blowup, ba_stream_t stream);
@@ -274,7 +270,8 @@ int ba_batch_plan_destroy(ba_batch_plan_t plan);
  * batch NTTs (tile_log: 10 = the latency-shaped passes, 1024-element tiles of 4 elements per
  * thread in radix-4 rounds, for every batch size, log_n 4..18 only; 12 = the 4096-element tiles
  * of the split above for every batch size; 0 = built-in choice: 1024-element tiles for batches of
- * at most 2^20 elements, else 4096).  LDE coset NTTs always run the 4096-element tiles.  Valid splits: log_n <= 12
+ * at most 2^20 elements, else 4096).  An LDE call's coset NTTs take the 1024-element tiles by that
+ * batch-size rule alone, counting every coset of a launch.  Valid splits: log_n <= 12
  * one pass of log_n bits; log_n > 12 a contiguous pass of 9..12 bits and strided passes of 4..10
  * bits (at most 8 passes).
  *

@@ -274,3 +274,22 @@ def test_lde_graph_replay(ba, lb):
         for t in (d_ev, d_mono, d_out, d_eager):
             t.free()
         stream.destroy()
+
+
+# Each pass of the coset NTTs is one launch over up to 8 cosets: small batches on the 1024-element
+# tiles (contiguous alone to 2^10, then strided + contiguous to 2^18), larger ones on the 4096-element
+# tiles; 16 and 32 cosets take two and four rounds of launches; tile counts that 8 divides and that it does not.
+@pytest.mark.parametrize("log_n,cols,lb", [(4, 1, 1), (4, 300, 5), (5, 7, 4), (7, 33, 3), (9, 3, 5), (10, 5, 2),
+                                           (11, 1, 1), (11, 5, 4), (12, 3, 3), (13, 1, 2), (15, 3, 1), (17, 3, 1),
+                                           (18, 1, 1), (18, 1, 3), (19, 1, 2),
+                                           (4, 40001, 1), (8, 3000, 1), (9, 1501, 1), (10, 700, 2), (11, 300, 3),
+                                           (12, 70, 3), (13, 43, 3), (14, 21, 3), (15, 37, 1), (16, 5, 4)])
+@pytest.mark.parametrize("layout", ["column", "coset"])
+def test_lde_merged_cosets(ba, log_n, cols, lb, layout):
+    n = 1 << log_n
+    log(f"lde merged log_n={log_n} cols={cols} blowup=2^{lb} {layout}")
+    ev = raw_u64(np.random.default_rng(cols + lb), cols * n)
+    got, ev_after, mono = run_lde(ba, ev, log_n, cols, lb, layout, keep_evals=True)
+    assert np.array_equal(got, gl_oracle.lde(ev, log_n, cols, lb, nthreads=8))
+    assert np.array_equal(mono, gl_oracle.batch_ntt(ev, log_n, cols, n, n, False, True, nthreads=8))
+    assert np.array_equal(ev_after, ev)

@@ -56,13 +56,6 @@ struct ba_context {
   std::atomic<int> users{0};
   // Poseidon2 round constants (30 x 12, device memory), installed by the caller
   uint64_t *p2_round_constants = nullptr;
-  // ba_lde_batch runs the coset NTTs after the first on these streams (created with the context),
-  // forked from and joined back into the caller's stream; the mutex keeps two callers' fork and
-  // join events from interleaving
-  static constexpr int kLdeAux = 7;
-  hipStream_t lde_aux[kLdeAux] = {};
-  hipEvent_t lde_fork = nullptr, lde_join[kLdeAux] = {};
-  std::mutex lde_mutex;
 };
 
 // The most recently created live context of `device`, or null.
@@ -90,6 +83,7 @@ NttPlan ba_plan_for(const ba_context *ctx, uint32_t log_n, bool n2b);
 #include "ntt_inst.h"
 struct BaPassLaunch {
   BaKernels kernels;
+  BaCosetKernel coset_kernel = nullptr;  // the gathered first pass of an LDE's coset NTTs
   gl::ntt::PassArgs args;
   uint64_t grid;
   const char *name;
@@ -98,21 +92,27 @@ struct BaPassLaunch {
 };
 
 // Which transforms may run the latency-shaped passes (1024-element tiles):
-//   BA_LAT_NEVER  LDE transforms (their coset NTTs gather, and their inverse NTT keeps the
-//                 cosets' pass count);
+//   BA_LAT_NEVER  an LDE's transforms inside batch plans (as BA_LAT_TUNED below), or one coset at a time;
 //   BA_LAT_TUNED  the size class's tuned tile_log is 10 (batch plans: a merged small transform
 //                 runs beside other groups of its level, where the throughput passes measured
 //                 as fast and the extra grouped launches cost more);
 //   BA_LAT_AUTO   that, or else the batch holds at most 2^BA_LAT_MAX_LOG_ELEMS elements and the
-//                 tuned tile_log is not 12 (single batch NTT calls).
+//                 tuned tile_log is not 12 (single batch NTT calls, an LDE call's inverse NTT);
+//                 for an LDE call's coset NTTs, by the elements of all cosets of a launch.
 enum BaLatPolicy { BA_LAT_NEVER = 0, BA_LAT_TUNED = 1, BA_LAT_AUTO = 2 };
 // Appends the pass launches of one batch NTT (arguments validated) to `launches`.  shared: the
 // launches will run beside other streams' work (serve batches), so strided passes whose default
-// build runs four waves per SIMD, filling a CU's LDS, take their three-waves build.
+// build runs four waves per SIMD, filling a CU's LDS, take their three-waves build.  cosets: that
+// many NTTs of the same shape run in each launch (an LDE call's cosets), which the choices that
+// depend on the size of a launch count.
 int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint32_t log_n,
                  uint32_t num_cols, uint64_t stride_in, uint64_t stride_out, bool bitrev_inputs,
                  bool inverse, uint32_t log_ext, uint32_t coset_idx, bool in_bitrev_gather,
-                 std::vector<BaPassLaunch> &launches, BaLatPolicy lat = BA_LAT_NEVER, bool shared = false);
+                 std::vector<BaPassLaunch> &launches, BaLatPolicy lat = BA_LAT_NEVER, bool shared = false,
+                 uint32_t cosets = 1);
+// The fused scale factors T[m] (PassArgs::scale_tab) of an NTT and its PassArgs::coset_mul.
+void ba_scale_factors(uint32_t log_n, bool inverse, uint32_t log_ext, uint32_t coset_idx,
+                      uint64_t (&scale_tab)[gl::ntt::VALS], uint32_t &coset_mul);
 // Per-call time over log_n 10..18 and batches of 2^14..2^22 elements (MI355X): up to 2^20
 // elements the latency passes take 1.0-3.1x less time per call, above it the throughput passes win.
 constexpr uint32_t BA_LAT_MAX_LOG_ELEMS = 20;
@@ -164,7 +164,7 @@ int ba_validate_lde(uint64_t *evals, uint64_t in_stride, uint64_t *monomials, ui
 int ba_build_lde(const ba_context *ctx, uint64_t *evals, uint64_t in_stride, uint64_t *monomials,
                  uint64_t *out, uint64_t out_col_stride, uint64_t out_coset_stride, uint32_t log_n,
                  uint32_t num_cols, uint32_t log_blowup, std::vector<BaLeveledLaunch> &launches,
-                 uint32_t first_level, size_t *inverse_launches = nullptr);
+                 uint32_t first_level);
 int ba_validate_ntt(uint32_t log_n, uint64_t stride_in, uint64_t stride_out, uint32_t log_ext,
                     uint32_t coset_idx);
 

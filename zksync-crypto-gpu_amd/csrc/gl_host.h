@@ -39,9 +39,13 @@ inline uint64_t pow(uint64_t a, uint64_t e) {
 
 inline uint64_t inv(uint64_t a) { return pow(a, P - 2); }
 
+// 2^-k for k <= 32: p - 1 is a multiple of 2^32, and 2^k (p - (p - 1) / 2^k) = 1 (mod p)
+inline uint64_t inv_pow2(unsigned k) { return P - ((P - 1) >> k); }
+
 // omega_{2^k}: the 2^32-th root 7^((p-1)/2^32) squared (32 - k) times
 inline uint64_t omega(unsigned log_size) {
-  uint64_t w = pow(7, (P - 1) >> 32);
+  static const uint64_t root = pow(7, (P - 1) >> 32);
+  uint64_t w = root;
   for (unsigned i = log_size; i < 32; i++) w = mul(w, w);
   return w;
 }

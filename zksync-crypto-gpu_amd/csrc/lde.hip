@@ -7,9 +7,9 @@
 //
 // Here the monomials stay in the bit-reversed order the inverse NTT leaves them in, and the
 // first pass of every coset NTT gathers them (coalesced chunk reads staged through LDS), so the
-// separate bit-reverse pass over the data disappears.  Launches: passes(iNTT) + B * passes(NTT);
-// the inverse NTT and coset 0 on the caller's stream, cosets 1.. on the context's auxiliary
-// streams forked from it and joined back, capturable into a hipGraph.
+// separate bit-reverse pass over the data disappears.  The coset NTTs of a call run pass by pass,
+// every pass one launch over up to 8 cosets: passes(iNTT) + passes(NTT) launches, all on the
+// caller's stream.
 #include <algorithm>
 #include <cstdlib>
 #include <vector>
@@ -93,7 +93,7 @@ int ba_validate_lde(uint64_t *evals, uint64_t in_stride, uint64_t *monomials, ui
 int ba_build_lde(const ba_context *ctx, uint64_t *evals, uint64_t in_stride, uint64_t *monomials,
                  uint64_t *out, uint64_t out_col_stride, uint64_t out_coset_stride, uint32_t log_n,
                  uint32_t num_cols, uint32_t log_blowup, std::vector<BaLeveledLaunch> &launches,
-                 uint32_t first_level, size_t *inverse_launches) {
+                 uint32_t first_level) {
   if (num_cols == 0) return BA_SUCCESS;
   const uint64_t n = 1ull << log_n;
   const uint32_t blowup = 1u << log_blowup;
@@ -108,7 +108,6 @@ int ba_build_lde(const ba_context *ctx, uint64_t *evals, uint64_t in_stride, uin
     launches.push_back({first_level + (uint32_t)l.pass, l});
     depth = std::max<uint32_t>(depth, (uint32_t)l.pass + 1);
   }
-  if (inverse_launches) *inverse_launches = ls.size();
   for (uint32_t c = 0; c < blowup; c++) {
     ls.clear();
     rc = ba_build_ntt(ctx, mono, out + (uint64_t)c * out_coset_stride, log_n, num_cols, mono_stride,
@@ -120,8 +119,8 @@ int ba_build_lde(const ba_context *ctx, uint64_t *evals, uint64_t in_stride, uin
   return BA_SUCCESS;
 }
 
-// BOOJUM_AMD_LDE_SERIAL=1 in the environment (read once) keeps every LDE's cosets in order on the
-// caller's stream, so that a profiler's per-kernel durations are each launch's own.
+// BOOJUM_AMD_LDE_SERIAL=1 in the environment (read once) launches every coset's passes on their own,
+// in order, so that a profiler's per-kernel figures are one transform's.
 static bool lde_serial() {
   static const bool serial = [] {
     const char *e = std::getenv("BOOJUM_AMD_LDE_SERIAL");
@@ -130,68 +129,77 @@ static bool lde_serial() {
   return serial;
 }
 
-// The LDE's launches on `stream` (cosets after the first forked onto the context's auxiliary
-// streams and joined back); with natural_monomials the monomials are bit-reversed in place once
+// The LDE's launches with each pass of the coset NTTs merged over the cosets.  A small LDE is a few
+// launches of latency-shaped passes (13 x 2^14 at blowup 4: 33 us, 110 as ten launches of 52
+// workgroups over four streams); a large one reads the monomials once for 8 cosets.
+static int lde_run_merged(const ba_context *ctx, uint64_t *evals, uint64_t in_stride, uint64_t *mono,
+                          uint64_t mono_stride, uint64_t *out, uint64_t out_col_stride, uint64_t out_coset_stride,
+                          uint32_t log_n, uint32_t num_cols, uint32_t log_blowup, hipStream_t stream) {
+  std::vector<BaPassLaunch> ls;
+  int rc = ba_build_ntt(ctx, evals, mono, log_n, num_cols, in_stride, mono_stride, false, true, 0, 0, false, ls,
+                        BA_LAT_AUTO);
+  if (rc || (rc = ba_run_launches(ls, stream))) return rc;
+  const uint32_t blowup = 1u << log_blowup;
+  const uint32_t log_at_once = std::min(log_blowup, 3u), at_once = 1u << log_at_once;
+  static_assert(gl::ntt::MAX_COSETS == 8, "cosets of one launch");
+  for (uint32_t c0 = 0; c0 < blowup; c0 += at_once) {
+    ls.clear();
+    rc = ba_build_ntt(ctx, mono, out + (uint64_t)c0 * out_coset_stride, log_n, num_cols, mono_stride, out_col_stride,
+                      false, false, log_blowup, bitrev_bits(c0, log_blowup), /*in_bitrev_gather=*/true, ls,
+                      BA_LAT_AUTO, false, at_once);
+    if (rc) return rc;
+    gl::ntt::CosetArgs first{};
+    first.coset_stride = out_coset_stride;
+    first.log_cosets = log_at_once;
+    for (uint32_t y = 0; y < at_once; y++)
+      ba_scale_factors(log_n, false, log_blowup, bitrev_bits(c0 + y, log_blowup), first.scale_tab[y],
+                       first.coset_mul[y]);
+    for (const BaPassLaunch &l : ls) {
+      if (l.pass == 0) {
+        first.a = l.args;
+        hipLaunchKernelGGL(l.coset_kernel, dim3((uint32_t)(l.grid << log_at_once)), dim3(gl::ntt::THREADS), 0, stream,
+                           first);
+      } else {
+        gl::ntt::PassArgs a = l.args;
+        a.slice_stride = out_coset_stride;
+        hipLaunchKernelGGL(l.kernels.single, dim3((uint32_t)l.grid, at_once), dim3(gl::ntt::THREADS), 0, stream, a);
+      }
+      const hipError_t err = hipGetLastError();
+      if (err != hipSuccess) return (int)err;
+    }
+  }
+  return BA_SUCCESS;
+}
+
+// The LDE's launches on `stream`; with natural_monomials the monomials are bit-reversed in place once
 // every coset has read them.
 static int lde_run(ba_context_t ctx, uint64_t *evals, uint64_t in_stride, uint64_t *monomials,
                    uint64_t *out, uint64_t out_col_stride, uint64_t out_coset_stride, uint32_t log_n,
                    uint32_t num_cols, uint32_t log_blowup, bool natural_monomials, ba_stream_t stream) {
+  // arguments first (host-only checks), then the context
+  int rc = ba_validate_lde(evals, in_stride, monomials, out, out_col_stride, out_coset_stride, log_n,
+                           num_cols, log_blowup);
+  if (rc) return rc;
+  if (!ctx) return BA_ERROR_NOT_INITIALIZED;
+  if (num_cols == 0) return BA_SUCCESS;
+  int device = -1;  // the context's tables live on its device
+  if (hipGetDevice(&device) != hipSuccess || device != ctx->device) return BA_ERROR_INVALID_VALUE;
   uint64_t *mono = monomials ? monomials : evals;
   const uint64_t mono_stride = monomials ? (1ull << log_n) : in_stride;
-  const int rc = [&]() -> int {
-    // arguments first (host-only checks), then the context
-    int rc = ba_validate_lde(evals, in_stride, monomials, out, out_col_stride, out_coset_stride, log_n,
-                             num_cols, log_blowup);
-    if (rc) return rc;
-    if (!ctx) return BA_ERROR_NOT_INITIALIZED;
-    if (num_cols == 0) return BA_SUCCESS;
-    int device = -1;  // the context's tables, and its auxiliary streams, live on its device
-    if (hipGetDevice(&device) != hipSuccess || device != ctx->device) return BA_ERROR_INVALID_VALUE;
+  if (log_n < 4 || ba_trace_active() || lde_serial()) {
+    // whole transforms per thread, or launches that a trace or profile wants one by one
     std::vector<BaLeveledLaunch> leveled;
-    size_t n_inv = 0;  // the inverse NTT's launches, first in the list
     rc = ba_build_lde(ctx, evals, in_stride, monomials, out, out_col_stride, out_coset_stride, log_n,
-                      num_cols, log_blowup, leveled, 0, &n_inv);
+                      num_cols, log_blowup, leveled, 0);
     if (rc) return rc;
     std::vector<BaPassLaunch> flat;
     for (const BaLeveledLaunch &l : leveled) flat.push_back(l.launch);  // already in dependency order
-    // flat = the inverse NTT's passes (their own plan), then each coset's (one plan shared by the
-    // cosets, which may have another pass count).  The coset NTTs only read the monomials, so
-    // cosets 1.. run on auxiliary streams forked after the inverse NTT and joined back: a pass's
-    // last partial wave of workgroups then overlaps another coset's passes (a graph captured from
-    // `stream` holds the same fork/join).
-    const uint32_t blowup = 1u << log_blowup;
-    const size_t per = (flat.size() - n_inv) / blowup;
-    // (under launch tracing the launches stay in order on one stream, so each one's timing is its own)
-    if (blowup == 1 || per == 0 || n_inv == 0 || n_inv + per * blowup != flat.size() || ba_trace_active() ||
-        !ctx->lde_fork || lde_serial())
-      return ba_run_launches(flat, (hipStream_t)stream);
-    const hipStream_t main = (hipStream_t)stream;
-    std::lock_guard<std::mutex> lock(ctx->lde_mutex);
-    hipError_t err = hipSuccess;
-    const int aux = (int)std::min<uint32_t>(blowup - 1, ba_context::kLdeAux);
-    rc = ba_run_launches(std::vector<BaPassLaunch>(flat.begin(), flat.begin() + n_inv), main);
-    if (rc) return rc;
-    if ((err = hipEventRecord(ctx->lde_fork, main)) != hipSuccess) return (int)err;
-    // Once forked, every auxiliary stream that waited on the fork is joined back even when a later
-    // step fails, so that `stream` still orders after all enqueued work and a capture is not left
-    // with unjoined streams; the first error is returned.
-    int forked = 0;
-    for (; forked < aux && !rc; forked++)
-      if ((err = hipStreamWaitEvent(ctx->lde_aux[forked], ctx->lde_fork, 0)) != hipSuccess) rc = (int)err;
-    if (rc) forked--;  // the failed wait did not fork that stream
-    for (uint32_t c = 0; c < blowup && !rc; c++) {
-      const hipStream_t sc = c == 0 ? main : ctx->lde_aux[(c - 1) % aux];
-      const auto first = flat.begin() + n_inv + per * c;
-      rc = ba_run_launches(std::vector<BaPassLaunch>(first, first + per), sc);
-    }
-    for (int i = 0; i < forked; i++) {
-      if ((err = hipEventRecord(ctx->lde_join[i], ctx->lde_aux[i])) == hipSuccess)
-        err = hipStreamWaitEvent(main, ctx->lde_join[i], 0);
-      if (err != hipSuccess && !rc) rc = (int)err;
-    }
-    return rc;
-  }();
-  if (rc || !natural_monomials || num_cols == 0) return rc;
+    rc = ba_run_launches(flat, (hipStream_t)stream);
+  } else {
+    rc = lde_run_merged(ctx, evals, in_stride, mono, mono_stride, out, out_col_stride, out_coset_stride, log_n,
+                        num_cols, log_blowup, (hipStream_t)stream);
+  }
+  if (rc || !natural_monomials) return rc;
   return ba_bit_reverse_in_place(mono, mono_stride, log_n, num_cols, stream);
 }
 

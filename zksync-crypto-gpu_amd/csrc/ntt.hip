@@ -165,6 +165,11 @@ static uint32_t lat_max_log_elems() {
   return v;
 }
 
+static bool small_batch(uint64_t cols, uint32_t log_n) {
+  const uint32_t m = lat_max_log_elems();
+  return m > 0 && (cols << log_n) <= (1ull << std::min(m, 40u));
+}
+
 bool ba_latency_shape_exists(uint32_t log_n) {
   uint32_t bits[2];
   return lat_bits(log_n, bits) > 0;
@@ -176,34 +181,37 @@ bool ba_use_latency_passes(const ba_context *ctx, uint32_t log_n, bool n2b, uint
   const BaTuned &t = ctx->tuned[n2b][log_n];
   if (t.valid && t.tile_log) return t.tile_log == LAT_TL;
   if (lat == BA_LAT_TUNED) return false;
-  const uint32_t m = lat_max_log_elems();
-  return m > 0 && ((uint64_t)num_cols << log_n) <= (1ull << std::min(m, 40u));
+  return small_batch(num_cols, log_n);
+}
+
+void ba_scale_factors(uint32_t log_n, bool inverse, uint32_t log_ext, uint32_t coset_idx,
+                      uint64_t (&scale_tab)[VALS], uint32_t &coset_mul) {
+  coset_mul = log_ext > 0 ? coset_idx << (gl::OMEGA_LOG_ORDER - log_n - log_ext) : 0;
+  // T[m] = Delta^m (times n^-1 for the inverse), Delta = s^(+-2^(L-4))
+  uint64_t delta = 1;
+  if (log_ext > 0 && log_n >= 4) {
+    delta = gl_host::pow(gl_host::coset_shift(log_n, log_ext, coset_idx), 1ull << (log_n - 4));
+    if (inverse) delta = gl_host::inv(delta);
+  }
+  uint64_t acc = inverse ? gl_host::inv_pow2(log_n) : 1;
+  for (int m = 0; m < VALS; m++) {
+    scale_tab[m] = acc;
+    if (log_ext > 0) acc = gl_host::mul(acc, delta);
+  }
 }
 
 int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint32_t log_n,
                  uint32_t num_cols, uint64_t stride_in, uint64_t stride_out, bool bitrev_inputs,
                  bool inverse, uint32_t log_ext, uint32_t coset_idx, bool in_bitrev_gather,
-                 std::vector<BaPassLaunch> &launches, BaLatPolicy lat, bool shared) {
+                 std::vector<BaPassLaunch> &launches, BaLatPolicy lat, bool shared, uint32_t cosets) {
   if (num_cols == 0) return BA_SUCCESS;
   const bool n2b = !bitrev_inputs;
   PassArgs base{};
   base.log_n = log_n;
   base.scale_coset = log_ext > 0;
-  base.coset_mul = log_ext > 0 ? coset_idx << (gl::OMEGA_LOG_ORDER - log_n - log_ext) : 0;
   base.tab = ctx->tab;
   const bool pre = !inverse && log_ext > 0;
-  // scale table T[m] = Delta^m (times n^-1 for the inverse), Delta = s^(+-2^(L-4))
-  {
-    const uint64_t s = gl_host::coset_shift(log_n, log_ext, coset_idx);
-    const uint64_t n_inv = gl_host::inv(1ull << log_n);
-    const uint64_t sd = log_n >= 4 ? gl_host::pow(s, 1ull << (log_n - 4)) : 1;
-    const uint64_t delta = inverse ? gl_host::inv(sd) : sd;
-    uint64_t acc = inverse ? n_inv : 1;
-    for (int m = 0; m < VALS; m++) {
-      base.scale_tab[m] = acc;
-      acc = gl_host::mul(acc, delta);
-    }
-  }
+  ba_scale_factors(log_n, inverse, log_ext, coset_idx, base.scale_tab, base.coset_mul);
 
   if (log_n < 4) {
     BaPassLaunch l;
@@ -224,7 +232,12 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
     return BA_SUCCESS;
   }
 
-  if (!in_bitrev_gather && ba_use_latency_passes(ctx, log_n, n2b, num_cols, lat)) {
+  // an LDE call's coset NTTs: by the elements of all its cosets (a tuned tile_log is for plain NTTs)
+  const bool latency = in_bitrev_gather
+                           ? lat == BA_LAT_AUTO && ba_latency_shape_exists(log_n) &&
+                                 small_batch((uint64_t)num_cols * cosets, log_n)
+                           : ba_use_latency_passes(ctx, log_n, n2b, num_cols, lat);
+  if (latency) {
     uint32_t bits[2];
     const int np = lat_bits(log_n, bits);
     for (int p = 0; p < np; p++) {
@@ -241,7 +254,8 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
       a.num_cols = num_cols;
       a.lo_bit = lo;
       a.reps = 1;
-      a.in_canonical = p > 0;
+      a.in_canonical = p > 0 || in_bitrev_gather;
+      a.in_bitrev = in_bitrev_gather && p == 0;
       a.scale = (pre && p == 0) ? SCALE_PRE : ((inverse && p == np - 1) ? SCALE_POST : SCALE_NONE);
       const bool scale = a.scale != SCALE_NONE;
       const uint64_t chunks = (uint64_t)num_cols << (log_n - S);
@@ -249,10 +263,11 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
                        : (chunks + (1u << (LAT_TL - S)) - 1) >> (LAT_TL - S);
       a.tile_count = (uint32_t)l.grid;
       l.kernels = ba_pick_lat(S, strided, n2b, inverse, top, scale);
+      if (a.in_bitrev) l.coset_kernel = ba_pick_lat_cosets(S, strided);
       l.name = ba_lat_kernel_name(S, strided, n2b, inverse, top, scale);
       l.pass = p;
       l.col0 = 0;
-      if (!l.kernels.single) return BA_ERROR_INVALID_VALUE;
+      if (!l.kernels.single || (a.in_bitrev && !l.coset_kernel)) return BA_ERROR_INVALID_VALUE;
       launches.push_back(l);
     }
     return BA_SUCCESS;
@@ -273,7 +288,7 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
     const uint32_t log_stride = big ? log_n - TILE_LOG : 0;
     const uint32_t cols_per_tile = big ? 1 : (1u << (TILE_LOG - log_n));
     // launch column groups small enough for 32-bit tile counts and grids
-    const uint64_t max_cols = big ? std::max<uint64_t>(1, (kMaxGrid >> log_stride)) : kMaxGrid;
+    const uint64_t max_cols = (big ? std::max<uint64_t>(1, (kMaxGrid >> log_stride)) : kMaxGrid) / cosets;
     for (uint64_t c0 = 0; c0 < num_cols; c0 += max_cols) {
       const uint32_t nc = (uint32_t)std::min<uint64_t>(max_cols, num_cols - c0);
       const uint64_t tiles = big ? ((uint64_t)nc << log_stride) : (nc + cols_per_tile - 1) / cols_per_tile;
@@ -290,7 +305,7 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
       a.log_tile_stride = log_stride;
       const uint32_t tuned_reps = tuning.valid ? tuning.reps[p] : 0;
       a.reps = tuned_reps ? std::min<uint32_t>(tuned_reps, big ? nc : (uint32_t)tiles)
-                     : ba_pick_reps(tiles, big ? nc : (uint32_t)tiles);
+                     : ba_pick_reps(tiles * cosets, big ? nc : (uint32_t)tiles);
       if (a.reps == 0) a.reps = 1;
       a.scale = (pre && p == 0) ? SCALE_PRE
                                 : ((inverse && p == plan.num_passes - 1) ? SCALE_POST : SCALE_NONE);
@@ -308,14 +323,19 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
       // sets the time -- and 4 waves above
       uint32_t waves = 3;
       if (contig && S >= 9)
-        waves = tuning.valid && tuning.contig_waves ? tuning.contig_waves : (l.grid < 2048 ? 3 : 4);
+        waves = tuning.valid && tuning.contig_waves ? tuning.contig_waves : (l.grid * cosets < 2048 ? 3 : 4);
       l.kernels = pick_kernel(contig, S, n2b, inverse, top, scale, big, gather, waves, shared);
       const bool shared_build =
           shared && !contig && l.kernels.single != pick_kernel(contig, S, n2b, inverse, top, scale, big, gather, waves, false).single;
       l.name = kernel_name(contig, S, n2b, inverse, contig ? big : top, scale, gather, waves, shared_build);
+      if (a.in_bitrev)
+        l.coset_kernel = !contig      ? ba_pick_strided_cosets(S)
+                         : S <= 8     ? ba_pick_contig_lo_cosets(S)
+                         : waves == 3 ? ba_pick_contig_hi3_cosets(S)
+                                      : ba_pick_contig_hi_cosets(S);
       l.pass = p;
       l.col0 = c0;
-      if (!l.kernels.single) return BA_ERROR_INVALID_VALUE;
+      if (!l.kernels.single || (a.in_bitrev && !l.coset_kernel)) return BA_ERROR_INVALID_VALUE;
       launches.push_back(l);
     }
   }

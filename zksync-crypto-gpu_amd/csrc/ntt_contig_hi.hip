@@ -50,3 +50,17 @@ BaKernels ba_pick_contig_hi(uint32_t S, bool n2b, bool inverse, int scale, bool 
   }
   return {nullptr, nullptr};
 }
+
+#if BA_CONTIG_W == 3
+BaCosetKernel ba_pick_contig_hi3_cosets(uint32_t S) {
+#else
+BaCosetKernel ba_pick_contig_hi_cosets(uint32_t S) {
+#endif
+  switch (S) {
+    case 9: return ntt_pass_contig_cosets<9, false, BA_CONTIG_W>;
+    case 10: return ntt_pass_contig_cosets<10, false, BA_CONTIG_W>;
+    case 11: return ntt_pass_contig_cosets<11, false, BA_CONTIG_W>;
+    case 12: return ntt_pass_contig_cosets<12, true, BA_CONTIG_W>;
+  }
+  return nullptr;
+}

@@ -42,3 +42,14 @@ BaKernels ba_pick_contig_lo(uint32_t S, bool n2b, bool inverse, int scale, bool 
   }
   return {nullptr, nullptr};
 }
+
+BaCosetKernel ba_pick_contig_lo_cosets(uint32_t S) {
+  switch (S) {
+    case 4: return ntt_pass_contig_cosets<4, false, 3>;
+    case 5: return ntt_pass_contig_cosets<5, false, 3>;
+    case 6: return ntt_pass_contig_cosets<6, false, 3>;
+    case 7: return ntt_pass_contig_cosets<7, false, 3>;
+    case 8: return ntt_pass_contig_cosets<8, false, 3>;
+  }
+  return nullptr;
+}

@@ -8,6 +8,8 @@
 typedef void (*BaPassKernel)(gl::ntt::PassArgs);
 typedef void (*BaGroupKernel)(const gl::ntt::PassArgs *, const uint32_t *, uint32_t);
 
+typedef void (*BaCosetKernel)(gl::ntt::CosetArgs);
+
 struct BaKernels {
   BaPassKernel single;
   BaGroupKernel group;
@@ -31,3 +33,11 @@ constexpr int BA_LAT_MIN_CONTIG = 4, BA_LAT_MAX_CONTIG = 10;
 constexpr int BA_LAT_MIN_STRIDED = 5, BA_LAT_MAX_STRIDED = 8;
 BaKernels ba_pick_lat(uint32_t S, bool strided, bool n2b, bool inverse, bool top, bool scale);
 const char *ba_lat_kernel_name(uint32_t S, bool strided, bool n2b, bool inverse, bool top, bool scale);
+
+// the first pass of several coset NTTs of an LDE (gathered, coset-scaled n2b forward): strided over
+// 4..8 bits; contiguous over the whole column of 4..8 / 9..12 bits (waves 4 or 3); latency-shaped
+BaCosetKernel ba_pick_strided_cosets(uint32_t S);
+BaCosetKernel ba_pick_contig_lo_cosets(uint32_t S);
+BaCosetKernel ba_pick_contig_hi_cosets(uint32_t S);
+BaCosetKernel ba_pick_contig_hi3_cosets(uint32_t S);
+BaCosetKernel ba_pick_lat_cosets(uint32_t S, bool strided);

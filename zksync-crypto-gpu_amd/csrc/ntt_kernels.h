@@ -275,9 +275,47 @@ struct PassArgs {
   // from separate buffers), else at in + k * stride_in / out + k * stride_out
   const u64 *const *in_cols;
   u64 *const *out_cols;
+  u64 slice_stride;      // grid slice y (blockIdx.y) reads and writes y slice_stride elements further
+                         // on: one launch for a later pass of an LDE's cosets (base and stride form)
   u64 scale_tab[VALS];   // T[m]
   Tables tab;
 };
+
+__device__ __forceinline__ void to_slice(PassArgs &a) {
+  const u64 at = blockIdx.y * a.slice_stride;
+  a.in += at;
+  a.out += at;
+}
+
+// The first pass of up to MAX_COSETS coset NTTs of one LDE in one launch.  They read the same
+// monomials and differ in their outputs and scale factors.  Workgroups of the cosets alternate, on
+// the same XCD (workgroups are dealt round-robin over the 8 XCDs), so the monomials of a tile are
+// read from HBM once and from L2 for the other cosets (64 x 2^20 at blowup 2: 1561 us by this order,
+// 1575 with plainly alternating workgroups, 1593 one coset after the other, 1606 as two launches on
+// two streams; 16 x 2^22 at blowup 4: 3300, 3346, 3568 and 3430).
+constexpr int MAX_COSETS = 8;
+struct CosetArgs {
+  PassArgs a;
+  u64 coset_stride;            // coset y's outputs start at a.out + y coset_stride
+  u32 log_cosets;
+  u32 coset_mul[MAX_COSETS];   // PassArgs::coset_mul and scale_tab of coset y
+  u64 scale_tab[MAX_COSETS][VALS];
+};
+// The workgroup's coset's arguments; returns its tile and the tile count through `tiles`.
+__device__ __forceinline__ u32 enter_coset(const CosetArgs &c, PassArgs &a, u32 &tiles) {
+  const u32 b = blockIdx.x, lc = c.log_cosets;
+  tiles = gridDim.x >> lc;
+  const bool by_xcd = (tiles & 7u) == 0;
+  const u32 y = (by_xcd ? b >> 3 : b) & ((1u << lc) - 1);
+  a = c.a;
+  a.out += y * c.coset_stride;
+  a.coset_mul = c.coset_mul[y];
+  static_for<VALS>([&](auto m_) {
+    constexpr int m = decltype(m_)::value;
+    a.scale_tab[m] = c.scale_tab[y][m];
+  });
+  return by_xcd ? ((b >> (3 + lc)) << 3) | (b & 7u) : b >> lc;
+}
 
 __device__ __forceinline__ const u64 *col_in(const PassArgs &a, u64 col) {
   return a.in_cols ? gload(a.in_cols + col) : a.in + col * a.stride_in;
@@ -898,21 +936,31 @@ __device__ __forceinline__ u32 group_of(const u32 *wg_start, u32 njobs, u32 b) {
 #define BA_XCD_REMAP_MAX_S 4
 #endif
 template <int S>
-__device__ __forceinline__ u32 strided_tile() {
+__device__ __forceinline__ u32 strided_tile(const u32 b, const u32 G) {
   if constexpr (S <= BA_XCD_REMAP_MAX_S || S >= 9) {
     // Workgroups are dealt round-robin over the 8 XCDs, so neighbouring tiles (neighbouring runs
     // of the same 2^S rows, 2^(log_n - S) elements apart) would run at once on all eight and
     // crowd the same HBM channels.  XCD x instead takes the contiguous tile range starting at
     // x q + min(x, r), q or q + 1 tiles (q = G / 8, r = G % 8): a bijection on [0, G).
-    const u32 G = gridDim.x, b = blockIdx.x, x = b & 7u, q = G >> 3, r = G & 7u;
+    const u32 x = b & 7u, q = G >> 3, r = G & 7u;
     return x * q + (x < r ? x : r) + (b >> 3);
   } else {
-    return blockIdx.x;
+    return b;
   }
 }
 template <int S, bool N2B, bool INV, bool TOP, bool SCALE, bool GATHER>
 __global__ __launch_bounds__(THREADS) void ntt_pass_strided(PassArgs a) {
-  strided_body<S, N2B, INV, TOP, SCALE, GATHER, !strided_four_waves<S, TOP, GATHER>()>(a, strided_tile<S>());
+  to_slice(a);
+  strided_body<S, N2B, INV, TOP, SCALE, GATHER, !strided_four_waves<S, TOP, GATHER>()>(
+      a, strided_tile<S>(blockIdx.x, gridDim.x));
+}
+// the LDE's gathered, scaled first pass over several cosets
+template <int S>
+__global__ __launch_bounds__(THREADS) void ntt_pass_strided_cosets(CosetArgs c) {
+  PassArgs a;
+  u32 tiles;
+  const u32 tile = enter_coset(c, a, tiles);
+  strided_body<S, true, false, true, true, true, !strided_four_waves<S, true, true>()>(a, strided_tile<S>(tile, tiles));
 }
 template <int S, bool N2B, bool INV, bool TOP, bool SCALE, bool GATHER>
 __global__ __launch_bounds__(THREADS) void ntt_pass_strided_group(const PassArgs *jobs, const u32 *wg_start,
@@ -924,7 +972,7 @@ __global__ __launch_bounds__(THREADS) void ntt_pass_strided_group(const PassArgs
 // the prefetching three-waves build of a four-waves variant, for launches that share the GPU
 template <int S, bool N2B, bool INV, bool TOP, bool SCALE, bool GATHER>
 __global__ __launch_bounds__(THREADS) void ntt_pass_strided_shared(PassArgs a) {
-  strided_body<S, N2B, INV, TOP, SCALE, GATHER, true>(a, strided_tile<S>());
+  strided_body<S, N2B, INV, TOP, SCALE, GATHER, true>(a, strided_tile<S>(blockIdx.x, gridDim.x));
 }
 template <int S, bool N2B, bool INV, bool TOP, bool SCALE, bool GATHER>
 __global__ __launch_bounds__(THREADS) void ntt_pass_strided_shared_group(const PassArgs *jobs,
@@ -939,7 +987,16 @@ __global__ __launch_bounds__(THREADS) void ntt_pass_strided_shared_group(const P
 // The autotuner picks W per size class (ba_tuned_plan.contig_waves).
 template <int S, bool N2B, bool INV, int SC, bool WHOLE, int W>
 __global__ __launch_bounds__(THREADS, SC == 2 && !WHOLE ? 2 : W) void ntt_pass_contig(PassArgs a) {
+  to_slice(a);
   contig_body<S, N2B, INV, SC, WHOLE, W == 3>(a, blockIdx.x);
+}
+// the LDE's only pass over columns of at most 4096 elements, several cosets
+template <int S, bool WHOLE, int W>
+__global__ __launch_bounds__(THREADS, WHOLE ? W : 2) void ntt_pass_contig_cosets(CosetArgs c) {
+  PassArgs a;
+  u32 tiles;
+  const u32 tile = enter_coset(c, a, tiles);
+  contig_body<S, true, false, 2, WHOLE, W == 3>(a, tile);
 }
 template <int S, bool N2B, bool INV, int SC, bool WHOLE, int W>
 __global__ __launch_bounds__(THREADS, SC == 2 && !WHOLE ? 2 : W) void ntt_pass_contig_group(const PassArgs *jobs,

@@ -58,7 +58,10 @@ __device__ __forceinline__ u32 window2(u32 q, u32 m) {
 // STRIDED: bits [lo_bit, lo_bit + S) (TOP: they are the top bits); else bits [0, S).
 // SCALE: this pass applies the fused scale (forward: before its first round, which then is
 // the transform's first; inverse: after its last).
-template <int S, bool N2B, bool INV, bool STRIDED, bool TOP, bool SCALE>
+// GATHER: the transform's first pass reads a column stored bit-reversed (an LDE's monomials); the
+// strided pass reads its C chunks of 2^S in address order and reverses in LDS, the contiguous one
+// (the whole column) reads each element where it is.
+template <int S, bool N2B, bool INV, bool STRIDED, bool TOP, bool SCALE, bool GATHER = false>
 __device__ __forceinline__ void lat_body(const PassArgs &a, const u32 bid) {
   using Sh = Shape2<S, N2B>;
   constexpr int R = Sh::ROUNDS;
@@ -93,21 +96,39 @@ __device__ __forceinline__ void lat_body(const PassArgs &a, const u32 bid) {
   const u64 *in = col_in(a, col);
   u64 *out = col_out(a, col);
   // LDS slot of tile element (c, r)
-  auto slot = [&](u32 r) {
-    const u32 u = STRIDED ? r * C + c : (c << S) + r;
+  auto slot_of = [&](u32 cc, u32 r) {
+    const u32 u = STRIDED ? r * C + cc : (cc << S) + r;
     return u + (u >> 4);
   };
+  auto slot = [&](u32 r) { return slot_of(c, r); };
   auto pos = [&](u32 r) { return pos0 + (r << P0); };
   const bool top = STRIDED ? TOP : (S == L);  // the pass holds the top bits: one round has no twiddle
 
   // first round's elements, then every round's twiddle powers (W^1..W^3 per round)
   u64 v[VALS];
   constexpr int WB0 = Sh::WB(0);
-  static_for<4>([&](auto m_) {
-    constexpr int m = decltype(m_)::value;
-    const u64 x = valid ? gload(in + pos(window2<WB0>(q, m))) : 0;
-    v[m] = a.in_canonical ? x : canon(x);
-  });
+  if constexpr (GATHER && STRIDED) {
+    static_assert(TOP && N2B, "the gathered pass is the n2b top pass");
+    const u32 l0 = pos0 - c;  // the tile's first column (the pass holds the top bits)
+    u64 x[4];
+    static_for<4>([&](auto k_) {
+      constexpr int k = decltype(k_)::value;
+      const u32 e = t + THREADS * k;
+      x[k] = gload(in + ((bitrev32(l0 + (e >> S), P0) << S) | (e & ((1u << S) - 1))));
+    });
+    static_for<4>([&](auto k_) {
+      constexpr int k = decltype(k_)::value;
+      const u32 e = t + THREADS * k;
+      lds[slot_of(e >> S, bitrev32(e & ((1u << S) - 1), S))] = a.in_canonical ? x[k] : canon(x[k]);
+    });
+  } else {
+    static_for<4>([&](auto m_) {
+      constexpr int m = decltype(m_)::value;
+      const u32 at = pos(window2<WB0>(q, m));
+      const u64 x = valid ? gload(in + (GATHER ? bitrev32(at, L) : at)) : 0;
+      v[m] = a.in_canonical ? x : canon(x);
+    });
+  }
   u64 tw[R][4];
   static_for<R>([&](auto r_) {
     constexpr int r = decltype(r_)::value;
@@ -129,6 +150,13 @@ __device__ __forceinline__ void lat_body(const PassArgs &a, const u32 bid) {
       v[m] = mul(v[m], a.scale_coset ? mul(f, tm) : tm);
     });
   };
+  if constexpr (GATHER && STRIDED) {  // each thread then writes back only the slots it reads
+    __syncthreads();
+    static_for<4>([&](auto m_) {
+      constexpr int m = decltype(m_)::value;
+      v[m] = lds[slot(window2<WB0>(q, m))];
+    });
+  }
   if constexpr (SCALE && !INV) scale4(pos(window2<WB0>(q, 0)));
 
   static_for<R>([&](auto r_) {
@@ -182,7 +210,16 @@ __device__ __forceinline__ void lat_body(const PassArgs &a, const u32 bid) {
 
 template <int S, bool N2B, bool INV, bool STRIDED, bool TOP, bool SCALE>
 __global__ __launch_bounds__(THREADS) void ntt_pass_lat(PassArgs a) {
+  to_slice(a);
   lat_body<S, N2B, INV, STRIDED, TOP, SCALE>(a, blockIdx.x);
+}
+// the LDE's gathered, scaled first pass over several cosets
+template <int S, bool STRIDED>
+__global__ __launch_bounds__(THREADS) void ntt_pass_lat_cosets(CosetArgs c) {
+  PassArgs a;
+  u32 tiles;
+  const u32 tile = enter_coset(c, a, tiles);
+  lat_body<S, true, false, STRIDED, STRIDED, true, true>(a, tile);
 }
 // a group of batches (batch plans), as the grouped throughput passes
 template <int S, bool N2B, bool INV, bool STRIDED, bool TOP, bool SCALE>

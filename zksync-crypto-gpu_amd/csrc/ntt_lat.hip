@@ -45,6 +45,29 @@ BaKernels ba_pick_lat(uint32_t S, bool strided, bool n2b, bool inverse, bool top
   return {nullptr, nullptr};
 }
 
+template <int S>
+static BaCosetKernel pick_cosets(bool strided) {
+  if (strided) {
+    if constexpr (S >= BA_LAT_MIN_STRIDED && S <= BA_LAT_MAX_STRIDED) return ntt_pass_lat_cosets<S, true>;
+  } else {
+    if constexpr (S >= BA_LAT_MIN_CONTIG && S <= BA_LAT_MAX_CONTIG) return ntt_pass_lat_cosets<S, false>;
+  }
+  return nullptr;
+}
+
+BaCosetKernel ba_pick_lat_cosets(uint32_t S, bool strided) {
+  switch (S) {
+    case 4: return pick_cosets<4>(strided);
+    case 5: return pick_cosets<5>(strided);
+    case 6: return pick_cosets<6>(strided);
+    case 7: return pick_cosets<7>(strided);
+    case 8: return pick_cosets<8>(strided);
+    case 9: return pick_cosets<9>(strided);
+    case 10: return pick_cosets<10>(strided);
+  }
+  return nullptr;
+}
+
 namespace {
 // [S][n2b][inverse][strided][top][scale], as rocprofv3 prints them; built by the first caller
 // (a function-local static initialiser, so concurrent first calls are safe)

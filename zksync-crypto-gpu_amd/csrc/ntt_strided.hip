@@ -65,3 +65,14 @@ BaKernels ba_pick_tiny(uint32_t log_n, bool n2b, bool inverse) {
 #undef BA_TINY
   return {nullptr, nullptr};
 }
+
+BaCosetKernel ba_pick_strided_cosets(uint32_t S) {
+  switch (S) {
+    case 4: return ntt_pass_strided_cosets<4>;
+    case 5: return ntt_pass_strided_cosets<5>;
+    case 6: return ntt_pass_strided_cosets<6>;
+    case 7: return ntt_pass_strided_cosets<7>;
+    case 8: return ntt_pass_strided_cosets<8>;
+  }
+  return nullptr;
+}
