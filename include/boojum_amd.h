@@ -266,7 +266,7 @@ int ba_batch_plan_destroy(ba_batch_plan_t plan);
  * per pass in the same order, the columns each workgroup repeats over (reps, 1..8; 0 = built-in
  * choice), and the waves per SIMD of a 9..12-bit contiguous pass (contig_waves: 3 = the variant
  * that loads the next tile while transforming, 4 = the 128-register variant without that
- * prefetch, 0 = built-in choice: 3 below 2048 workgroups, else 4), and the tile shape of plain
+ * prefetch, 0 = built-in choice: 4), and the tile shape of plain
  * batch NTTs (tile_log: 10 = the latency-shaped passes, 1024-element tiles of 4 elements per
  * thread in radix-4 rounds, for every batch size, log_n 4..18 only; 12 = the 4096-element tiles
  * of the split above for every batch size; 0 = built-in choice: 1024-element tiles for batches of

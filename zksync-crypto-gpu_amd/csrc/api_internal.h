@@ -121,7 +121,6 @@ bool ba_latency_shape_exists(uint32_t log_n);
 bool ba_use_latency_passes(const ba_context *ctx, uint32_t log_n, bool n2b, uint32_t num_cols, BaLatPolicy lat);
 // Launches them one after another on `stream` (single-batch kernels).
 int ba_run_launches(const std::vector<BaPassLaunch> &launches, hipStream_t stream);
-uint32_t ba_pick_reps(uint64_t tiles, uint32_t cols);
 
 // A pass launch tagged with its dependency level inside a batch plan: every launch at level l
 // only reads what launches at levels < l wrote.

@@ -134,12 +134,40 @@ constexpr uint64_t kMaxGrid = 0x7FFFFFFFull;
 
 }  // namespace
 
-// Columns (tile repeats) per workgroup: enough to amortise the twiddle and scale-factor set-up,
-// while keeping >= ~1024 workgroups (4 per CU) in flight.
-uint32_t ba_pick_reps(uint64_t tiles, uint32_t cols) {
-  uint32_t reps = 1;
-  while (reps < 8 && reps < cols && tiles / (2ull * reps) >= 1024) reps *= 2;
-  return reps;
+// Columns (tile repeats) per workgroup, at most 8.  More of them spread the workgroup's set-up (round
+// twiddles, scale factors) over more tiles, but leave fewer workgroups to even out the last ones:
+// 1024 run at once (4 per CU).  `tiles` counts every tile of the launch, `cols` what a workgroup may
+// repeat over.  The lines are measured; microseconds per launch, by columns per workgroup:
+//   contiguous, 12 bits:  1792 tiles: 47 (1), 41 (2), 53 (4); 4096: 85, 85, 85, 104 (8); 6400: 127 (1),
+//                         126 (2), 134 (4); 8192: 175, 158, 150 (3), 162 (8); 16384: 459 (1), 358 (2),
+//                         307 (5), 313 (8).  From 14336 tiles on, 8 where that leaves a shorter last
+//                         group (19 columns of 2^22: 340 against 356 by 5) and 5 where it divides
+//                         (16 of 2^22: 287 against 307 by 8): workgroups of one length run in step,
+//                         all loading and all computing at once.  A transform's only pass (short
+//                         columns) takes 8: 16384 columns of 2^12 354 against 360 by 5.
+//   strided, plain top pass: hardly any set-up (one round without twiddles) and HBM-bound:
+//                         4 bits 2^26 elements: 180 (1), 189 (8); 5 bits 144 (1), 171 (4); 6 bits 184 (1),
+//                         209 (8); 7 bits 204 (1), 199 (2), 213 (8); 8 bits 2^27: 439 (1), 424 (2), 450 (8);
+//                         below the top, 6 bits: 198 (1), 181 (3), 191 (8).
+//   strided, one factor for every element (n^-1): 4 bits 185 (1), 204 (8); 5 bits 177 (1), 158 (3), 176 (8);
+//                         8 bits 257 (1), 242 (2..8).
+//   strided, a factor per element (coset, gathered coset pass): 16 factors of set-up.  4 bits 263 (1),
+//                         252 (4), 272 (8); 5 bits 215 (1), 177 (5), 195 (8); 6 bits 290 (1), 222 (7);
+//                         8 bits 341 (1), 256 (7).  At least 768 workgroups: 2^24 elements by 8 bits
+//                         77 (3), 72 (5), 80 (8).
+static uint32_t pick_reps(bool contig, uint32_t S, bool top, int scale, uint64_t tiles, uint32_t cols,
+                          bool only_pass) {
+  uint32_t reps;
+  if (contig) {
+    reps = tiles < 1536 ? 1 : tiles < 7168 ? 2 : tiles < 14336 ? 3 : only_pass || cols % 8 ? 8 : 5;
+  } else if (scale == 2) {
+    reps = std::min<uint32_t>(S == 4 ? 4 : S == 5 ? 5 : 7, (uint32_t)std::min<uint64_t>(8, tiles / 768));
+  } else if (scale == 1) {
+    reps = S == 4 ? 1 : 3;
+  } else {
+    reps = !top ? 3 : S <= 6 ? 1 : 2;
+  }
+  return std::max(1u, std::min(reps, cols));
 }
 
 // Latency-shaped plan (ntt_lat.h): the bits of each pass from the low bits up (a contiguous
@@ -303,27 +331,25 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
       a.lo_bit = plan.lo_bit[p];
       a.tile_count = (uint32_t)tiles;
       a.log_tile_stride = log_stride;
-      const uint32_t tuned_reps = tuning.valid ? tuning.reps[p] : 0;
-      a.reps = tuned_reps ? std::min<uint32_t>(tuned_reps, big ? nc : (uint32_t)tiles)
-                     : ba_pick_reps(tiles * cosets, big ? nc : (uint32_t)tiles);
-      if (a.reps == 0) a.reps = 1;
       a.scale = (pre && p == 0) ? SCALE_PRE
                                 : ((inverse && p == plan.num_passes - 1) ? SCALE_POST : SCALE_NONE);
       a.in_bitrev = in_bitrev_gather && p == 0;
       // later passes read this transform's own output, and the gathered LDE coset pass reads the
       // monomials the inverse NTT wrote: values < p
       a.in_canonical = p > 0 || in_bitrev_gather;
-      const uint64_t groups = big ? (nc + a.reps - 1) / a.reps : (tiles + a.reps - 1) / a.reps;
-      l.grid = groups << log_stride;
       const bool top = plan.lo_bit[p] + S == log_n;
       const int scale = a.scale == SCALE_NONE ? 0 : (a.scale_coset ? 2 : 1);
+      const uint32_t tuned_reps = tuning.valid ? tuning.reps[p] : 0;
+      const uint32_t most = big ? nc : (uint32_t)tiles;
+      a.reps = std::max(1u, tuned_reps ? std::min(tuned_reps, most)
+                                       : pick_reps(contig, S, top, scale, tiles * cosets, most, log_n == S));
+      const uint64_t groups = big ? (nc + a.reps - 1) / a.reps : (tiles + a.reps - 1) / a.reps;
+      l.grid = groups << log_stride;
       const bool gather = !contig && a.in_bitrev;
-      // the 9..12-bit contiguous pass: as tuned, else 3 waves per SIMD (with the next-tile
-      // prefetch) below 2048 workgroups -- few tiles, where a workgroup's own instruction stream
-      // sets the time -- and 4 waves above
-      uint32_t waves = 3;
-      if (contig && S >= 9)
-        waves = tuning.valid && tuning.contig_waves ? tuning.contig_waves : (l.grid * cosets < 2048 ? 3 : 4);
+      // the 9..12-bit contiguous pass: as tuned, else 4 waves per SIMD.  (The three-waves build with its
+      // prefetch takes as long on up to 512 tiles, 18 and 22 us, and longer above: 34.6 against 29.9 us
+      // on 1024 tiles, 146 against 127 on 6400.)
+      const uint32_t waves = S < 9 ? 3 : tuning.valid && tuning.contig_waves ? tuning.contig_waves : 4;
       l.kernels = pick_kernel(contig, S, n2b, inverse, top, scale, big, gather, waves, shared);
       const bool shared_build =
           shared && !contig && l.kernels.single != pick_kernel(contig, S, n2b, inverse, top, scale, big, gather, waves, false).single;
