@@ -341,3 +341,27 @@ def test_stepped_powers_past_the_grid_stride(ba, tables):
     finally:
         d.free()
         d_src.free()
+
+
+# From 2^22 elements a lane of the stepped kernels has several elements, four at a time and a remainder.
+@pytest.mark.parametrize("count", [(1 << 22) - 1, (1 << 22) + 1, (1 << 24) - 5, (1 << 24) + 3, 5 * (1 << 22) + 77])
+def test_omega_shift_and_powers_of_long_vectors(ba, count):
+    log_degree, offset, shift = 26, 12345, 3
+    x = raw_u64(np.random.default_rng(count), count)
+    d_x, d_y = ba.DeviceAllocation.from_host(x), ba.DeviceAllocation(count)
+    try:
+        for inverse in (False, True):
+            log(f"omega shift of {count} inverse={inverse}")
+            want = gl_oracle.omega_shift(x, log_degree, offset, inverse, shift)
+            ba.ops.omega_shift(d_x, log_degree, offset, inverse, shift, d_y)
+            ba.synchronize()
+            assert np.array_equal(d_y.to_host(), want)
+            ba.ops.get_powers_of_w(log_degree, offset, inverse, False, d_y)
+            ba.synchronize()
+            assert np.array_equal(d_y.to_host(), gl_oracle.powers_of_w(log_degree, offset, inverse, False, count))
+        ba.ops.omega_shift_in_place(d_x, log_degree, offset, True, shift)
+        ba.synchronize()
+        assert np.array_equal(d_x.to_host(), want)
+    finally:
+        d_x.free()
+        d_y.free()

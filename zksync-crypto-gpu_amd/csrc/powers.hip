@@ -22,7 +22,13 @@ using gl::u64;
 
 constexpr u32 kThreads = 256;
 
-u32 grid_for(u64 count) { return (u32)std::max<u64>(1, std::min<u64>((count + kThreads - 1) / kThreads, 65536)); }
+u32 grid_for(u64 count, u32 most = 65536) {
+  return (u32)std::max<u64>(1, std::min<u64>((count + kThreads - 1) / kThreads, most));
+}
+// Kernels whose lanes step a power by the grid stride: fewer workgroups spread the first power over
+// more elements.  2^26 elements, omega shift and natural-order powers, us: 65536 workgroups 263 and 126,
+// 16384 227 and 100, 4096 237 and 111.
+constexpr u32 kSteppedGrid = 16384;
 
 __device__ __forceinline__ u32 raw_exponent(u32 i, u32 log_degree, bool bit_reverse) {
   return bit_reverse ? gl::ntt::bitrev32(i, log_degree) : i;
@@ -134,8 +140,12 @@ __global__ __launch_bounds__(kThreads) void powers_ef_kernel(const u64 *base_ptr
   }
 }
 
-// the exponent (shift (i + offset)) << degree_shift is linear in i modulo 2^30: each lane steps its
-// factor by omega^(+-((shift stride) << degree_shift)) per grid stride
+// The exponent (shift (i + offset)) << degree_shift is linear in i modulo 2^30: a lane's elements are a
+// grid stride apart and their factors step by one constant, omega^(+-((shift stride) << degree_shift)).
+// What bounds it: HBM (16 B per element).  A lane loads kShiftBatch elements before it multiplies any,
+// on a grid that fills the chip: 2^26 elements take 227 us (4.7 TB/s),
+// where one load, product and store at a time on four times the workgroups took 263.
+constexpr u32 kShiftBatch = 4;
 __global__ __launch_bounds__(kThreads) void omega_shift_kernel(gl::Tables tab, const u64 *src, u32 log_degree,
                                                                u32 offset, bool inverse, u32 shift, u64 *dst,
                                                                u32 count) {
@@ -145,11 +155,20 @@ __global__ __launch_bounds__(kThreads) void omega_shift_kernel(gl::Tables tab, c
   if (i >= count) return;
   u64 w = gl::pow_w(tab, (shift * (i + offset)) << degree_shift, inverse);
   const u64 step = gl::pow_w(tab, (shift * stride) << degree_shift, inverse);
-  for (;;) {
+  u32 left = (count - 1 - i) / stride + 1;  // this lane's elements
+  for (; left >= kShiftBatch; left -= kShiftBatch, i += kShiftBatch * stride) {
+    u64 x[kShiftBatch];
+#pragma unroll
+    for (u32 k = 0; k < kShiftBatch; k++) x[k] = src[i + k * stride];
+#pragma unroll
+    for (u32 k = 0; k < kShiftBatch; k++) {
+      dst[i + k * stride] = gl::mul(x[k], w);
+      w = gl::mul_lazy(w, step);
+    }
+  }
+  for (; left; left--, i += stride) {
     dst[i] = gl::mul(src[i], w);
-    if (count - i <= stride) break;
-    i += stride;
-    w = gl::mul(w, step);
+    w = gl::mul_lazy(w, step);
   }
 }
 
@@ -168,7 +187,8 @@ extern "C" int ba_get_powers_of_w(uint32_t log_degree, uint32_t offset, int inve
   const gl::Tables *t;
   if (int rc = tables(&t)) return rc;
   if (!count) return BA_SUCCESS;
-  hipLaunchKernelGGL(powers_of_w_kernel, dim3(grid_for(count)), dim3(kThreads), 0, (hipStream_t)stream, *t,
+  const u32 grid = bit_reverse ? grid_for(count) : grid_for(count, kSteppedGrid);
+  hipLaunchKernelGGL(powers_of_w_kernel, dim3(grid), dim3(kThreads), 0, (hipStream_t)stream, *t,
                      log_degree, offset, inverse != 0, bit_reverse != 0, result, count);
   return (int)hipGetLastError();
 }
@@ -229,7 +249,7 @@ extern "C" int ba_omega_shift(const uint64_t *src, uint32_t log_degree, uint32_t
   const gl::Tables *t;
   if (int rc = tables(&t)) return rc;
   if (!count) return BA_SUCCESS;
-  hipLaunchKernelGGL(omega_shift_kernel, dim3(grid_for(count)), dim3(kThreads), 0, (hipStream_t)stream, *t, src,
+  hipLaunchKernelGGL(omega_shift_kernel, dim3(grid_for(count, kSteppedGrid)), dim3(kThreads), 0, (hipStream_t)stream, *t, src,
                      log_degree, offset, inverse != 0, shift, dst, count);
   return (int)hipGetLastError();
 }
