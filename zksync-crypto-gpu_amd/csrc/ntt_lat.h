@@ -134,10 +134,18 @@ __device__ __forceinline__ void lat_body(const PassArgs &a, const u32 bid) {
     constexpr int r = decltype(r_)::value;
     constexpr int K = Sh::K(r);
     const u32 e = round_exp(a, pos(window2<Sh::WB(r)>(q, 0)), P0 + Sh::AB(r), K);
-    static_for<(1 << K)>([&](auto i_) {
-      constexpr int i = decltype(i_)::value;
-      if constexpr (i > 0) tw[r][i] = e ? pow_w(a.tab, e * i, INV) : 1;
-    });
+    // Contiguous passes of 7 and 8 bits, whose reads scatter over the table, read W and multiply its
+    // powers: two reads per round instead of six (2^16 in two passes 11.4 -> 10.9 us).  Narrower, wider
+    // and strided ones keep the shorter chain: with the products 2^12 takes 8.8 us instead of 8.6, 2^10
+    // 6.0 instead of 5.4 and 4 columns of 2^18 26.0 instead of 24.9.
+    tw[r][1] = e ? pow_w(a.tab, e, INV) : 1;
+    if constexpr (K == 2 && !STRIDED && (S == 7 || S == 8)) {
+      tw[r][2] = sqr(tw[r][1]);
+      tw[r][3] = mul(tw[r][2], tw[r][1]);
+    } else if constexpr (K == 2) {
+      tw[r][2] = e ? pow_w(a.tab, e * 2, INV) : 1;
+      tw[r][3] = e ? pow_w(a.tab, e * 3, INV) : 1;
+    }
   });
   // fused scale: natural j0 of register 0 of the scaled round and the factor of register m
   constexpr bool PERM = N2B != !INV;  // the scaled round's layout is bit-reversed
