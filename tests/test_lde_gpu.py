@@ -281,7 +281,7 @@ def test_lde_graph_replay(ba, lb):
 # tiles; 16 and 32 cosets take two and four rounds of launches; tile counts that 8 divides and that it does not.
 @pytest.mark.parametrize("log_n,cols,lb", [(4, 1, 1), (4, 300, 5), (5, 7, 4), (7, 33, 3), (9, 3, 5), (10, 5, 2),
                                            (11, 1, 1), (11, 5, 4), (12, 3, 3), (13, 1, 2), (15, 3, 1), (17, 3, 1),
-                                           (18, 1, 1), (18, 1, 3), (19, 1, 2),
+                                           (18, 1, 1), (18, 1, 3), (19, 1, 2), (11, 256, 2), (11, 257, 2), (12, 23, 2), (12, 24, 2), (12, 65, 2),
                                            (4, 40001, 1), (8, 3000, 1), (9, 1501, 1), (10, 700, 2), (11, 300, 3),
                                            (12, 70, 3), (13, 43, 3), (14, 21, 3), (15, 37, 1), (16, 5, 4)])
 @pytest.mark.parametrize("layout", ["column", "coset"])

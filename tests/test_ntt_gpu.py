@@ -297,3 +297,25 @@ def test_latency_path_choice_and_agreement(ba, log_n, cols):
     finally:
         for t in (a, b, c):
             t.free()
+
+
+# Whole columns of 2^11 and 2^12 per workgroup in one launch: either side of the column counts where the
+# launch rule changes (2^11: up to 1024 columns; 2^12: 96 to 256), every mode and fused scale.
+@pytest.mark.parametrize("log_n,cols", [(11, 1), (11, 37), (11, 1024), (11, 1025), (12, 95), (12, 96), (12, 256), (12, 257)])
+def test_whole_column_workgroups(ba, log_n, cols):
+    n, stride = 1 << log_n, (1 << log_n) + 3
+    x = raw_u64(np.random.default_rng(cols), cols * stride)
+    d_in, d_out = ba.DeviceAllocation.from_host(x), ba.DeviceAllocation.from_host(x)
+    try:
+        for bitrev in (False, True):
+            for inverse, lext, coset in ((False, 0, 0), (True, 0, 0), (False, 2, 3), (True, 1, 1)):
+                log(f"whole columns log_n={log_n} cols={cols} bitrev={bitrev} inverse={inverse} lext={lext}")
+                ba.ntt.batch_ntt_internal(d_in.ptr, d_out.ptr, log_n, cols, stride, stride, bitrev, inverse, lext, coset)
+                ba.synchronize()
+                want = gl_oracle.batch_ntt(x, log_n, cols, stride, stride, bitrev, inverse, lext, coset, nthreads=8)
+                got = d_out.to_host().reshape(cols, stride)
+                assert np.array_equal(got[:, :n], want.reshape(cols, stride)[:, :n])
+                assert np.array_equal(got[:, n:], x.reshape(cols, stride)[:, n:])
+    finally:
+        d_in.free()
+        d_out.free()

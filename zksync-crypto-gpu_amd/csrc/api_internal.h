@@ -86,6 +86,7 @@ struct BaPassLaunch {
   BaCosetKernel coset_kernel = nullptr;  // the gathered first pass of an LDE's coset NTTs
   gl::ntt::PassArgs args;
   uint64_t grid;
+  uint32_t threads = gl::ntt::THREADS;
   const char *name;
   int pass;       // index of the pass inside its transform
   uint64_t col0;  // first column of the transform this launch covers

@@ -157,12 +157,12 @@ static int lde_run_merged(const ba_context *ctx, uint64_t *evals, uint64_t in_st
     for (const BaPassLaunch &l : ls) {
       if (l.pass == 0) {
         first.a = l.args;
-        hipLaunchKernelGGL(l.coset_kernel, dim3((uint32_t)(l.grid << log_at_once)), dim3(gl::ntt::THREADS), 0, stream,
+        hipLaunchKernelGGL(l.coset_kernel, dim3((uint32_t)(l.grid << log_at_once)), dim3(l.threads), 0, stream,
                            first);
       } else {
         gl::ntt::PassArgs a = l.args;
         a.slice_stride = out_coset_stride;
-        hipLaunchKernelGGL(l.kernels.single, dim3((uint32_t)l.grid, at_once), dim3(gl::ntt::THREADS), 0, stream, a);
+        hipLaunchKernelGGL(l.kernels.single, dim3((uint32_t)l.grid, at_once), dim3(l.threads), 0, stream, a);
       }
       const hipError_t err = hipGetLastError();
       if (err != hipSuccess) return (int)err;

@@ -193,9 +193,16 @@ static uint32_t lat_max_log_elems() {
   return v;
 }
 
+// Columns that run a whole 2^11- or 2^12-element transform per workgroup (ntt_lat.h): every latency-
+// shaped batch of 2^11, which as one launch beats the 4096-element tiles up to 2^21 elements (us per
+// call, one launch / two / 4096-element tiles: 1 column 6.6 / 8.5, 256 7.7 / 11.0, 700 13.8 / 23 / 18,
+// 2048 28.1 / - / 28.9); of 2^12, whose 1024-thread workgroup is one chain per CU, those that give the
+// chip enough of them (1 column 9.5 / 8.5, 64 10.2 / 10.0, 128 10.7 / 11.5, 256 11.6 / 16.1).
+static bool wide_columns(uint32_t log_n, uint64_t cols) { return log_n == 11 || (log_n == 12 && cols >= 96); }
+
 static bool small_batch(uint64_t cols, uint32_t log_n) {
   const uint32_t m = lat_max_log_elems();
-  return m > 0 && (cols << log_n) <= (1ull << std::min(m, 40u));
+  return m > 0 && (cols << log_n) <= (1ull << std::min(m + (log_n == 11), 40u));
 }
 
 bool ba_latency_shape_exists(uint32_t log_n) {
@@ -265,6 +272,31 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
                            ? lat == BA_LAT_AUTO && ba_latency_shape_exists(log_n) &&
                                  small_batch((uint64_t)num_cols * cosets, log_n)
                            : ba_use_latency_passes(ctx, log_n, n2b, num_cols, lat);
+  // single calls only: a batch plan's groups have 256 threads per workgroup
+  if (latency && lat == BA_LAT_AUTO && wide_columns(log_n, (uint64_t)num_cols * cosets)) {
+    BaPassLaunch l;
+    PassArgs &a = l.args;
+    a = base;
+    a.in = in;
+    a.out = out;
+    a.stride_in = stride_in;
+    a.stride_out = stride_out;
+    a.num_cols = num_cols;
+    a.reps = 1;
+    a.in_canonical = in_bitrev_gather;
+    a.in_bitrev = in_bitrev_gather;
+    a.scale = pre ? SCALE_PRE : (inverse ? SCALE_POST : SCALE_NONE);
+    l.grid = num_cols;
+    a.tile_count = num_cols;
+    l.threads = (uint32_t)wide_threads((int)log_n);
+    l.kernels = {ba_pick_lat_wide(log_n, n2b, inverse, a.scale != SCALE_NONE), nullptr};
+    if (in_bitrev_gather) l.coset_kernel = ba_pick_lat_wide_cosets(log_n);
+    l.name = "ntt_pass_lat_wide";
+    l.pass = 0;
+    l.col0 = 0;
+    launches.push_back(l);
+    return BA_SUCCESS;
+  }
   if (latency) {
     uint32_t bits[2];
     const int np = lat_bits(log_n, bits);
@@ -371,7 +403,7 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
 int ba_run_launches(const std::vector<BaPassLaunch> &launches, hipStream_t stream) {
   for (const BaPassLaunch &l : launches) {
     ba_trace_before(stream, l.name);
-    hipLaunchKernelGGL(l.kernels.single, dim3((uint32_t)l.grid), dim3(THREADS), 0, stream, l.args);
+    hipLaunchKernelGGL(l.kernels.single, dim3((uint32_t)l.grid), dim3(l.threads), 0, stream, l.args);
     ba_trace_after(stream);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return (int)err;

@@ -41,3 +41,6 @@ BaCosetKernel ba_pick_contig_lo_cosets(uint32_t S);
 BaCosetKernel ba_pick_contig_hi_cosets(uint32_t S);
 BaCosetKernel ba_pick_contig_hi3_cosets(uint32_t S);
 BaCosetKernel ba_pick_lat_cosets(uint32_t S, bool strided);
+// whole columns of 2^11 and 2^12 per workgroup of 2^(S-2) threads (no grouped kernel)
+BaPassKernel ba_pick_lat_wide(uint32_t S, bool n2b, bool inverse, bool scale);
+BaCosetKernel ba_pick_lat_wide_cosets(uint32_t S);

@@ -61,14 +61,16 @@ __device__ __forceinline__ u32 window2(u32 q, u32 m) {
 // GATHER: the transform's first pass reads a column stored bit-reversed (an LDE's monomials); the
 // strided pass reads its C chunks of 2^S in address order and reverses in LDS, the contiguous one
 // (the whole column) reads each element where it is.
-template <int S, bool N2B, bool INV, bool STRIDED, bool TOP, bool SCALE, bool GATHER = false>
+// TL: log2 of the tile's elements, 4 per thread.
+template <int S, bool N2B, bool INV, bool STRIDED, bool TOP, bool SCALE, bool GATHER = false, int TL = LAT_TL>
 __device__ __forceinline__ void lat_body(const PassArgs &a, const u32 bid) {
   using Sh = Shape2<S, N2B>;
   constexpr int R = Sh::ROUNDS;
-  constexpr int LOG_C = LAT_TL - S;
+  constexpr int LOG_C = TL - S;
   constexpr int C = 1 << LOG_C;
+  static_assert(!STRIDED || TL == LAT_TL, "strided latency passes run 1024-element tiles");
   static_assert(!STRIDED || LOG_C >= 2, "strided latency passes keep runs of >= 4 elements");
-  __shared__ u64 lds[LAT_TILE + LAT_TILE / 16];
+  __shared__ u64 lds[(1 << TL) + (1 << TL) / 16];
   const u32 t = threadIdx.x;
   const u32 L = a.log_n;
   // thread -> (c, q): c picks the run (strided) or chunk (contiguous), q the element pairs;
@@ -228,6 +230,22 @@ __global__ __launch_bounds__(THREADS) void ntt_pass_lat_cosets(CosetArgs c) {
   u32 tiles;
   const u32 tile = enter_coset(c, a, tiles);
   lat_body<S, true, false, STRIDED, STRIDED, true, true>(a, tile);
+}
+// A whole column of 2^11 or 2^12 in one workgroup of 512 or 1024 threads: one launch instead of a
+// strided and a contiguous one (256 columns of 2^11 in 7.7 us instead of 11.0; the launch rule says
+// where each wins).  What bounds it is the chain of a thread, six rounds and their table reads.
+constexpr int wide_threads(int S) { return 1 << (S - 2); }
+template <int S, bool N2B, bool INV, bool SCALE>
+__global__ __launch_bounds__(wide_threads(S)) void ntt_pass_lat_wide(PassArgs a) {
+  to_slice(a);
+  lat_body<S, N2B, INV, false, false, SCALE, false, S>(a, blockIdx.x);
+}
+template <int S>
+__global__ __launch_bounds__(wide_threads(S)) void ntt_pass_lat_wide_cosets(CosetArgs c) {
+  PassArgs a;
+  u32 tiles;
+  const u32 tile = enter_coset(c, a, tiles);
+  lat_body<S, true, false, false, false, true, true, S>(a, tile);
 }
 // a group of batches (batch plans), as the grouped throughput passes
 template <int S, bool N2B, bool INV, bool STRIDED, bool TOP, bool SCALE>

@@ -68,6 +68,23 @@ BaCosetKernel ba_pick_lat_cosets(uint32_t S, bool strided) {
   return nullptr;
 }
 
+template <int S, bool N2B, bool INV>
+static BaPassKernel wide(bool scale) {
+  return scale ? ntt_pass_lat_wide<S, N2B, INV, true> : ntt_pass_lat_wide<S, N2B, INV, false>;
+}
+template <int S>
+static BaPassKernel wide(bool n2b, bool inverse, bool scale) {
+  if (n2b) return inverse ? wide<S, true, true>(scale) : wide<S, true, false>(scale);
+  return inverse ? wide<S, false, true>(scale) : wide<S, false, false>(scale);
+}
+
+BaPassKernel ba_pick_lat_wide(uint32_t S, bool n2b, bool inverse, bool scale) {
+  return S == 11 ? wide<11>(n2b, inverse, scale) : S == 12 ? wide<12>(n2b, inverse, scale) : nullptr;
+}
+BaCosetKernel ba_pick_lat_wide_cosets(uint32_t S) {
+  return S == 11 ? ntt_pass_lat_wide_cosets<11> : S == 12 ? ntt_pass_lat_wide_cosets<12> : nullptr;
+}
+
 namespace {
 // [S][n2b][inverse][strided][top][scale], as rocprofv3 prints them; built by the first caller
 // (a function-local static initialiser, so concurrent first calls are safe)
