@@ -319,3 +319,33 @@ def test_whole_column_workgroups(ba, log_n, cols):
     finally:
         d_in.free()
         d_out.free()
+
+
+# Vectors whose sums hit 0, p and the words around them at every stage, where lazy residues differ from
+# canonical ones: constants, alternating and short-period signs, impulses, and draws from edge values.
+@pytest.mark.parametrize("log_n,cols", [(4, 70000), (9, 2100), (12, 280), (13, 140), (15, 40), (16, 20), (18, 5), (20, 2),
+                                        (22, 1)])
+def test_edge_patterns(ba, log_n, cols):
+    n = 1 << log_n
+    rng = np.random.default_rng(log_n)
+    edges = np.array([0, 1, 2, P - 1, P - 2, 0xFFFFFFFF, 1 << 32, P - (1 << 32), P, 2**64 - 1], dtype=np.uint64)
+    x = rng.choice(edges, (cols, n))
+    j = np.arange(n)
+    signs = np.array([1, P - 1], dtype=np.uint64)
+    for k, row in enumerate([np.ones(n, np.uint64), signs[j & 1], signs[(j >> 1) & 1], signs[(j >> (log_n - 1)) & 1],
+                             signs[(j >> (log_n - 2)) & 1], (j == 0).astype(np.uint64), np.full(n, P - 1, np.uint64)]):
+        if k < cols:
+            x[k] = row
+    x = np.ascontiguousarray(x.reshape(-1))
+    d_in, d_out = ba.DeviceAllocation.from_host(x), ba.DeviceAllocation(cols * n)
+    try:
+        for bitrev in (False, True):
+            for inverse, lext, coset in ((False, 0, 0), (True, 0, 0), (False, 1, 1), (True, 2, 1)):
+                log(f"edge patterns log_n={log_n} cols={cols} bitrev={bitrev} inverse={inverse} lext={lext}")
+                ba.ntt.batch_ntt_internal(d_in.ptr, d_out.ptr, log_n, cols, n, n, bitrev, inverse, lext, coset)
+                ba.synchronize()
+                want = gl_oracle.batch_ntt(x, log_n, cols, n, n, bitrev, inverse, lext, coset, nthreads=8)
+                assert np.array_equal(d_out.to_host(), want)
+    finally:
+        d_in.free()
+        d_out.free()

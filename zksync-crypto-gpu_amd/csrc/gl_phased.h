@@ -41,8 +41,8 @@ struct Mul {
 };
 constexpr int MUL_PHASES = 12;
 
-// phase P of gl::mul(s.a, s.b) -> s.r
-template <int P>
+// phase P of gl::mul(s.a, s.b) -> s.r (LAZY: gl::mul_lazy)
+template <int P, bool LAZY = false>
 __device__ __forceinline__ void mul_phase(Mul &s) {
   using namespace isa;
   if constexpr (P == 0) {
@@ -68,15 +68,16 @@ __device__ __forceinline__ void mul_phase(Mul &s) {
   } else if constexpr (P == 9) {
     s.R = mad_eps(s.r2, pack(s.t0, s.t1), s.c);
   } else if constexpr (P == 10) {
-    s.one = one_if(s.c | ge_p(s.R));
+    s.one = one_if(LAZY ? s.c : s.c | ge_p(s.R));
   } else if constexpr (P == 11) {
     s.r = (u64)s.one * (u32)EPS + s.R;
   }
 }
 
 // For i < N (compile-time): x(i) *= y(i), where x(ic) returns a reference to the operand and
-// y(ic) its multiplier (ic: std::integral_constant<int, i>), interleaved ILP at a time.
-template <int N, typename X, typename Y>
+// y(ic) its multiplier (ic: std::integral_constant<int, i>), interleaved ILP at a time; the first
+// LAZY products are lazy.
+template <int N, int LAZY = 0, typename X, typename Y>
 __device__ __forceinline__ void mul_batch(X &&x, Y &&y) {
   constexpr int GROUPS = (N + ILP - 1) / ILP;
   sfor<GROUPS>([&](auto g_) {
@@ -89,7 +90,10 @@ __device__ __forceinline__ void mul_batch(X &&x, Y &&y) {
       st[j].b = y(std::integral_constant<int, g * ILP + j>{});
     });
     sfor<MUL_PHASES>([&](auto p_) {
-      sfor<M>([&](auto j_) { mul_phase<decltype(p_)::value>(st[decltype(j_)::value]); });
+      sfor<M>([&](auto j_) {
+        constexpr int j = decltype(j_)::value;
+        mul_phase<decltype(p_)::value, (g * ILP + j < LAZY)>(st[j]);
+      });
     });
     sfor<M>([&](auto j_) {
       constexpr int j = decltype(j_)::value;
@@ -168,7 +172,8 @@ __device__ __forceinline__ void shift_phase(Shift &s) {
 }
 
 // ---------------------------------------------------------------- add and subtract
-// (s, d) = (a + b, a - b), canonical, from canonical a, b: 4 phases.
+// (s, d) = (a + b, a - b), canonical, from canonical a, b: 4 phases.  LAZY: a any u64, b canonical,
+// s and d lazy residues (gl::add_lazy, gl::sub).
 struct AddSub {
   u64 a, b, s, d;
   u64 cs, c2, cd, bw, kd;
@@ -176,7 +181,7 @@ struct AddSub {
 };
 constexpr int ADDSUB_PHASES = 4;
 
-template <int P>
+template <int P, bool LAZY = false>
 __device__ __forceinline__ void addsub_phase(AddSub &s) {
   using namespace isa;
   if constexpr (P == 0) {
@@ -186,7 +191,7 @@ __device__ __forceinline__ void addsub_phase(AddSub &s) {
     s.s1 = addc(hi(s.a), hi(s.b), s.cs, s.c2);
     s.d1 = subb(hi(s.a), hi(s.b), s.cd, s.bw);
   } else if constexpr (P == 2) {
-    s.one = one_if(s.c2 | ge_p(pack(s.s0, s.s1)));
+    s.one = one_if(LAZY ? s.c2 : s.c2 | ge_p(pack(s.s0, s.s1)));
     s.d0 = addc0(s.d0, s.bw, s.kd);
   } else if constexpr (P == 3) {
     s.s = (u64)s.one * (u32)EPS + pack(s.s0, s.s1);
@@ -212,21 +217,25 @@ struct Bfly {
   AddSub as;
 };
 
-template <int E, int P>
+// LAZY: a any u64, results lazy; b canonical, or any u64 where a shift or REDUCE (E = 0: gl::reduce1, 2
+// phases) makes it canonical first.
+constexpr int dit_pre_phases(int E, bool reduce) { return shift_phases(E % 96) + (reduce ? 2 : 0); }
+
+template <int E, int P, bool LAZY, bool REDUCE>
 __device__ __forceinline__ void dit_phase(Bfly &s) {
   using Fm = PowForm<E>;
+  static_assert(!REDUCE || Fm::SP == 0, "a shift makes its result canonical");
+  constexpr int SP = dit_pre_phases(E, REDUCE);
   if constexpr (P == 0) s.sh.x = s.b, s.as.a = s.a;
-  if constexpr (P < Fm::SP) shift_phase<Fm::F, P>(s.sh);
-  if constexpr (P == Fm::SP) s.as.b = Fm::SP ? s.sh.t : s.sh.x;
-  if constexpr (P >= Fm::SP && P < Fm::SP + ADDSUB_PHASES) addsub_phase<P - Fm::SP>(s.as);
-  if constexpr (P == Fm::SP + ADDSUB_PHASES - 1) {
+  if constexpr (REDUCE && P == 0) s.sh.one = isa::one_if(isa::ge_p(s.sh.x));
+  if constexpr (REDUCE && P == 1) s.sh.x = (u64)s.sh.one * (u32)EPS + s.sh.x;
+  if constexpr (!REDUCE && P < SP) shift_phase<Fm::F, P>(s.sh);
+  if constexpr (P == SP) s.as.b = Fm::SP ? s.sh.t : s.sh.x;
+  if constexpr (P >= SP && P < SP + ADDSUB_PHASES) addsub_phase<P - SP, LAZY>(s.as);
+  if constexpr (P == SP + ADDSUB_PHASES - 1) {
     s.a = Fm::NEG ? s.as.d : s.as.s;
     s.b = Fm::NEG ? s.as.s : s.as.d;
   }
-}
-template <int E>
-constexpr int dit_phases() {
-  return PowForm<E>::SP + ADDSUB_PHASES;
 }
 
 template <int E, int P>

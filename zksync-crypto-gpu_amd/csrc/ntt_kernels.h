@@ -80,6 +80,19 @@ __device__ __forceinline__ void bfly_dit(u64 &a, u64 &b) {
   }
 }
 
+// The same with a any u64 and results lazy (any u64 residues): t must be canonical, which the shift's
+// result is and REDUCE makes b (E = 0).  CANON: a is canonical too, and the sum comes out canonical.
+template <int E, bool REDUCE, bool CANON>
+__device__ __forceinline__ void bfly_dit_lazy(u64 &a, u64 &b) {
+  const u64 a0 = a;
+  bool negate;
+  const u64 t = REDUCE ? reduce1(b) : mul_pow2_signed<E>(b, negate);
+  if constexpr (REDUCE) negate = false;
+  const u64 s = CANON ? add(a0, t) : add_lazy(a0, t), d = sub(a0, t);
+  a = negate ? d : s;
+  b = negate ? s : d;
+}
+
 // (a, b) <- (a + b, 2^E (a - b))
 template <int E>
 __device__ __forceinline__ void bfly_dif(u64 &a, u64 &b) {
@@ -103,6 +116,34 @@ __device__ __forceinline__ void dit_group(u64 (&v)[VALS]) {
       static_for<half>([&](auto j_) {
         constexpr int j = q * 2 * half + decltype(j_)::value;
         bfly_dit<E>(v[BASE + j * STRIDE], v[BASE + (j + half) * STRIDE]);
+      });
+    });
+  });
+}
+
+// The same with lazy results, from inputs of which i >= 2^(K-2) are canonical and the rest any u64.  A
+// butterfly needs its b canonical: in stage 0 the inputs i >= 2^(K-1) are; from stage 1 on a factor
+// other than 1 makes it so; stage 1's b's without one are stage 0's sums of inputs i >= 2^(K-2), left
+// canonical; later stages reduce theirs (3 of 32 butterflies for K = 4).  Per 16 elements 28 of 32 sums
+// skip the comparison with p, for 9 instructions of reductions: the 12-bit contiguous pass 126 -> 123
+// VALU an element, 64 x 2^20 562 -> 557 us, the blowup-2 LDE of 64 x 2^20 1555 -> 1519 us.
+template <int K>
+struct DitLazy {
+  static constexpr bool canon(int t, int j) { return t == 0 && K >= 2 && j >= (1 << K) / 4; }
+  static constexpr bool reduce(int t, int q) { return t >= 2 && q == 0; }
+};
+template <int K, int STRIDE, int BASE, bool INV>
+__device__ __forceinline__ void dit_group_lazy(u64 (&v)[VALS]) {
+  static_for<K>([&](auto t_) {
+    constexpr int t = decltype(t_)::value;
+    constexpr int half = 1 << (K - 1 - t);
+    static_for<(1 << t)>([&](auto q_) {
+      constexpr int q = decltype(q_)::value;
+      constexpr int E = local_exp(t + 1, cbitrev(q, t), INV);
+      static_for<half>([&](auto j_) {
+        constexpr int j = q * 2 * half + decltype(j_)::value;
+        bfly_dit_lazy<E, DitLazy<K>::reduce(t, q), DitLazy<K>::canon(t, j)>(v[BASE + j * STRIDE],
+                                                                           v[BASE + (j + half) * STRIDE]);
       });
     });
   });
@@ -142,19 +183,26 @@ struct RoundStage {
     const int q = (b & ((1 << (K - 1)) - 1)) / half(t);
     return N2B ? local_exp(t + 1, cbitrev(q, t), INV) : local_exp(K - t, cbitrev(q, K - t - 1), INV);
   }
-  static constexpr int phases(int t, int b) {
+  // LAZY (n2b): the butterflies of DitLazy
+  static constexpr bool reduce(int t, int b) {
+    return DitLazy<K>::reduce(t, (b & ((1 << (K - 1)) - 1)) / half(t));
+  }
+  static constexpr bool canon(int t, int b) { return DitLazy<K>::canon(t, j(t, b)); }
+  static constexpr int phases(int t, int b, bool lazy) {
     const int e = E(t, b), f = e % 96;
-    return ph::ADDSUB_PHASES + ph::shift_phases(f);
+    return ph::ADDSUB_PHASES + (N2B ? ph::dit_pre_phases(e, lazy && reduce(t, b)) : ph::shift_phases(f));
   }
 };
 
 // One radix-2^K round over all 16 registers, one butterfly after another (register
 // m = i * 2^(4-K) + m_lo, i active).
-template <int K, bool N2B, bool INV>
+template <int K, bool N2B, bool INV, bool LAZY>
 __device__ __forceinline__ void local_round_seq(u64 (&v)[VALS]) {
   static_for<(1 << (4 - K))>([&](auto lo_) {
     constexpr int lo = decltype(lo_)::value;
-    if constexpr (N2B)
+    if constexpr (N2B && LAZY)
+      dit_group_lazy<K, (1 << (4 - K)), lo, INV>(v);
+    else if constexpr (N2B)
       dit_group<K, (1 << (4 - K)), lo, INV>(v);
     else
       dif_group<K, (1 << (4 - K)), lo, INV>(v);
@@ -163,7 +211,7 @@ __device__ __forceinline__ void local_round_seq(u64 (&v)[VALS]) {
 
 // The same round stage by stage; each stage's 8 independent butterflies run ph::ILP at a time,
 // phase-interleaved.
-template <int K, bool N2B, bool INV>
+template <int K, bool N2B, bool INV, bool LAZY>
 __device__ __forceinline__ void local_round_ilv(u64 (&v)[VALS]) {
   using St = RoundStage<K, N2B, INV>;
   static_assert(8 % ph::ILP == 0, "interleave width must divide a stage's 8 butterflies");
@@ -179,7 +227,10 @@ __device__ __forceinline__ void local_round_ilv(u64 (&v)[VALS]) {
       });
       constexpr int MAXP = [] {
         int m = 0;
-        for (int k = 0; k < ph::ILP; k++) m = St::phases(t, g * ph::ILP + k) > m ? St::phases(t, g * ph::ILP + k) : m;
+        for (int k = 0; k < ph::ILP; k++) {
+          const int n = St::phases(t, g * ph::ILP + k, LAZY);
+          m = n > m ? n : m;
+        }
         return m;
       }();
       static_for<MAXP>([&](auto p_) {
@@ -187,9 +238,9 @@ __device__ __forceinline__ void local_round_ilv(u64 (&v)[VALS]) {
         static_for<ph::ILP>([&](auto j_) {
           constexpr int b = g * ph::ILP + decltype(j_)::value;
           constexpr int e = St::E(t, b);
-          if constexpr (p < St::phases(t, b)) {
+          if constexpr (p < St::phases(t, b, LAZY)) {
             if constexpr (N2B)
-              ph::dit_phase<e, p>(st[decltype(j_)::value]);
+              ph::dit_phase<e, p, LAZY && !St::canon(t, b), LAZY && St::reduce(t, b)>(st[decltype(j_)::value]);
             else
               ph::dif_phase<e, p>(st[decltype(j_)::value]);
           }
@@ -215,17 +266,19 @@ __device__ __forceinline__ void twiddle_powers(u64 (&pw)[VALS], u64 w) {
   });
 }
 
-// v[m] *= W^(m >> (4-K)) for the registers with a factor other than W^0; ILV: interleaved
-template <int K, bool ILV>
+// v[m] *= W^(m >> (4-K)) for the registers with a factor other than W^0; ILV: interleaved; LAZY: the
+// products that dit_group_lazy takes unreduced (local indices below 2^(K-2)) stay so
+template <int K, bool ILV, bool LAZY>
 __device__ __forceinline__ void apply_twiddles(u64 (&v)[VALS], const u64 (&pw)[VALS]) {
   constexpr int FIRST = 1 << (4 - K);
+  constexpr int LAZY_END = LAZY && K >= 3 ? VALS / 4 : FIRST;  // registers [FIRST, LAZY_END)
   if constexpr (ILV) {
-    ph::mul_batch<VALS - FIRST>([&](auto i) -> u64 & { return v[FIRST + decltype(i)::value]; },
+    ph::mul_batch<VALS - FIRST, LAZY_END - FIRST>([&](auto i) -> u64 & { return v[FIRST + decltype(i)::value]; },
                                 [&](auto i) { return pw[(FIRST + decltype(i)::value) >> (4 - K)]; });
   } else {
     static_for<VALS>([&](auto m_) {
       constexpr int m = decltype(m_)::value;
-      if constexpr (m >= FIRST) v[m] = mul(v[m], pw[m >> (4 - K)]);
+      if constexpr (m >= FIRST) v[m] = m < LAZY_END ? mul_lazy(v[m], pw[m >> (4 - K)]) : mul(v[m], pw[m >> (4 - K)]);
     });
   }
 }
@@ -244,12 +297,12 @@ __device__ __forceinline__ void mul_all(u64 (&v)[VALS], F &&f) {
   }
 }
 
-template <int K, bool N2B, bool INV, bool ILV>
+template <int K, bool N2B, bool INV, bool ILV, bool LAZY = false>
 __device__ __forceinline__ void local_round(u64 (&v)[VALS]) {
   if constexpr (ILV)
-    local_round_ilv<K, N2B, INV>(v);
+    local_round_ilv<K, N2B, INV, LAZY>(v);
   else
-    local_round_seq<K, N2B, INV>(v);
+    local_round_seq<K, N2B, INV, LAZY>(v);
 }
 
 enum : u32 { SCALE_NONE = 0, SCALE_PRE = 1, SCALE_POST = 2 };
@@ -269,8 +322,9 @@ struct PassArgs {
   u32 scale_coset;       // the factor depends on j (log_extension_degree > 0)
   u32 coset_mul;         // s^j = 7^j omega_{2^30}^(j * coset_mul)
   u32 in_bitrev;         // first n2b pass: natural element j is read from position bitrev_L(j)
-  u32 in_canonical;      // the input was written by a pass of this library (values < p): loads
-                         // skip the reduction that a caller's raw u64 input needs
+  u32 in_canonical;      // the input was written by a pass of this library: loads skip the reduction
+                         // that a caller's raw u64 input needs (an n2b strided pass leaves lazy
+                         // residues, which the next pass's first round takes; all others values < p)
   // column k starts at in_cols[k] / out_cols[k] when these lists are given (columns gathered
   // from separate buffers), else at in + k * stride_in / out + k * stride_out
   const u64 *const *in_cols;
@@ -385,11 +439,15 @@ __device__ __forceinline__ u64 round_twiddle(const PassArgs &a, u32 gidx, u32 P,
 
 // ILV: the round's products and butterflies phase-interleaved (the strided pass, where that
 // measured faster) or one after another (the contiguous pass, where it measured slower)
-template <int K, bool N2B, bool INV, bool ILV>
+// LAZY (n2b): the round's results are lazy residues, which every later round's products take; the
+// registers without a product (local index 0) may be lazy on entry.  Without twiddles (the top
+// round) all inputs are canonical.
+template <int K, bool N2B, bool INV, bool ILV, bool LAZY>
 __device__ __forceinline__ void do_round(u64 (&v)[VALS], const u64 (&pw)[VALS], bool twiddle) {
-  if (N2B && twiddle) apply_twiddles<K, ILV>(v, pw);
-  local_round<K, N2B, INV, ILV>(v);
-  if (!N2B && twiddle) apply_twiddles<K, ILV>(v, pw);
+  static_assert(N2B || !LAZY, "only n2b rounds leave lazy residues");
+  if (N2B && twiddle) apply_twiddles<K, ILV, LAZY>(v, pw);
+  local_round<K, N2B, INV, ILV, LAZY>(v);
+  if (!N2B && twiddle) apply_twiddles<K, ILV, false>(v, pw);
 }
 
 // Loads/stores address a column as a uniform base plus a 32-bit per-thread byte offset
@@ -567,7 +625,8 @@ __device__ __forceinline__ void strided_body(const PassArgs &a, const u32 bid) {
         });
         __syncthreads();
       }
-      do_round<Sh::K(r), N2B, INV, true>(v, tw[r], !(TOP && r == Sh::TOP));
+      // an n2b strided pass is never a transform's last
+      do_round<Sh::K(r), N2B, INV, true, N2B>(v, tw[r], !(TOP && r == Sh::TOP));
     });
     if constexpr (!N2B && SCALE) mul_all<true>(v, [&](int m) { return fac[m]; });
     u32 o = offL;
@@ -820,6 +879,9 @@ __device__ __forceinline__ void contig_body(const PassArgs &a, const u32 bid) {
         wave_sync();
       }
       if (SC != 0 && !INV && r == 0) scale_all(v);
+      // n2b rounds but the last leave lazy residues; the last reduces the register it does not multiply
+      constexpr bool LAZY = N2B && r < R - 1;
+      if constexpr (N2B && r == R - 1 && R > 1 && !(FOLD && WB < 4)) v[0] = reduce1(v[0]);
       if constexpr (WB >= 4) {
         constexpr int K = Sh::K(r), QB = S - 4 - WB;
         const u32 base = ((c << QB) | (q >> WB)) << K;
@@ -828,13 +890,13 @@ __device__ __forceinline__ void contig_body(const PassArgs &a, const u32 bid) {
           constexpr int i = decltype(i_)::value;
           pw[i] = ltw[r][base + i];
         });
-        do_round<K, N2B, INV, false>(v, pw, !(top && r == Sh::TOP));
+        do_round<K, N2B, INV, false, LAZY>(v, pw, !(top && r == Sh::TOP));
       } else if constexpr (FOLD && r == R - 1) {
         constexpr int K = Sh::K(r);
         mul_all<false>(v, [&](int m) { return tw[r][m >> (4 - K)]; });
         local_round<K, N2B, INV, false>(v);
       } else {
-        do_round<Sh::K(r), N2B, INV, false>(v, tw[r], !(top && r == Sh::TOP));
+        do_round<Sh::K(r), N2B, INV, false, LAZY>(v, tw[r], !(top && r == Sh::TOP));
       }
       if (SC != 0 && INV && r == R - 1 && !FOLD) scale_all(v);
     });
