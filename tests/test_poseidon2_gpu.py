@@ -220,3 +220,35 @@ def test_leaves_either_side_of_the_quad_rule(ba, rc, log_rows, cols, count):
     finally:
         d_v.free()
         d_r.free()
+
+
+# Up to 8192 digests run on rows of 16 threads, 16 rows a block.
+@pytest.mark.parametrize("count", [1, 15, 16, 17, 8191, 8192, 8193])
+def test_digests_either_side_of_the_row_rule(ba, rc, count):
+    rng = np.random.default_rng(count)
+    edges = np.array([0, 1, 0x1FFFFF, 0x200000, 0xFFFFFFFF, 0x100000000, 0x3FFFFFFFFFF, 1 << 42, gl_oracle.P - 1,
+                      gl_oracle.P, 2**64 - 1], dtype=np.uint64)
+    rows, cols = 2, 7  # 14 values a leaf: a full chunk, then one filled up with zeros
+    nodes, leaves = raw_u64(rng, 8 * count), raw_u64(rng, rows * cols * count)
+    for v in (nodes, leaves):
+        v[:: 3] = rng.choice(edges, v[:: 3].size)
+        v[: v.size // 8] = np.uint64(2**64 - 1)
+    d_n, d_l, d_r = ba.DeviceAllocation.from_host(nodes), ba.DeviceAllocation.from_host(leaves), ba.DeviceAllocation(
+        4 * count)
+    try:
+        log(f"poseidon2 row rule count={count}")
+        ba.poseidon2.compute_node_hashes(d_n, d_r)
+        ba.synchronize()
+        assert np.array_equal(d_r.to_host(), gl_oracle.poseidon2_nodes(nodes, count, rc))
+        want = gl_oracle.poseidon2_leaves(leaves, rows, cols, count, rc)
+        ba.poseidon2.compute_leaf_hashes(d_l, d_r, 1)
+        ba.synchronize()
+        assert np.array_equal(d_r.to_host(), want)
+        first = 4 * rows * count  # the first chunk's columns, then the capacity carried over
+        ba.poseidon2.compute_leaf_hashes(d_l.sub(0, first), d_r, 1, store_intermediate=True)
+        ba.poseidon2.compute_leaf_hashes(d_l.sub(first, 3 * rows * count), d_r, 1, load_intermediate=True)
+        ba.synchronize()
+        assert np.array_equal(d_r.to_host(), want)
+    finally:
+        for d in (d_n, d_l, d_r):
+            d.free()

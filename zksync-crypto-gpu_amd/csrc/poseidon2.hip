@@ -15,9 +15,9 @@
 // What bounds it: VALU issue, ~9.9 k instructions per permutation against 64 bytes of input, the
 // digests being independent.  The state stays lazy (any u64 residue) between layers, see below:
 // 2^20 leaves of 64 values take 2.23 ms (3.8 G permutations/s), where canonical lanes at 16.2 k
-// instructions took 3.0 ms.  Two kernels share the arithmetic: one thread per digest with all 12
-// lanes in registers (throughput), and one quad of threads per digest (latency, few digests),
-// chosen by the digest count (QUAD_MAX below).
+// instructions took 3.0 ms.  Three kernels share the arithmetic: one thread per digest with all 12
+// lanes in registers (throughput), a quad of threads per digest (latency, few digests), and 16 threads
+// per digest (latency, fewest), chosen by the digest count (QUAD_MAX, ROW_MAX below).
 #include <utility>
 #include <vector>
 
@@ -38,6 +38,10 @@ constexpr int QUADS = THREADS / 4;
 // 18 us and does 1.7 times the work.  Node hashes, thread / quad, us: 2^10 39 / 18, 2^15 39 / 24,
 // 2^16 40 / 40, 2^16.6 47 / 61, 2^18 87 / 128.
 constexpr u32 QUAD_MAX = 65536;
+// Below that, up to which count 16 threads take a digest: a row's chain is 11.5 us, which two waves per
+// SIMD (2^13 digests) still nearly hide.  Node hashes, quad / row, us: 2^4 18.1 / 11.4, 2^10 18.6 /
+// 11.6, 2^12 18.9 / 12.2, 2^13 19.3 / 16.0, 2^14 20.0 / 25.8, 2^16 40 / 84.
+constexpr u32 ROW_MAX = 8192;
 
 // Lazy arithmetic: state lanes are any u64 (a residue mod p, not reduced below it).  gl::mul_lazy
 // takes and returns such values; the linear layers take a value's two words into two 64-bit
@@ -313,6 +317,99 @@ __device__ __forceinline__ void quad_permute(u64 (&s)[3], const Quad &q, const u
   }
 }
 
+// ---------------------------------------------------------------- 16 threads per digest
+// Thread i < 12 of a row of 16 holds lane i; the last four only keep the row sums whole.  Sums over
+// tiles and over all lanes are DPP row rotations.  A permutation is a chain of ~2.6 k instructions, for
+// 2.4 times the quad's work in all.
+struct Row {
+  u32 lane;
+  u32 m4[4];  // M4[j][(j + k) mod 4], j the position in the tile; 0 in idle threads
+  u32 mu;     // 2^mu of the lane; 0 in idle threads
+  u32 mask;   // the lane's low 21 bits, nothing in idle threads
+  u32 width;  // 22, 0 in idle threads
+};
+
+template <int N>
+__device__ __forceinline__ u32 row_ror(u32 x) {
+  return (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x120 + N, 0xF, 0xF, true);
+}
+
+__device__ __forceinline__ Row row_of(u32 lane) {
+  const bool live = lane < WIDTH;
+  const u32 rows = !live ? 0 : lane & 1 ? 0x4116u : 0x3175u;
+  constexpr u64 MUS = 0xC36D'9250'8BE4ull;  // mu, 4 bits per lane
+  Row q;
+  q.lane = lane;
+#pragma unroll
+  for (int k = 0; k < 4; k++) q.m4[k] = (rows >> (4 * k)) & 15u;
+  q.mu = live ? 1u << ((u32)(MUS >> (4 * lane)) & 15u) : 0;
+  q.mask = live ? 0x1FFFFFu : 0;
+  q.width = live ? 22 : 0;
+  return q;
+}
+
+__device__ __forceinline__ u64 row_external(u64 s, const Row &q, u64 rc) {
+  using namespace gl::isa;
+  const u32 l = lo(s), h = hi(s);
+  Planes m{mul32(l, q.m4[0]), mul32(h, q.m4[0])};
+  m = {mac(quad_perm<NEXT1>(l), q.m4[1], m.l), mac(quad_perm<NEXT1>(h), q.m4[1], m.h)};
+  m = {mac(quad_perm<NEXT2>(l), q.m4[2], m.l), mac(quad_perm<NEXT2>(h), q.m4[2], m.h)};
+  m = {mac(quad_perm<NEXT3>(l), q.m4[3], m.l), mac(quad_perm<NEXT3>(h), q.m4[3], m.h)};
+  auto across = [](u64 x, auto ror) { return shl_add<0>(x, pack(ror(lo(x)), ror(hi(x)))); };
+  auto eight = [](u32 w) { return row_ror<8>(w); };
+  auto four = [](u32 w) { return row_ror<4>(w); };
+  const Planes sum{across(across(m.l, eight), four), across(across(m.h, eight), four)};
+  const Planes v = m + sum;
+  return folded({mac_const<1>(lo(rc), v.l), mac_const<1>(hi(rc), v.h)});
+}
+
+// The sum over the row runs on three 21/22-bit limbs, whose 16 values stay inside a word: a step is
+// three 32-bit additions instead of two 64-bit ones with two moves each.  rc: 0 outside lane 0, but
+// after the last partial round
+__device__ __forceinline__ u64 row_internal(u64 s, const Row &q, u64 rc) {
+  using namespace gl::isa;
+  u32 a = lo(s) & q.mask;
+  u32 b = __builtin_amdgcn_alignbit(hi(s), lo(s), 21) & q.mask;
+  u32 c = __builtin_amdgcn_ubfe(hi(s), 10, q.width);
+  a += row_ror<8>(a), b += row_ror<8>(b), c += row_ror<8>(c);
+  a += row_ror<4>(a), b += row_ror<4>(b), c += row_ror<4>(c);
+  a += row_ror<2>(a), b += row_ror<2>(b), c += row_ror<2>(c);
+  a += row_ror<1>(a), b += row_ror<1>(b), c += row_ror<1>(c);
+  // a + 2^21 b + 2^42 c: planes below 2^47 and 2^36
+  const Planes sum{mac_const<1 << 21>(b, mac_const<1>(a, lo(rc))), mac_const<1 << 10>(c, hi(rc))};
+  return folded({mac(lo(s), q.mu, sum.l), mac(hi(s), q.mu, sum.h)});
+}
+
+__device__ __forceinline__ u64 row_permute(u64 s, const Row &q, const u64 *__restrict__ rc) {
+  // each round's constants are loaded one round ahead
+  const u64 *row = rc + (q.lane < WIDTH ? q.lane : WIDTH - 1);
+  u64 k = row[0], kr = k;
+  auto step = [&]() {
+    kr = k;
+    row += WIDTH;
+    k = row[0];
+  };
+  step();
+  s = row_external(s, q, kr);
+#pragma unroll 1
+  for (int half = 0; half < 2; half++) {
+#pragma unroll 1
+    for (int r = 0; r < HALF_FULL_ROUNDS; r++) {
+      kr = k;
+      if (!(half && r + 1 == HALF_FULL_ROUNDS)) step();
+      s = row_external(sbox(s), q, kr);
+    }
+    if (half) break;
+#pragma unroll 1
+    for (int r = 0; r < PARTIAL_ROUNDS; r++) {
+      step();
+      const u64 x = sbox(s);
+      s = row_internal(q.lane == 0 ? x : s, q, kr);
+    }
+  }
+  return s;
+}
+
 // Leaf gid absorbs values[gid * rows + r + c * rows * count] (c < cols, r < rows, column by
 // column) RATE at a time into lanes 0..7 (overwrite mode, zero-filled past the last value) and
 // permutes after each chunk; digest word k goes to results[gid + k * count].
@@ -404,6 +501,42 @@ __global__ __launch_bounds__(THREADS) void nodes_quad_kernel(const u64 *__restri
   results[at] = gl::reduce1(s[0]);
 }
 
+// The same two hashes by rows: thread i < 8 absorbs value i of each chunk, thread i < 4 holds word i of
+// a digest.
+constexpr int DIGEST_ROWS = THREADS / 16;
+__global__ __launch_bounds__(THREADS) void leaves_row_kernel(const u64 *__restrict__ values,
+                                                             u64 *__restrict__ results, u32 rows, u32 cols,
+                                                             u32 count, int load_intermediate,
+                                                             int store_intermediate, const u64 *__restrict__ rc) {
+  const u32 gid = blockIdx.x * DIGEST_ROWS + (threadIdx.x >> 4);
+  if (gid >= count) return;
+  const Row q = row_of(threadIdx.x & 15);
+  u64 s = load_intermediate && q.lane >= RATE && q.lane < WIDTH ? results[gid + (u64)(q.lane - RATE) * count] : 0;
+  const u64 *leaf = values + (u64)gid * rows;
+  const u64 col_stride = (u64)rows * count;
+  const u64 total = (u64)rows * cols;
+  const u32 log_rows = 31 - __builtin_clz(rows);
+  for (u64 off = 0; off < total; off += RATE) {
+    const u64 v = off + q.lane;
+    if (q.lane < RATE) s = v < total ? leaf[(v & (rows - 1)) + (v >> log_rows) * col_stride] : 0;
+    s = row_permute(s, q, rc);
+  }
+  const u32 word = q.lane - (store_intermediate ? RATE : 0);
+  if (word < CAPACITY) results[gid + (u64)word * count] = gl::reduce1(s);
+}
+
+__global__ __launch_bounds__(THREADS) void nodes_row_kernel(const u64 *__restrict__ values,
+                                                            u64 *__restrict__ results, u32 count,
+                                                            const u64 *__restrict__ rc) {
+  const u32 gid = blockIdx.x * DIGEST_ROWS + (threadIdx.x >> 4);
+  if (gid >= count) return;
+  const Row q = row_of(threadIdx.x & 15);
+  // word k of the left child in lane k, of the right child in lane 4 + k
+  u64 s = q.lane < RATE ? values[2 * (gid + (u64)(q.lane & 3) * count) + (q.lane >> 2)] : 0;
+  s = row_permute(s, q, rc);
+  if (q.lane < CAPACITY) results[gid + (u64)q.lane * count] = gl::reduce1(s);
+}
+
 // The current device's context with installed round constants, or an error code.
 int hasher_context(ba_context *&ctx) {
   ctx = ba_context_for_current_device();
@@ -415,7 +548,10 @@ u32 blocks_for(u64 count, u32 per_block) { return (u32)((count + per_block - 1) 
 
 int launch_nodes(const ba_context *ctx, const u64 *values, u64 *results, u32 count, hipStream_t stream) {
   if (count == 0) return BA_SUCCESS;
-  if (count <= QUAD_MAX)
+  if (count <= ROW_MAX)
+    nodes_row_kernel<<<blocks_for(count, DIGEST_ROWS), THREADS, 0, stream>>>(values, results, count,
+                                                                            ctx->p2_round_constants);
+  else if (count <= QUAD_MAX)
     nodes_quad_kernel<<<blocks_for(count, QUADS), THREADS, 0, stream>>>(values, results, count,
                                                                         ctx->p2_round_constants);
   else
@@ -500,9 +636,10 @@ extern "C" int ba_poseidon2_gl_compute_leaf_hashes(const uint64_t *values, size_
     if (store_intermediate && (rows * cols) % RATE != 0) return BA_ERROR_INVALID_VALUE;
     if (cols > 0xFFFFFFFFull || count > 0xFFFFFFFFull || (values_len && !values) || !results)
       return BA_ERROR_INVALID_VALUE;
-    const bool quad = count <= QUAD_MAX;
-    const auto kernel = quad ? leaves_quad_kernel : leaves_kernel;
-    kernel<<<blocks_for(count, quad ? QUADS : THREADS), THREADS, 0, (hipStream_t)stream>>>(
+    const bool row = count <= ROW_MAX, quad = count <= QUAD_MAX;
+    const auto kernel = row ? leaves_row_kernel : quad ? leaves_quad_kernel : leaves_kernel;
+    const u32 per_block = row ? DIGEST_ROWS : quad ? QUADS : THREADS;
+    kernel<<<blocks_for(count, per_block), THREADS, 0, (hipStream_t)stream>>>(
         values, results, (u32)rows, (u32)cols, (u32)count, load_intermediate, store_intermediate,
         ctx->p2_round_constants);
     return (int)hipGetLastError();
