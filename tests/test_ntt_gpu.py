@@ -349,3 +349,26 @@ def test_edge_patterns(ba, log_n, cols):
     finally:
         d_in.free()
         d_out.free()
+
+
+# 2^21 runs as 12 + 9 bits; scaled 9-bit passes take 2 columns a workgroup up to 16 columns, 4 above.
+@pytest.mark.parametrize("cols", [1, 16, 17])
+def test_default_plan_of_2p21(ba, cols):
+    n = 1 << 21
+    x = raw_u64(np.random.default_rng(cols), cols * n)
+    d_in, d_out = ba.DeviceAllocation.from_host(x), ba.DeviceAllocation(cols * n)
+    try:
+        for bitrev, inverse, lext, coset in ((False, False, 0, 0), (False, False, 1, 1), (True, True, 0, 0),
+                                             (True, True, 2, 3), (False, True, 1, 0)):
+            log(f"2^21 cols={cols} bitrev={bitrev} inverse={inverse} lext={lext}")
+            ba.ntt.batch_ntt_internal(d_in.ptr, d_out.ptr, 21, cols, n, n, bitrev, inverse, lext, coset)
+            ba.synchronize()
+            want = gl_oracle.batch_ntt(x, 21, cols, n, n, bitrev, inverse, lext, coset, nthreads=8)
+            assert np.array_equal(d_out.to_host(), want)
+            d_out.copy_from_host(x)
+            ba.ntt.batch_ntt_internal(d_out.ptr, d_out.ptr, 21, cols, n, n, bitrev, inverse, lext, coset)
+            ba.synchronize()
+            assert np.array_equal(d_out.to_host(), want)
+    finally:
+        d_in.free()
+        d_out.free()

@@ -69,13 +69,11 @@ inline ba_context *ba_context_for_current_device() {
 }
 
 // Pass decomposition for a 2^log_n transform (n2b order: strided passes from the top bits
-// down, then the contiguous pass; b2n runs the same passes in reverse).
-NttPlan ba_plan_ntt(uint32_t log_n, bool n2b);
+// down, then the contiguous pass; b2n runs the same passes in reverse).  gather: an LDE's coset NTT.
+NttPlan ba_plan_ntt(uint32_t log_n, bool n2b, bool gather);
 // The plan whose passes cover bits[0] (contiguous pass, lowest bits), bits[1], ... upwards;
 // false when no kernel shape covers that split.
 bool ba_plan_from_bits(uint32_t log_n, bool n2b, const uint32_t *bits, int num_passes, NttPlan &plan);
-// The plan a transform of this size class runs with on `ctx` (tuned or built-in).
-NttPlan ba_plan_for(const ba_context *ctx, uint32_t log_n, bool n2b);
 
 // One pass launch of a batch NTT: the kernel pair of its shape, its arguments and grid.
 #include <utility>

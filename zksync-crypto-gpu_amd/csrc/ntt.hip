@@ -47,9 +47,14 @@ bool ba_plan_from_bits(uint32_t log_n, bool n2b, const uint32_t *bits, int num_p
   return true;
 }
 
-NttPlan ba_plan_ntt(uint32_t log_n, bool n2b) {
+NttPlan ba_plan_ntt(uint32_t log_n, bool n2b, bool gather) {
   // passes listed from the low bits up: a contiguous pass of 12 bits, then strided passes of
-  // 8 bits, the last of 4..8 (bits borrowed from the pass below when fewer than 4 remain)
+  // 8 bits, the last of 4..8 (bits borrowed from the pass below when fewer than 4 remain).
+  // 2^21 takes one strided pass of 9 bits, in 64-byte runs, for two of 5 and 4 that each move every
+  // element: 32 columns 704 -> 583 us (n2b), 703 -> 632 (b2n inverse), 716 -> 630 (coset), 13 columns
+  // 269 -> 257, 275 -> 277, 287 -> 276, one column 46 -> 41.  A 10-bit one at 2^22, in 32-byte runs,
+  // is no faster than 6 and 4 bits (16 columns 717 against 720, with a coset 800 against 720).  The
+  // gathered pass of an LDE's coset NTT has no 9-bit build.
   uint32_t bits[8];
   int np = 0;
   if (log_n <= (uint32_t)gl::ntt::TILE_LOG) {
@@ -64,7 +69,7 @@ NttPlan ba_plan_ntt(uint32_t log_n, bool n2b) {
     bits[np++] = sc;
     while (rest > 0) {
       uint32_t take = rest;
-      if (rest > 8) take = (rest - 8 >= 4) ? 8 : rest - 4;
+      if (rest > 8 && (log_n != 21 || gather)) take = (rest - 8 >= 4) ? 8 : rest - 4;
       bits[np++] = take;
       rest -= take;
     }
@@ -72,11 +77,6 @@ NttPlan ba_plan_ntt(uint32_t log_n, bool n2b) {
   NttPlan plan{};
   (void)ba_plan_from_bits(log_n, n2b, bits, np, plan);
   return plan;
-}
-
-NttPlan ba_plan_for(const ba_context *ctx, uint32_t log_n, bool n2b) {
-  const BaTuned &t = ctx->tuned[n2b][log_n];
-  return t.valid ? t.plan : ba_plan_ntt(log_n, n2b);
 }
 
 namespace {
@@ -151,6 +151,9 @@ constexpr uint64_t kMaxGrid = 0x7FFFFFFFull;
 //                         below the top, 6 bits: 198 (1), 181 (3), 191 (8).
 //   strided, one factor for every element (n^-1): 4 bits 185 (1), 204 (8); 5 bits 177 (1), 158 (3), 176 (8);
 //                         8 bits 257 (1), 242 (2..8).
+//   strided, 9 bits, any factor: 8192 tiles 336 (1), 330 (2), 345 (3), 333 (4), 355 (8); 6656: 274, 277,
+//                         286, 289, 309; 12288: 491 (1), 477 (2), 473 (4), 485 (8); with a coset 532,
+//                         500, 482, 486.
 //   strided, a factor per element (coset, gathered coset pass): 16 factors of set-up.  4 bits 263 (1),
 //                         252 (4), 272 (8); 5 bits 215 (1), 177 (5), 195 (8); 6 bits 290 (1), 222 (7);
 //                         8 bits 341 (1), 256 (7).  At least 768 workgroups: 2^24 elements by 8 bits
@@ -160,6 +163,8 @@ static uint32_t pick_reps(bool contig, uint32_t S, bool top, int scale, uint64_t
   uint32_t reps;
   if (contig) {
     reps = tiles < 1536 ? 1 : tiles < 7168 ? 2 : tiles < 14336 ? 3 : only_pass || cols % 8 ? 8 : 5;
+  } else if (scale && S >= 9) {
+    reps = tiles <= 8192 ? 2 : 4;
   } else if (scale == 2) {
     reps = std::min<uint32_t>(S == 4 ? 4 : S == 5 ? 5 : 7, (uint32_t)std::min<uint64_t>(8, tiles / 768));
   } else if (scale == 1) {
@@ -338,7 +343,7 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
   // carry over (the gathered, scaled first pass has other costs; it has no 9- or 10-bit variant).
   const int kind = in_bitrev_gather ? BA_TUNING_LDE_COSETS : (n2b ? 1 : 0);
   const BaTuned &tuning = ctx->tuned[kind][log_n].valid ? ctx->tuned[kind][log_n] : BaTuned{};
-  const NttPlan plan = tuning.valid ? tuning.plan : ba_plan_ntt(log_n, n2b);
+  const NttPlan plan = tuning.valid ? tuning.plan : ba_plan_ntt(log_n, n2b, in_bitrev_gather);
   for (int p = 0; p < plan.num_passes; p++) {
     const uint32_t S = plan.bits[p];
     const bool contig = plan.contig[p];

@@ -221,7 +221,7 @@ extern "C" int ba_tuning_get(ba_context_t ctx, uint32_t log_n, int bitrev_inputs
     const int kind = bitrev_inputs == BA_TUNING_LDE_COSETS ? BA_TUNING_LDE_COSETS : (bitrev_inputs ? 0 : 1);
     const bool n2b = kind != 0;
     const BaTuned &t = ctx->tuned[kind][log_n];
-    const NttPlan p = t.valid ? t.plan : ba_plan_ntt(log_n, n2b);
+    const NttPlan p = t.valid ? t.plan : ba_plan_ntt(log_n, n2b, kind == BA_TUNING_LDE_COSETS);
     *plan = ba_tuned_plan{};
     plan->num_passes = (uint32_t)p.num_passes;
     for (int i = 0; i < p.num_passes; i++) {
