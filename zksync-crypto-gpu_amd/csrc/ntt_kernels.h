@@ -125,8 +125,8 @@ __device__ __forceinline__ void dit_group(u64 (&v)[VALS]) {
 // butterfly needs its b canonical: in stage 0 the inputs i >= 2^(K-1) are; from stage 1 on a factor
 // other than 1 makes it so; stage 1's b's without one are stage 0's sums of inputs i >= 2^(K-2), left
 // canonical; later stages reduce theirs (3 of 32 butterflies for K = 4).  Per 16 elements 28 of 32 sums
-// skip the comparison with p, for 9 instructions of reductions: the 12-bit contiguous pass 126 -> 123
-// VALU an element, 64 x 2^20 562 -> 557 us, the blowup-2 LDE of 64 x 2^20 1555 -> 1519 us.
+// skip the comparison with p, for 9 instructions of reductions: the 12-bit contiguous pass's column loop
+// 126 -> 123 VALU an element, 64 x 2^20 562 -> 557 us, the blowup-2 LDE of 64 x 2^20 1555 -> 1519 us.
 template <int K>
 struct DitLazy {
   static constexpr bool canon(int t, int j) { return t == 0 && K >= 2 && j >= (1 << K) / 4; }
@@ -346,7 +346,8 @@ __device__ __forceinline__ void to_slice(PassArgs &a) {
 // the same XCD (workgroups are dealt round-robin over the 8 XCDs), so the monomials of a tile are
 // read from HBM once and from L2 for the other cosets (64 x 2^20 at blowup 2: 1561 us by this order,
 // 1575 with plainly alternating workgroups, 1593 one coset after the other, 1606 as two launches on
-// two streams; 16 x 2^22 at blowup 4: 3300, 3346, 3568 and 3430).
+// two streams; 16 x 2^22 at blowup 4: 3300, 3346, 3568 and 3430; before the lazy rounds, which took
+// the first to 1519).
 constexpr int MAX_COSETS = 8;
 struct CosetArgs {
   PassArgs a;
@@ -664,8 +665,8 @@ __device__ __forceinline__ void wave_sync() {
 // global memory and registers) or the wave's own block of 1024 elements, 64 consecutive ones per
 // instruction, staged through LDS within the wave: n2b loads the former and stores the latter, b2n
 // the other way round.  With workgroup barriers and tile-wide staging around every exchange the
-// 12-bit pass over 2^26 elements took 352 us b2n and 329 n2b; it takes 338 and 325, and moves 5
-// LDS words per element either way (7 before for b2n).
+// 12-bit pass over 2^26 elements took 352 us b2n and 329 n2b; without, 338 and 325 (n2b 308 with the
+// lazy rounds and 5 columns a workgroup), and moves 5 LDS words per element either way (7 for b2n).
 template <int S, bool N2B, bool INV, int SC, bool WHOLE, bool PREFETCH>
 __device__ __forceinline__ void contig_body(const PassArgs &a, const u32 bid) {
   constexpr bool SCALE = SC == 2;
@@ -1031,14 +1032,16 @@ __global__ __launch_bounds__(THREADS) void ntt_pass_strided_group(const PassArgs
   strided_body<S, N2B, INV, TOP, SCALE, GATHER, !strided_four_waves<S, TOP, GATHER>()>(jobs[j],
                                                                                        blockIdx.x - wg_start[j]);
 }
-// the prefetching three-waves build of a four-waves variant, for launches that share the GPU
+// The prefetching three-waves build of a four-waves variant, for launches that share the GPU.  The cap on
+// waves holds where a variant needs no more than 128 registers (the 6-bit n2b pass below the top: 126),
+// which would otherwise fill the CUs' LDS: serve's small requests' p99 60-72 ms against 91-100 without.
 template <int S, bool N2B, bool INV, bool TOP, bool SCALE, bool GATHER>
-__global__ __launch_bounds__(THREADS) void ntt_pass_strided_shared(PassArgs a) {
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 3))) void ntt_pass_strided_shared(PassArgs a) {
   strided_body<S, N2B, INV, TOP, SCALE, GATHER, true>(a, strided_tile<S>(blockIdx.x, gridDim.x));
 }
 template <int S, bool N2B, bool INV, bool TOP, bool SCALE, bool GATHER>
-__global__ __launch_bounds__(THREADS) void ntt_pass_strided_shared_group(const PassArgs *jobs,
-                                                                         const u32 *wg_start, u32 njobs) {
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 3))) void ntt_pass_strided_shared_group(
+    const PassArgs *jobs, const u32 *wg_start, u32 njobs) {
   const u32 j = group_of(wg_start, njobs, blockIdx.x);
   strided_body<S, N2B, INV, TOP, SCALE, GATHER, true>(jobs[j], blockIdx.x - wg_start[j]);
 }
