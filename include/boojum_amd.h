@@ -266,15 +266,15 @@ int ba_batch_plan_destroy(ba_batch_plan_t plan);
  * per pass in the same order, the columns each workgroup repeats over (reps, 1..8; 0 = built-in
  * choice), and the waves per SIMD of a 9..12-bit contiguous pass (contig_waves: 3 = the variant
  * that loads the next tile while transforming, 4 = the 128-register variant without that
- * prefetch, 0 = built-in choice: 4), and the tile shape of plain
- * batch NTTs (tile_log: 10 = the latency-shaped passes, 1024-element tiles of 4 elements per
- * thread in radix-4 rounds, for every batch size, log_n 4..18 only; 12 = the 4096-element tiles
- * of the split above for every batch size; 0 = built-in choice: 1024-element tiles for batches of
- * at most 2^20 elements (2^21 for columns of 2^11), else 4096).  A call's columns of 2^11, and 96 or
- * more of 2^12, take one whole column per workgroup in place of the 1024-element tiles.  An LDE call's coset NTTs take the 1024-element tiles by that
- * batch-size rule alone, counting every coset of a launch.  Valid splits: log_n <= 12
- * one pass of log_n bits; log_n > 12 a contiguous pass of 9..12 bits and strided passes of 4..10
- * bits (at most 8 passes).
+ * prefetch, 0 = built-in choice: 4), and the tile shape of plain batch NTTs (tile_log: 10 = the
+ * latency-shaped passes, 1024-element tiles of 4 elements per thread in radix-4 rounds, for every
+ * batch size, log_n 4..18 only; 12 = the 4096-element tiles of the split above for every batch
+ * size; 0 = built-in choice: 1024-element tiles for batches of at most 2^20 elements (2^21 for
+ * columns of 2^11), else 4096).  A call's columns of 2^11, and 96 or more of 2^12, take one whole
+ * column per workgroup in place of the 1024-element tiles.  An LDE call's coset NTTs take the
+ * 1024-element tiles by that batch-size rule alone, counting every coset of a launch.  Valid splits:
+ * log_n <= 12 one pass of log_n bits; log_n > 12 a contiguous pass of 9..12 bits and strided passes
+ * of 4..10 bits (at most 8 passes).
  *
  * ba_autotune times every valid split, then each pass's reps, then contig_waves, then (log_n 4..18)
  * the 1024-element tiles against the best of those, for plain NTTs of both input orders and for

@@ -40,10 +40,9 @@ __device__ __forceinline__ void gstore(T *p, T v) {
 // inserts the wait states a VALU-written SGPR needs before a VALU or SALU instruction reads it.
 // What they cost (measured on MI355X, waves of 64 at 8 per SIMD): every instruction here issues
 // at the full-width VALU rate (4.2-4.9 cycles per wave instruction per SIMD: carry-writing adds,
-// v_mad_u64_u32, 64-bit compares and shifts alike), while the SALU mask logic runs beside the
-// VALU; so the arithmetic below is written for the fewest VALU instructions, with the carry
-// cases resolved by mask logic on the carries (plain C on the 64-bit lane masks, which the
-// compiler emits as SALU instructions) and carry-in adds rather than by selects.
+// v_mad_u64_u32, 64-bit compares and shifts alike); so the arithmetic below is written for the
+// fewest VALU instructions, and among those for the fewest scalar mask operations (plain C on the
+// 64-bit lane masks) between them, each of which costs the chain wait states (see add_eps).
 namespace isa {
 
 __device__ __forceinline__ u32 lo(u64 x) { return (u32)x; }

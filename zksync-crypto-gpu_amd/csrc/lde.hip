@@ -130,7 +130,7 @@ static bool lde_serial() {
 }
 
 // The LDE's launches with each pass of the coset NTTs merged over the cosets.  A small LDE is a few
-// launches of latency-shaped passes (13 x 2^14 at blowup 4: 33 us, 110 as ten launches of 52
+// launches of latency-shaped passes (13 x 2^14 at blowup 4: 29 us, 110 as ten launches of 52
 // workgroups over four streams); a large one reads the monomials once for 8 cosets.
 static int lde_run_merged(const ba_context *ctx, uint64_t *evals, uint64_t in_stride, uint64_t *mono,
                           uint64_t mono_stride, uint64_t *out, uint64_t out_col_stride, uint64_t out_coset_stride,

@@ -213,7 +213,7 @@ __device__ __forceinline__ void permute(u64 (&s)[WIDTH], const u64 *__restrict__
 // ---------------------------------------------------------------- one quad of threads per digest
 // Thread j of a quad holds lanes j, 4 + j and 8 + j (position j of each tile): the sums over tiles
 // are its own, M4 and the sum over all lanes are quad permutations.  A permutation is then a chain
-// of ~4.4 k instructions instead of ~9.9 k, for 1.7 times the work in all.
+// of ~4.2 k instructions instead of ~9.9 k, for 1.7 times the work in all.
 struct Quad {
   u32 j;       // position in the quad
   u32 m4[4];   // M4[j][(j + k) mod 4]
@@ -319,8 +319,8 @@ __device__ __forceinline__ void quad_permute(u64 (&s)[3], const Quad &q, const u
 
 // ---------------------------------------------------------------- 16 threads per digest
 // Thread i < 12 of a row of 16 holds lane i; the last four only keep the row sums whole.  Sums over
-// tiles and over all lanes are DPP row rotations.  A permutation is a chain of ~2.6 k instructions, for
-// 2.4 times the quad's work in all.
+// tiles and over all lanes are DPP row rotations.  A permutation is a chain of ~2.7 k instructions, for
+// 2.6 times the quad's work in all.
 struct Row {
   u32 lane;
   u32 m4[4];  // M4[j][(j + k) mod 4], j the position in the tile; 0 in idle threads
