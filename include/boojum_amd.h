@@ -150,7 +150,7 @@ int ba_bit_reverse_in_place(uint64_t *values, uint64_t stride, uint32_t log_rows
  * log_n + log_blowup <= 30, strides >= n, out distinct from evals / monomials, the context's
  * device current.  Every launch is on `stream`, in order: the inverse NTT's passes, then each pass
  * of the coset NTTs as one launch over up to 8 cosets (under ba_profile_begin, or with
- * BOOJUM_AMD_LDE_SERIAL=1 in the environment, one launch per coset). */
+ * BOOJUM_AMD_LDE_SERIAL=1 in the environment, one launch per coset of the same kernels). */
 int ba_lde_batch(ba_context_t ctx, uint64_t *evals, uint64_t in_stride, uint64_t *monomials,
                  uint64_t *out, uint64_t out_col_stride, uint64_t out_coset_stride, uint32_t log_n,
                  uint32_t num_cols, uint32_t log_blowup, ba_stream_t stream);

@@ -293,3 +293,36 @@ def test_lde_merged_cosets(ba, log_n, cols, lb, layout):
     assert np.array_equal(got, gl_oracle.lde(ev, log_n, cols, lb, nthreads=8))
     assert np.array_equal(mono, gl_oracle.batch_ntt(ev, log_n, cols, n, n, False, True, nthreads=8))
     assert np.array_equal(ev_after, ev)
+
+
+# A traced LDE launches each coset on its own, by the kernels and names of the untraced call's launches.
+@pytest.mark.parametrize("log_n,cols,lb,inverse,coset", [
+    (10, 5, 2, ["lat<10, true, true, false, false, true>"], ["lat_cosets<10, false>"]),
+    (11, 3, 1, ["lat_wide<11, true, true, true>"], ["lat_wide_cosets<11>"]),
+    (12, 100, 1, ["lat_wide<12, true, true, true>"], ["lat_wide_cosets<12>"]),
+    (12, 100, 2, ["lat_wide<12, true, true, true>"], ["contig_cosets<12, true, 4>"]),  # past 2^20 elements
+    (14, 13, 2, ["lat<7, true, true, true, true, false>", "lat<7, true, true, false, false, true>"],
+     ["lat_cosets<7, true>", "lat<7, true, false, false, false, false>"]),
+    (9, 3000, 2, ["contig<9, true, true, 1, false, 4>"], ["contig_cosets<9, false, 4>"]),
+    (16, 40, 4, ["strided<4, true, true, true, false, false>", "contig<12, true, true, 1, true, 4>"],
+     ["strided_cosets<4>", "contig<12, true, false, 0, true, 4>"])])
+def test_traced_lde_runs_the_calls_kernels(ba, log_n, cols, lb, inverse, coset):
+    from boojum_amd.profile import LaunchTrace
+    n = 1 << log_n
+    log(f"traced lde log_n={log_n} cols={cols} blowup=2^{lb}")
+    ev = raw_u64(np.random.default_rng(log_n), cols * n)
+    d_ev, d_out = ba.DeviceAllocation.from_host(ev), ba.DeviceAllocation(cols * (n << lb))
+    try:
+        with LaunchTrace(64) as tr:
+            ba.lde.lde_batch(ba._test_ctx, d_ev, log_n, cols, lb, d_out)
+        ba.synchronize()
+        names = list(tr.names)
+        tr.destroy()
+        got = d_out.to_host()
+    finally:
+        d_ev.free()
+        d_out.free()
+    args = {True: "gl::ntt::CosetArgs", False: "gl::ntt::PassArgs"}
+    want = [f"void gl::ntt::ntt_pass_{k}({args['cosets' in k]})" for k in inverse + coset * (1 << lb)]
+    assert names == want
+    assert np.array_equal(got, gl_oracle.lde(ev, log_n, cols, lb, nthreads=8))

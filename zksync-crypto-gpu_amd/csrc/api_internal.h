@@ -86,6 +86,7 @@ struct BaPassLaunch {
   uint64_t grid;
   uint32_t threads = gl::ntt::THREADS;
   const char *name;
+  const char *coset_name = nullptr;
   int pass;       // index of the pass inside its transform
   uint64_t col0;  // first column of the transform this launch covers
 };

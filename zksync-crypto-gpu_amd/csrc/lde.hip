@@ -120,7 +120,8 @@ int ba_build_lde(const ba_context *ctx, uint64_t *evals, uint64_t in_stride, uin
 }
 
 // BOOJUM_AMD_LDE_SERIAL=1 in the environment (read once) launches every coset's passes on their own,
-// in order, so that a profiler's per-kernel figures are one transform's.
+// in order, so that a profiler's per-kernel figures are one transform's; so does launch tracing.  The
+// kernels and their launch choices are those of the merged launches.
 static bool lde_serial() {
   static const bool serial = [] {
     const char *e = std::getenv("BOOJUM_AMD_LDE_SERIAL");
@@ -134,19 +135,20 @@ static bool lde_serial() {
 // workgroups over four streams); a large one reads the monomials once for 8 cosets.
 static int lde_run_merged(const ba_context *ctx, uint64_t *evals, uint64_t in_stride, uint64_t *mono,
                           uint64_t mono_stride, uint64_t *out, uint64_t out_col_stride, uint64_t out_coset_stride,
-                          uint32_t log_n, uint32_t num_cols, uint32_t log_blowup, hipStream_t stream) {
+                          uint32_t log_n, uint32_t num_cols, uint32_t log_blowup, bool apart, hipStream_t stream) {
   std::vector<BaPassLaunch> ls;
   int rc = ba_build_ntt(ctx, evals, mono, log_n, num_cols, in_stride, mono_stride, false, true, 0, 0, false, ls,
                         BA_LAT_AUTO);
   if (rc || (rc = ba_run_launches(ls, stream))) return rc;
   const uint32_t blowup = 1u << log_blowup;
-  const uint32_t log_at_once = std::min(log_blowup, 3u), at_once = 1u << log_at_once;
   static_assert(gl::ntt::MAX_COSETS == 8, "cosets of one launch");
+  const uint32_t log_merged = std::min(log_blowup, 3u);
+  const uint32_t log_at_once = apart ? 0 : log_merged, at_once = 1u << log_at_once;
   for (uint32_t c0 = 0; c0 < blowup; c0 += at_once) {
     ls.clear();
     rc = ba_build_ntt(ctx, mono, out + (uint64_t)c0 * out_coset_stride, log_n, num_cols, mono_stride, out_col_stride,
                       false, false, log_blowup, bitrev_bits(c0, log_blowup), /*in_bitrev_gather=*/true, ls,
-                      BA_LAT_AUTO, false, at_once);
+                      BA_LAT_AUTO, false, 1u << log_merged);
     if (rc) return rc;
     gl::ntt::CosetArgs first{};
     first.coset_stride = out_coset_stride;
@@ -157,13 +159,16 @@ static int lde_run_merged(const ba_context *ctx, uint64_t *evals, uint64_t in_st
     for (const BaPassLaunch &l : ls) {
       if (l.pass == 0) {
         first.a = l.args;
+        ba_trace_before(stream, l.coset_name);
         hipLaunchKernelGGL(l.coset_kernel, dim3((uint32_t)(l.grid << log_at_once)), dim3(l.threads), 0, stream,
                            first);
       } else {
         gl::ntt::PassArgs a = l.args;
         a.slice_stride = out_coset_stride;
+        ba_trace_before(stream, l.name);
         hipLaunchKernelGGL(l.kernels.single, dim3((uint32_t)l.grid, at_once), dim3(l.threads), 0, stream, a);
       }
+      ba_trace_after(stream);
       const hipError_t err = hipGetLastError();
       if (err != hipSuccess) return (int)err;
     }
@@ -186,8 +191,7 @@ static int lde_run(ba_context_t ctx, uint64_t *evals, uint64_t in_stride, uint64
   if (hipGetDevice(&device) != hipSuccess || device != ctx->device) return BA_ERROR_INVALID_VALUE;
   uint64_t *mono = monomials ? monomials : evals;
   const uint64_t mono_stride = monomials ? (1ull << log_n) : in_stride;
-  if (log_n < 4 || ba_trace_active() || lde_serial()) {
-    // whole transforms per thread, or launches that a trace or profile wants one by one
+  if (log_n < 4) {  // whole transforms per thread
     std::vector<BaLeveledLaunch> leveled;
     rc = ba_build_lde(ctx, evals, in_stride, monomials, out, out_col_stride, out_coset_stride, log_n,
                       num_cols, log_blowup, leveled, 0);
@@ -197,7 +201,7 @@ static int lde_run(ba_context_t ctx, uint64_t *evals, uint64_t in_stride, uint64
     rc = ba_run_launches(flat, (hipStream_t)stream);
   } else {
     rc = lde_run_merged(ctx, evals, in_stride, mono, mono_stride, out, out_col_stride, out_coset_stride, log_n,
-                        num_cols, log_blowup, (hipStream_t)stream);
+                        num_cols, log_blowup, ba_trace_active() || lde_serial(), (hipStream_t)stream);
   }
   if (rc || !natural_monomials) return rc;
   return ba_bit_reverse_in_place(mono, mono_stride, log_n, num_cols, stream);

@@ -130,6 +130,23 @@ const char *kernel_name(bool contig, uint32_t S, bool n2b, bool inverse, bool to
   return names.n[contig ? 1 : (shared_build ? 2 : 0)][S][n2b][inverse][top][scale][contig ? waves == 4 : gather];
 }
 
+// the same for the gathered first pass of an LDE's coset NTTs (4096-element tiles)
+struct CosetNames {
+  char n[3][13][80];  // strided, contiguous at 3 waves per SIMD, at 4
+  CosetNames() {
+    for (int s = 0; s < 13; s++) {
+      snprintf(n[0][s], sizeof(n[0][s]), "void gl::ntt::ntt_pass_strided_cosets<%d>(gl::ntt::CosetArgs)", s);
+      for (int w = 3; w <= 4; w++)
+        snprintf(n[w - 2][s], sizeof(n[w - 2][s]), "void gl::ntt::ntt_pass_contig_cosets<%d, %s, %d>(gl::ntt::CosetArgs)",
+                 s, s == TILE_LOG ? "true" : "false", w);
+    }
+  }
+};
+const char *coset_name(bool contig, uint32_t S, uint32_t waves) {
+  static const CosetNames names;
+  return names.n[!contig ? 0 : waves == 4 ? 2 : 1][S];
+}
+
 constexpr uint64_t kMaxGrid = 0x7FFFFFFFull;
 
 }  // namespace
@@ -295,8 +312,11 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
     a.tile_count = num_cols;
     l.threads = (uint32_t)wide_threads((int)log_n);
     l.kernels = {ba_pick_lat_wide(log_n, n2b, inverse, a.scale != SCALE_NONE), nullptr};
-    if (in_bitrev_gather) l.coset_kernel = ba_pick_lat_wide_cosets(log_n);
-    l.name = "ntt_pass_lat_wide";
+    l.name = ba_lat_wide_kernel_name(log_n, n2b, inverse, a.scale != SCALE_NONE);
+    if (in_bitrev_gather) {
+      l.coset_kernel = ba_pick_lat_wide_cosets(log_n);
+      l.coset_name = ba_lat_wide_cosets_kernel_name(log_n);
+    }
     l.pass = 0;
     l.col0 = 0;
     launches.push_back(l);
@@ -328,8 +348,11 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
                        : (chunks + (1u << (LAT_TL - S)) - 1) >> (LAT_TL - S);
       a.tile_count = (uint32_t)l.grid;
       l.kernels = ba_pick_lat(S, strided, n2b, inverse, top, scale);
-      if (a.in_bitrev) l.coset_kernel = ba_pick_lat_cosets(S, strided);
-      l.name = ba_lat_kernel_name(S, strided, n2b, inverse, top, scale);
+      if (a.in_bitrev) {
+        l.coset_kernel = ba_pick_lat_cosets(S, strided);
+        l.coset_name = ba_lat_cosets_kernel_name(S, strided);
+      }
+      l.name = ba_lat_kernel_name(S, strided, n2b, inverse, strided && top, scale);
       l.pass = p;
       l.col0 = 0;
       if (!l.kernels.single || (a.in_bitrev && !l.coset_kernel)) return BA_ERROR_INVALID_VALUE;
@@ -391,11 +414,13 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
       const bool shared_build =
           shared && !contig && l.kernels.single != pick_kernel(contig, S, n2b, inverse, top, scale, big, gather, waves, false).single;
       l.name = kernel_name(contig, S, n2b, inverse, contig ? big : top, scale, gather, waves, shared_build);
-      if (a.in_bitrev)
+      if (a.in_bitrev) {
         l.coset_kernel = !contig      ? ba_pick_strided_cosets(S)
                          : S <= 8     ? ba_pick_contig_lo_cosets(S)
                          : waves == 3 ? ba_pick_contig_hi3_cosets(S)
                                       : ba_pick_contig_hi_cosets(S);
+        l.coset_name = coset_name(contig, S, waves);
+      }
       l.pass = p;
       l.col0 = c0;
       if (!l.kernels.single || (a.in_bitrev && !l.coset_kernel)) return BA_ERROR_INVALID_VALUE;

@@ -32,7 +32,11 @@ BaKernels ba_pick_tiny(uint32_t log_n, bool n2b, bool inverse);
 constexpr int BA_LAT_MIN_CONTIG = 4, BA_LAT_MAX_CONTIG = 10;
 constexpr int BA_LAT_MIN_STRIDED = 5, BA_LAT_MAX_STRIDED = 8;
 BaKernels ba_pick_lat(uint32_t S, bool strided, bool n2b, bool inverse, bool top, bool scale);
+// kernel names as rocprofv3 prints them
 const char *ba_lat_kernel_name(uint32_t S, bool strided, bool n2b, bool inverse, bool top, bool scale);
+const char *ba_lat_cosets_kernel_name(uint32_t S, bool strided);
+const char *ba_lat_wide_kernel_name(uint32_t S, bool n2b, bool inverse, bool scale);
+const char *ba_lat_wide_cosets_kernel_name(uint32_t S);
 
 // the first pass of several coset NTTs of an LDE (gathered, coset-scaled n2b forward): strided over
 // 4..8 bits; contiguous over the whole column of 4..8 / 9..12 bits (waves 4 or 3); latency-shaped

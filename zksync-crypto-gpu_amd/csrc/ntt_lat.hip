@@ -86,10 +86,13 @@ BaCosetKernel ba_pick_lat_wide_cosets(uint32_t S) {
 }
 
 namespace {
-// [S][n2b][inverse][strided][top][scale], as rocprofv3 prints them; built by the first caller
-// (a function-local static initialiser, so concurrent first calls are safe)
+// as rocprofv3 prints them; built by the first caller (a function-local static initialiser, so
+// concurrent first calls are safe)
 struct LatNames {
-  char n[11][2][2][2][2][2][100];
+  char n[11][2][2][2][2][2][100];  // [S][n2b][inverse][strided][top][scale]
+  char cosets[11][2][80];          // [S][strided]
+  char wide[2][2][2][2][80];       // [S - 11][n2b][inverse][scale]
+  char wide_cosets[2][80];         // [S - 11]
   LatNames() {
     static const char *tf[2] = {"false", "true"};
     for (int s = 0; s < 11; s++)
@@ -101,11 +104,36 @@ struct LatNames {
                 snprintf(n[s][d][i][st][tp][sc], sizeof(n[s][d][i][st][tp][sc]),
                          "void gl::ntt::ntt_pass_lat<%d, %s, %s, %s, %s, %s>(gl::ntt::PassArgs)", s, tf[d], tf[i],
                          tf[st], tf[tp], tf[sc]);
+    for (int s = 0; s < 11; s++)
+      for (int st = 0; st < 2; st++)
+        snprintf(cosets[s][st], sizeof(cosets[s][st]), "void gl::ntt::ntt_pass_lat_cosets<%d, %s>(gl::ntt::CosetArgs)",
+                 s, tf[st]);
+    for (int s = 0; s < 2; s++) {
+      for (int d = 0; d < 2; d++)
+        for (int i = 0; i < 2; i++)
+          for (int sc = 0; sc < 2; sc++)
+            snprintf(wide[s][d][i][sc], sizeof(wide[s][d][i][sc]),
+                     "void gl::ntt::ntt_pass_lat_wide<%d, %s, %s, %s>(gl::ntt::PassArgs)", s + 11, tf[d], tf[i], tf[sc]);
+      snprintf(wide_cosets[s], sizeof(wide_cosets[s]), "void gl::ntt::ntt_pass_lat_wide_cosets<%d>(gl::ntt::CosetArgs)",
+               s + 11);
+    }
   }
 };
+const LatNames &lat_names() {
+  static const LatNames names;
+  return names;
+}
 }  // namespace
 
 const char *ba_lat_kernel_name(uint32_t S, bool strided, bool n2b, bool inverse, bool top, bool scale) {
-  static const LatNames names;
-  return S <= 10 ? names.n[S][n2b][inverse][strided][top][scale] : "ntt_pass_lat";
+  return S <= 10 ? lat_names().n[S][n2b][inverse][strided][top][scale] : "ntt_pass_lat";
+}
+const char *ba_lat_cosets_kernel_name(uint32_t S, bool strided) {
+  return S <= 10 ? lat_names().cosets[S][strided] : "ntt_pass_lat_cosets";
+}
+const char *ba_lat_wide_kernel_name(uint32_t S, bool n2b, bool inverse, bool scale) {
+  return S == 11 || S == 12 ? lat_names().wide[S - 11][n2b][inverse][scale] : "ntt_pass_lat_wide";
+}
+const char *ba_lat_wide_cosets_kernel_name(uint32_t S) {
+  return S == 11 || S == 12 ? lat_names().wide_cosets[S - 11] : "ntt_pass_lat_wide_cosets";
 }
