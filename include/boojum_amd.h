@@ -272,9 +272,9 @@ int ba_batch_plan_destroy(ba_batch_plan_t plan);
  * size; 0 = built-in choice: 1024-element tiles for batches of at most 2^20 elements (2^21 for
  * columns of 2^11), else 4096).  A call's columns of 2^11, and 96 or more of 2^12, take one whole
  * column per workgroup in place of the 1024-element tiles.  An LDE call's coset NTTs take the
- * 1024-element tiles by that batch-size rule alone, counting every coset of a launch.  Valid splits:
- * log_n <= 12 one pass of log_n bits; log_n > 12 a contiguous pass of 9..12 bits and strided passes
- * of 4..10 bits (at most 8 passes).
+ * 1024-element tiles by that batch-size rule, counting every coset of a launch, while no plan of
+ * theirs (BA_TUNING_LDE_COSETS below) is set.  Valid splits: log_n <= 12 one pass of log_n bits;
+ * log_n > 12 a contiguous pass of 9..12 bits and strided passes of 4..10 bits (at most 8 passes).
  *
  * ba_autotune times every valid split, then each pass's reps, then contig_waves, then (log_n 4..18)
  * the 1024-element tiles against the best of those, for plain NTTs of both input orders and for

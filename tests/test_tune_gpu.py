@@ -383,3 +383,52 @@ def test_contiguous_pass_gathers_short_lde_columns(ba, log_n, waves):
                     d.free()
     finally:
         ctx.destroy()
+
+
+def _pass_names(ba, fn):
+    """The traced passes of fn's launches, as "contig<9, true, false, 0, true, 4>"."""
+    from boojum_amd.profile import LaunchTrace
+    with LaunchTrace(256) as tr:
+        fn()
+    ba.synchronize()
+    names = [s.split("ntt_pass_")[1].split("(")[0] for s in tr.names]
+    tr.destroy()
+    return names
+
+
+# A plan of the LDE's coset NTTs runs at every size, the small ones included that would take the latency-
+# shaped passes without one: every width of the gathered contiguous pass, both its builds, every width of
+# the gathered strided pass; one column and a partial last tile, one and several launches of cosets.
+@pytest.mark.parametrize("log_n,bits,waves", [(k, [k], 0) for k in range(4, 9)] +
+                         [(k, [k], w) for k in range(9, 13) for w in (3, 4)] +
+                         [(13, [9, 4], 3), (14, [9, 5], 0), (15, [9, 6], 3), (16, [9, 7], 4), (17, [9, 8], 3)])
+def test_lde_coset_plan_runs_at_small_sizes(ba, log_n, bits, waves):
+    n = 1 << log_n
+    w = 3 if bits[0] < 9 else waves or 4
+    if len(bits) == 1:
+        want = [f"contig_cosets<{log_n}, {'true' if log_n == 12 else 'false'}, {w}>"]
+    else:
+        want = [f"strided_cosets<{bits[1]}>", f"contig<{bits[0]}, true, false, 0, true, {w}>"]
+    ctx = ba.Context.create(12, 12)
+    try:
+        for cols, reps, lb in ((1, 1, 1), (max(2, 3 * 4096 >> log_n) + 1, 2, 2), (2, 1, 4)):
+            small = cols << (log_n + min(lb, 3)) <= 1 << (LAT_MAX_LOG_ELEMS + (log_n == 11))
+            x = raw_u64(np.random.default_rng(log_n), n * cols)
+            d_ev, d_mono = ba.DeviceAllocation.from_host(x), ba.DeviceAllocation(n * cols)
+            d_out = ba.DeviceAllocation(cols * (n << lb))
+            call = lambda: ba.lde.lde_batch(ctx, d_ev, log_n, cols, lb, d_out, monomials=d_mono)  # noqa: E731
+            try:
+                log(f"lde plan log_n={log_n} bits={bits} waves={waves} cols={cols} blowup={1 << lb}")
+                ba.tune.set_plan(ctx, log_n, ba.tune.LDE_COSETS, bits, [reps] * len(bits), waves)
+                assert _pass_names(ba, call)[-(len(want) << lb):] == want * (1 << lb)
+                d_out.copy_from_host(np.zeros(cols * (n << lb), dtype=np.uint64))
+                call()  # untraced: the cosets of a pass in one launch
+                ba.synchronize()
+                assert np.array_equal(d_out.to_host(), gl_oracle.lde(x, log_n, cols, lb, nthreads=8))
+                ba.tune.set_plan(ctx, log_n, ba.tune.LDE_COSETS, None)
+                assert any("cosets" in s and "lat" in s for s in _pass_names(ba, call)) == small
+            finally:
+                for d in (d_ev, d_mono, d_out):
+                    d.free()
+    finally:
+        ctx.destroy()

@@ -289,10 +289,11 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
     return BA_SUCCESS;
   }
 
-  // an LDE call's coset NTTs: by the elements of all its cosets (a tuned tile_log is for plain NTTs)
+  // an LDE call's coset NTTs: by the elements of all its cosets, unless they have a plan of their own
+  // (whose passes are those of 4096-element tiles)
   const bool latency = in_bitrev_gather
-                           ? lat == BA_LAT_AUTO && ba_latency_shape_exists(log_n) &&
-                                 small_batch((uint64_t)num_cols * cosets, log_n)
+                           ? lat == BA_LAT_AUTO && !ctx->tuned[BA_TUNING_LDE_COSETS][log_n].valid &&
+                                 ba_latency_shape_exists(log_n) && small_batch((uint64_t)num_cols * cosets, log_n)
                            : ba_use_latency_passes(ctx, log_n, n2b, num_cols, lat);
   // single calls only: a batch plan's groups have 256 threads per workgroup
   if (latency && lat == BA_LAT_AUTO && wide_columns(log_n, (uint64_t)num_cols * cosets)) {
