@@ -432,3 +432,31 @@ def test_lde_coset_plan_runs_at_small_sizes(ba, log_n, bits, waves):
                     d.free()
     finally:
         ctx.destroy()
+
+
+# The LDE's inverse NTT takes the latency-shaped passes in small LDEs (unless tile_log says 12), and its class's
+# split in larger ones, also where tile_log 10 puts every plain NTT of the class on them.
+@pytest.mark.parametrize("log_n,bits", [(9, [9]), (12, [12]), (14, [10, 4]), (18, [9, 5, 4])])
+def test_lde_inverse_under_tile_log(ba, log_n, bits):
+    n = 1 << log_n
+    ctx = ba.Context.create(12, 12)
+    try:
+        for cols in (2, (1 << (LAT_MAX_LOG_ELEMS + 1) >> log_n) + 1):
+            x = raw_u64(np.random.default_rng(log_n), n * cols)
+            want = gl_oracle.lde(x, log_n, cols, 1, nthreads=8)
+            d_ev, d_mono = ba.DeviceAllocation.from_host(x), ba.DeviceAllocation(n * cols)
+            d_out = ba.DeviceAllocation(2 * n * cols)
+            try:
+                for tile in (0, 10, 12):
+                    log(f"lde inverse log_n={log_n} cols={cols} tile_log={tile}")
+                    ba.tune.set_plan(ctx, log_n, False, bits, [1] * len(bits), tile_log=tile)
+                    names = _pass_names(ba, lambda: ba.lde.lde_batch(ctx, d_ev, log_n, cols, 1, d_out, monomials=d_mono))
+                    lat = cols == 2 and tile != 12
+                    assert names[0].startswith("lat") == lat, names
+                    assert lat or [s.split("<")[1].split(",")[0] for s in names[:len(bits)]] == [str(b) for b in bits[::-1]]
+                    assert np.array_equal(d_out.to_host(), want)
+            finally:
+                for d in (d_ev, d_mono, d_out):
+                    d.free()
+    finally:
+        ctx.destroy()

@@ -92,13 +92,14 @@ struct BaPassLaunch {
 };
 
 // Which transforms may run the latency-shaped passes (1024-element tiles):
-//   BA_LAT_NEVER  an LDE's transforms inside batch plans (as BA_LAT_TUNED below), or one coset at a time;
+//   BA_LAT_NEVER  an LDE's transforms inside batch plans, and the inverse NTT of a large LDE call;
 //   BA_LAT_TUNED  the size class's tuned tile_log is 10 (batch plans: a merged small transform
 //                 runs beside other groups of its level, where the throughput passes measured
 //                 as fast and the extra grouped launches cost more);
 //   BA_LAT_AUTO   that, or else the batch holds at most 2^BA_LAT_MAX_LOG_ELEMS elements and the
-//                 tuned tile_log is not 12 (single batch NTT calls, an LDE call's inverse NTT);
-//                 for an LDE call's coset NTTs, by the elements of all cosets of a launch.
+//                 tuned tile_log is not 12 (single batch NTT calls, the inverse NTT of a small LDE
+//                 call); for an LDE call's coset NTTs, by the elements of all cosets of a launch, and
+//                 only without a plan of their own.
 enum BaLatPolicy { BA_LAT_NEVER = 0, BA_LAT_TUNED = 1, BA_LAT_AUTO = 2 };
 // Appends the pass launches of one batch NTT (arguments validated) to `launches`.  shared: the
 // launches will run beside other streams' work (serve batches), so strided passes whose default
@@ -118,6 +119,8 @@ void ba_scale_factors(uint32_t log_n, bool inverse, uint32_t log_ext, uint32_t c
 constexpr uint32_t BA_LAT_MAX_LOG_ELEMS = 20;
 // log_n has a latency-shaped plan (4..18); a batch NTT of num_cols columns of 2^log_n runs it.
 bool ba_latency_shape_exists(uint32_t log_n);
+// The built-in rule: a batch of at most 2^BA_LAT_MAX_LOG_ELEMS elements (twice that at log_n 11).
+bool ba_small_batch(uint64_t cols, uint32_t log_n);
 bool ba_use_latency_passes(const ba_context *ctx, uint32_t log_n, bool n2b, uint32_t num_cols, BaLatPolicy lat);
 // Launches them one after another on `stream` (single-batch kernels).
 int ba_run_launches(const std::vector<BaPassLaunch> &launches, hipStream_t stream);

@@ -137,8 +137,11 @@ static int lde_run_merged(const ba_context *ctx, uint64_t *evals, uint64_t in_st
                           uint64_t mono_stride, uint64_t *out, uint64_t out_col_stride, uint64_t out_coset_stride,
                           uint32_t log_n, uint32_t num_cols, uint32_t log_blowup, bool apart, hipStream_t stream) {
   std::vector<BaPassLaunch> ls;
+  // The inverse NTT is latency-shaped by size alone: a tile_log of 10 says that plain NTTs of the class take
+  // those passes whatever the batch, which costs a large LDE up to a third of its time (blowup 2, 128
+  // columns of 2^18: 1000 us against 754; 2048 of 2^14: 753 against 660).
   int rc = ba_build_ntt(ctx, evals, mono, log_n, num_cols, in_stride, mono_stride, false, true, 0, 0, false, ls,
-                        BA_LAT_AUTO);
+                        ba_small_batch(num_cols, log_n) ? BA_LAT_AUTO : BA_LAT_NEVER);
   if (rc || (rc = ba_run_launches(ls, stream))) return rc;
   const uint32_t blowup = 1u << log_blowup;
   static_assert(gl::ntt::MAX_COSETS == 8, "cosets of one launch");

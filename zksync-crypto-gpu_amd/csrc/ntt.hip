@@ -222,7 +222,7 @@ static uint32_t lat_max_log_elems() {
 // chip enough of them (1 column 9.5 / 8.5, 64 10.2 / 10.0, 128 10.7 / 11.5, 256 11.6 / 16.1).
 static bool wide_columns(uint32_t log_n, uint64_t cols) { return log_n == 11 || (log_n == 12 && cols >= 96); }
 
-static bool small_batch(uint64_t cols, uint32_t log_n) {
+bool ba_small_batch(uint64_t cols, uint32_t log_n) {
   const uint32_t m = lat_max_log_elems();
   return m > 0 && (cols << log_n) <= (1ull << std::min(m + (log_n == 11), 40u));
 }
@@ -238,7 +238,7 @@ bool ba_use_latency_passes(const ba_context *ctx, uint32_t log_n, bool n2b, uint
   const BaTuned &t = ctx->tuned[n2b][log_n];
   if (t.valid && t.tile_log) return t.tile_log == LAT_TL;
   if (lat == BA_LAT_TUNED) return false;
-  return small_batch(num_cols, log_n);
+  return ba_small_batch(num_cols, log_n);
 }
 
 void ba_scale_factors(uint32_t log_n, bool inverse, uint32_t log_ext, uint32_t coset_idx,
@@ -293,7 +293,7 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
   // (whose passes are those of 4096-element tiles)
   const bool latency = in_bitrev_gather
                            ? lat == BA_LAT_AUTO && !ctx->tuned[BA_TUNING_LDE_COSETS][log_n].valid &&
-                                 ba_latency_shape_exists(log_n) && small_batch((uint64_t)num_cols * cosets, log_n)
+                                 ba_latency_shape_exists(log_n) && ba_small_batch((uint64_t)num_cols * cosets, log_n)
                            : ba_use_latency_passes(ctx, log_n, n2b, num_cols, lat);
   // single calls only: a batch plan's groups have 256 threads per workgroup
   if (latency && lat == BA_LAT_AUTO && wide_columns(log_n, (uint64_t)num_cols * cosets)) {
