@@ -277,10 +277,11 @@ int ba_batch_plan_destroy(ba_batch_plan_t plan);
  * log_n > 12 a contiguous pass of 9..12 bits and strided passes of 4..10 bits (at most 8 passes).
  *
  * ba_autotune times every valid split, then each pass's reps, then contig_waves, then (log_n 4..18)
- * the 1024-element tiles against the best of those, for plain NTTs of both input orders and for
- * the LDE's coset NTTs (BA_TUNING_LDE_COSETS below), for log_n in [log_n_min,
- * log_n_max] and both input orders, on batches of max(elems_per_trial, 2^log_n) elements of
- * scratch memory it allocates and frees, and keeps the fastest on `ctx`; every later transform
+ * the 1024-element tiles against the best of those (log_n 11 and 12: as calls run them and as batch
+ * plans do), for plain NTTs of both input orders and for the LDE's coset NTTs (BA_TUNING_LDE_COSETS
+ * below), for log_n in [log_n_min, log_n_max], on batches of max(elems_per_trial, 2^log_n) elements
+ * (an LDE's: of its two cosets, or one column's) of scratch memory it allocates and frees, and keeps
+ * the fastest on `ctx`; every later transform
  * (NTT, LDE, batch plan) on `ctx` uses it.  Results are bit-identical for every plan.  Tuning
  * state is per context and must not change while other threads launch with that context. */
 typedef struct {
@@ -294,9 +295,11 @@ int ba_autotune(ba_context_t ctx, uint32_t log_n_min, uint32_t log_n_max, uint64
                 ba_stream_t stream);
 /* bitrev_inputs = BA_TUNING_LDE_COSETS addresses the plan of the LDE's coset NTTs (natural ->
  * bit-reversed forward NTTs that gather the bit-reversed monomials and scale by the coset in their
- * first pass), which ba_autotune times on that transform: its strided passes are at most 8 bits
- * and its tile_log is 0.  0 and 1 address plain batch NTTs of natural and bit-reversed input
- * (the LDE's inverse NTT follows 0). */
+ * first pass), which ba_autotune times as an LDE call at blowup 2 launches them: its strided passes
+ * are at most 8 bits and its tile_log is 0.  A plan set here runs at every size; a tuned one leaves
+ * small LDEs to the built-in rule where that measured faster on the largest of them.  0 and 1 address
+ * plain batch NTTs of natural and bit-reversed input (the LDE's inverse NTT follows 0, its tile_log of
+ * 10 in small LDEs only). */
 #define BA_TUNING_LDE_COSETS 2
 /* the plan in use for (log_n, bitrev_inputs): tuned if set, else the built-in one */
 int ba_tuning_get(ba_context_t ctx, uint32_t log_n, int bitrev_inputs, ba_tuned_plan *plan);

@@ -460,3 +460,48 @@ def test_lde_inverse_under_tile_log(ba, log_n, bits):
                     d.free()
     finally:
         ctx.destroy()
+
+
+@pytest.mark.parametrize("log_n,elems", [(11, 1 << 16), (12, 1 << 19), (14, 1 << 19), (3, 1 << 12)])
+def test_autotune_times_the_calls_launches(ba, log_n, elems):
+    """The tuner times an LDE's coset NTTs by the launches that an LDE call makes, under the plan and under
+    the built-in rule for small ones, and whole-column latency passes also in the two-pass form that batch
+    plans run; what it keeps gives exact LDEs, small and large, and so does a plan read back and set."""
+    from boojum_amd.profile import LaunchTrace
+    n = 1 << log_n
+    ctx = ba.Context.create(12, 12)
+    try:
+        with LaunchTrace(1 << 14) as tr:
+            ba.tune.autotune(ctx, log_n, log_n, elems_per_trial=elems)
+        assert tr.count < 1 << 14
+        names = {s.split("ntt_")[1].split("(")[0] for s in tr.names if "ntt_" in s}
+        tr.destroy()
+        first = {11: ["pass_contig_cosets<11, false, 4>", "pass_lat_wide_cosets<11>"],
+                 12: ["pass_contig_cosets<12, true, 4>", "pass_lat_wide_cosets<12>"],
+                 14: ["pass_strided_cosets<4>", "pass_strided_cosets<5>", "pass_lat_cosets<7, true>"], 3: []}[log_n]
+        assert set(first) <= names, names
+        # no launch of one coset by the kernels of batch plans
+        assert not any(s.startswith("pass_contig<") and ", 2, " in s for s in names), names
+        assert not any(s.startswith("pass_strided<") and s.endswith("true>") for s in names), names
+        if log_n == 11:  # columns of 2^11 as calls and as batch plans run them
+            assert {"pass_lat_wide<11, true, false, false>", "pass_lat<6, true, false, false, false, false>"} <= names
+        for cols in (3, (1 << (LAT_MAX_LOG_ELEMS + 1) >> log_n) + 1):
+            x = raw_u64(np.random.default_rng(log_n), n * cols)
+            want = gl_oracle.lde(x, log_n, cols, 1, nthreads=8)
+            d_ev, d_mono, d_out = (ba.DeviceAllocation(k * n * cols) for k in (1, 1, 2))
+            try:
+                d_ev.copy_from_host(x)
+                for read_back in (False, True):
+                    if read_back:
+                        bits, reps = ba.tune.get_plan(ctx, log_n, ba.tune.LDE_COSETS)
+                        ba.tune.set_plan(ctx, log_n, ba.tune.LDE_COSETS, bits, reps,
+                                         ba.tune.get_contig_waves(ctx, log_n, ba.tune.LDE_COSETS))
+                    log(f"lde after tuning log_n={log_n} cols={cols} read_back={read_back}")
+                    ba.lde.lde_batch(ctx, d_ev, log_n, cols, 1, d_out, monomials=d_mono)
+                    ba.synchronize()
+                    assert np.array_equal(d_out.to_host(), want)
+            finally:
+                for d in (d_ev, d_mono, d_out):
+                    d.free()
+    finally:
+        ctx.destroy()

@@ -40,6 +40,8 @@ struct BaTuned {
   uint32_t reps[8];
   uint32_t contig_waves;  // waves per SIMD of the 9..12-bit contiguous pass: 3, 4, or 0 = built-in
   uint32_t tile_log;      // plain batch NTTs: 10 latency-shaped tiles, 12 4096-element tiles, 0 by batch size
+  bool small_by_size;     // LDE coset NTTs, tuned: the plan lost to the built-in rule for small LDEs, which
+                          // they keep (a plan that a caller sets runs at every size)
 };
 
 struct ba_context {
@@ -167,6 +169,11 @@ int ba_build_lde(const ba_context *ctx, uint64_t *evals, uint64_t in_stride, uin
                  uint64_t *out, uint64_t out_col_stride, uint64_t out_coset_stride, uint32_t log_n,
                  uint32_t num_cols, uint32_t log_blowup, std::vector<BaLeveledLaunch> &launches,
                  uint32_t first_level);
+// Enqueues the coset NTTs of an LDE call (log_n >= 4) from its bit-reversed monomials: each pass as one
+// launch over up to 8 cosets, or with `apart` over one, by the same kernels.
+int ba_launch_lde_cosets(const ba_context *ctx, const uint64_t *mono, uint64_t mono_stride, uint64_t *out,
+                         uint64_t out_col_stride, uint64_t out_coset_stride, uint32_t log_n, uint32_t num_cols,
+                         uint32_t log_blowup, bool apart, hipStream_t stream);
 int ba_validate_ntt(uint32_t log_n, uint64_t stride_in, uint64_t stride_out, uint32_t log_ext,
                     uint32_t coset_idx);
 

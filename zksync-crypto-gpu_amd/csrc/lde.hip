@@ -130,26 +130,20 @@ static bool lde_serial() {
   return serial;
 }
 
-// The LDE's launches with each pass of the coset NTTs merged over the cosets.  A small LDE is a few
-// launches of latency-shaped passes (13 x 2^14 at blowup 4: 29 us, 110 as ten launches of 52
-// workgroups over four streams); a large one reads the monomials once for 8 cosets.
-static int lde_run_merged(const ba_context *ctx, uint64_t *evals, uint64_t in_stride, uint64_t *mono,
-                          uint64_t mono_stride, uint64_t *out, uint64_t out_col_stride, uint64_t out_coset_stride,
-                          uint32_t log_n, uint32_t num_cols, uint32_t log_blowup, bool apart, hipStream_t stream) {
+// Each pass of the coset NTTs is merged over the cosets.  A small LDE is a few launches of
+// latency-shaped passes (13 x 2^14 at blowup 4: 29 us, 110 as ten launches of 52 workgroups over four
+// streams); a large one reads the monomials once for 8 cosets.
+int ba_launch_lde_cosets(const ba_context *ctx, const uint64_t *mono, uint64_t mono_stride, uint64_t *out,
+                         uint64_t out_col_stride, uint64_t out_coset_stride, uint32_t log_n, uint32_t num_cols,
+                         uint32_t log_blowup, bool apart, hipStream_t stream) {
   std::vector<BaPassLaunch> ls;
-  // The inverse NTT is latency-shaped by size alone: a tile_log of 10 says that plain NTTs of the class take
-  // those passes whatever the batch, which costs a large LDE up to a third of its time (blowup 2, 128
-  // columns of 2^18: 1000 us against 754; 2048 of 2^14: 753 against 660).
-  int rc = ba_build_ntt(ctx, evals, mono, log_n, num_cols, in_stride, mono_stride, false, true, 0, 0, false, ls,
-                        ba_small_batch(num_cols, log_n) ? BA_LAT_AUTO : BA_LAT_NEVER);
-  if (rc || (rc = ba_run_launches(ls, stream))) return rc;
   const uint32_t blowup = 1u << log_blowup;
   static_assert(gl::ntt::MAX_COSETS == 8, "cosets of one launch");
   const uint32_t log_merged = std::min(log_blowup, 3u);
   const uint32_t log_at_once = apart ? 0 : log_merged, at_once = 1u << log_at_once;
   for (uint32_t c0 = 0; c0 < blowup; c0 += at_once) {
     ls.clear();
-    rc = ba_build_ntt(ctx, mono, out + (uint64_t)c0 * out_coset_stride, log_n, num_cols, mono_stride, out_col_stride,
+    int rc = ba_build_ntt(ctx, mono, out + (uint64_t)c0 * out_coset_stride, log_n, num_cols, mono_stride, out_col_stride,
                       false, false, log_blowup, bitrev_bits(c0, log_blowup), /*in_bitrev_gather=*/true, ls,
                       BA_LAT_AUTO, false, 1u << log_merged);
     if (rc) return rc;
@@ -203,8 +197,15 @@ static int lde_run(ba_context_t ctx, uint64_t *evals, uint64_t in_stride, uint64
     for (const BaLeveledLaunch &l : leveled) flat.push_back(l.launch);  // already in dependency order
     rc = ba_run_launches(flat, (hipStream_t)stream);
   } else {
-    rc = lde_run_merged(ctx, evals, in_stride, mono, mono_stride, out, out_col_stride, out_coset_stride, log_n,
-                        num_cols, log_blowup, ba_trace_active() || lde_serial(), (hipStream_t)stream);
+    // The inverse NTT is latency-shaped by size alone: a tile_log of 10 says that plain NTTs of the class
+    // take those passes whatever the batch, which costs a large LDE up to a third of its time (blowup 2,
+    // 128 columns of 2^18: 1000 us against 754; 2048 of 2^14: 753 against 660).
+    std::vector<BaPassLaunch> ls;
+    rc = ba_build_ntt(ctx, evals, mono, log_n, num_cols, in_stride, mono_stride, false, true, 0, 0, false, ls,
+                      ba_small_batch(num_cols, log_n) ? BA_LAT_AUTO : BA_LAT_NEVER);
+    if (rc || (rc = ba_run_launches(ls, (hipStream_t)stream))) return rc;
+    rc = ba_launch_lde_cosets(ctx, mono, mono_stride, out, out_col_stride, out_coset_stride, log_n, num_cols,
+                              log_blowup, ba_trace_active() || lde_serial(), (hipStream_t)stream);
   }
   if (rc || !natural_monomials) return rc;
   return ba_bit_reverse_in_place(mono, mono_stride, log_n, num_cols, stream);

@@ -291,8 +291,9 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
 
   // an LDE call's coset NTTs: by the elements of all its cosets, unless they have a plan of their own
   // (whose passes are those of 4096-element tiles)
+  const BaTuned &of_cosets = ctx->tuned[BA_TUNING_LDE_COSETS][log_n];
   const bool latency = in_bitrev_gather
-                           ? lat == BA_LAT_AUTO && !ctx->tuned[BA_TUNING_LDE_COSETS][log_n].valid &&
+                           ? lat == BA_LAT_AUTO && (!of_cosets.valid || of_cosets.small_by_size) &&
                                  ba_latency_shape_exists(log_n) && ba_small_batch((uint64_t)num_cols * cosets, log_n)
                            : ba_use_latency_passes(ctx, log_n, n2b, num_cols, lat);
   // single calls only: a batch plan's groups have 256 threads per workgroup

@@ -69,12 +69,13 @@ struct Timer {
     if (err == hipSuccess) err = hipEventCreate(&e1);
     return (int)err;
   }
-  // mean ms per run of `ls` over enough repeats to fill ~1 ms, best of two groups
-  int time(const std::vector<BaPassLaunch> &ls, float &ms) {
-    int rc = ba_run_launches(ls, stream);  // warm-up, and a first estimate
+  // mean ms per run() over enough repeats to fill ~1 ms, best of two groups
+  template <typename F>
+  int time(F &&run, float &ms) {
+    int rc = run();  // warm-up, and a first estimate
     if (rc) return rc;
     hipError_t err = hipEventRecord(e0, stream);
-    if (err == hipSuccess) rc = ba_run_launches(ls, stream);
+    if (err == hipSuccess) rc = run();
     if (err == hipSuccess && rc == 0) err = hipEventRecord(e1, stream);
     if (err == hipSuccess && rc == 0) err = hipEventSynchronize(e1);
     float one = 0;
@@ -84,7 +85,7 @@ struct Timer {
     float best = 1e30f;
     for (int g = 0; g < 2; g++) {
       err = hipEventRecord(e0, stream);
-      for (int i = 0; err == hipSuccess && rc == 0 && i < reps; i++) rc = ba_run_launches(ls, stream);
+      for (int i = 0; err == hipSuccess && rc == 0 && i < reps; i++) rc = run();
       if (err == hipSuccess && rc == 0) err = hipEventRecord(e1, stream);
       if (err == hipSuccess && rc == 0) err = hipEventSynchronize(e1);
       float t = 0;
@@ -97,18 +98,23 @@ struct Timer {
   }
 };
 
-// kind: 0 plain b2n forward, 1 plain n2b forward, BA_TUNING_LDE_COSETS the LDE's coset NTT (n2b
-// forward with coset scale, reading its input bit-reversed through the gathered first pass)
+// kind: 0 plain b2n forward, 1 plain n2b forward, BA_TUNING_LDE_COSETS an LDE call's coset NTTs (n2b
+// forward with coset scale, reading their input bit-reversed through the gathered first pass) at
+// blowup 2, launched as the call launches them.  lat: plain NTTs as a call runs them (BA_LAT_AUTO) or
+// as a batch plan does (BA_LAT_TUNED).
 int time_entry(ba_context *ctx, const BaTuned &entry, uint32_t log_n, int kind, const uint64_t *in, uint64_t *out,
-               uint32_t cols, Timer &timer, float &ms) {
+               uint32_t cols, Timer &timer, float &ms, BaLatPolicy lat = BA_LAT_AUTO) {
   ctx->tuned[kind][log_n] = entry;
   const uint64_t n = 1ull << log_n;
-  std::vector<BaPassLaunch> ls;
   const bool lde = kind == BA_TUNING_LDE_COSETS;
+  if (lde && log_n >= 4)
+    return timer.time(
+        [&] { return ba_launch_lde_cosets(ctx, in, n, out, 2 * n, n, log_n, cols, 1, false, timer.stream); }, ms);
+  std::vector<BaPassLaunch> ls;
   const int rc = lde ? ba_build_ntt(ctx, in, out, log_n, cols, n, n, false, false, 1, 1, true, ls, BA_LAT_NEVER)
-                     : ba_build_ntt(ctx, in, out, log_n, cols, n, n, kind == 0, false, 0, 0, false, ls, BA_LAT_AUTO);
+                     : ba_build_ntt(ctx, in, out, log_n, cols, n, n, kind == 0, false, 0, 0, false, ls, lat);
   if (rc) return rc;
-  return timer.time(ls, ms);
+  return timer.time([&] { return ba_run_launches(ls, timer.stream); }, ms);
 }
 
 // the gathered first pass (top strided pass) of an LDE coset NTT exists for 4..8 bits
@@ -122,7 +128,8 @@ int tune_class(ba_context *ctx, uint32_t log_n, int kind, const uint64_t *in, ui
                Timer &timer) {
   const bool n2b = kind != 0;
   const bool lde = kind == BA_TUNING_LDE_COSETS;
-  const uint32_t cols = (uint32_t)std::max<uint64_t>(1, elems >> log_n);
+  // an LDE's trial writes `elems` elements too, two cosets of half as many columns
+  const uint32_t cols = (uint32_t)std::max<uint64_t>(1, elems >> (log_n + lde));
   BaTuned best{};
   float best_ms = 1e30f;
   // the 4096-element-tile candidates are timed as such (tile_log 12) whatever the trial size
@@ -163,17 +170,33 @@ int tune_class(ba_context *ctx, uint32_t log_n, int kind, const uint64_t *in, ui
   }
   // then the latency-shaped passes (1024-element tiles, 4 elements per thread) for every batch
   // size of the class; if they lose, the class keeps the built-in rule (they still run batches of
-  // at most 2^20 elements, where they measured faster throughout)
-  bool lat = false;
-  if (!lde && ba_latency_shape_exists(log_n)) {
+  // at most 2^20 elements, where they measured faster throughout).  Columns of 2^11 and 2^12 run other
+  // kernels of them in calls (a whole column per workgroup) than in batch plans (two passes): they are
+  // kept for the class only where both are faster.
+  bool lat = !lde && ba_latency_shape_exists(log_n);
+  for (BaLatPolicy form : {BA_LAT_AUTO, BA_LAT_TUNED}) {
+    if (!lat) break;
     BaTuned e = best;
     e.tile_log = gl::ntt::LAT_TL;
     float ms = 0;
-    const int rc = time_entry(ctx, e, log_n, kind, in, out, cols, timer, ms);
+    const int rc = time_entry(ctx, e, log_n, kind, in, out, cols, timer, ms, form);
     if (rc) return rc;
     lat = ms < best_ms * 0.99f;
   }
   best.tile_log = lat ? gl::ntt::LAT_TL : 0;
+  // small LDEs: the plan against the built-in rule, on the largest batch that the rule gives the
+  // latency-shaped passes (where they gain least)
+  if (lde && ba_latency_shape_exists(log_n)) {
+    uint32_t small = cols;
+    while (small && !ba_small_batch(2ull * small, log_n)) small /= 2;
+    float by_plan = 0, by_size = 0;
+    BaTuned e = best;
+    int rc = small ? time_entry(ctx, e, log_n, kind, in, out, small, timer, by_plan) : BA_SUCCESS;
+    e.small_by_size = true;
+    if (small && rc == BA_SUCCESS) rc = time_entry(ctx, e, log_n, kind, in, out, small, timer, by_size);
+    if (rc) return rc;
+    best.small_by_size = by_size < by_plan;
+  }
   ctx->tuned[kind][log_n] = best;
   return BA_SUCCESS;
 }
@@ -194,7 +217,8 @@ extern "C" int ba_autotune(ba_context_t ctx, uint32_t log_n_min, uint32_t log_n_
     const uint64_t elems = std::max<uint64_t>(elems_per_trial, 1ull << log_n_max);
     uint64_t *in = nullptr, *out = nullptr;
     hipError_t err = hipMalloc(&in, elems * 8);
-    if (err == hipSuccess) err = hipMalloc(&out, elems * 8);
+    // room for two cosets of one column of the largest size
+    if (err == hipSuccess) err = hipMalloc(&out, std::max<uint64_t>(elems, 2ull << log_n_max) * 8);
     int rc = (int)err;
     const auto saved = std::vector<BaTuned>(&ctx->tuned[0][0], &ctx->tuned[0][0] + 3 * (BA_MAX_LOG_N + 1));
     if (rc == BA_SUCCESS) rc = ba_fill_uniform(in, elems, elems, 1, 0x7475u, stream);
