@@ -2,6 +2,7 @@
 and when it runs in a mix of concurrently submitted requests, and matches the oracle; admission
 keeps the arena within its budget; invalid requests are refused."""
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -312,3 +313,36 @@ def test_batches_hold_one_size_class(ba):
         assert st["failed"] == 0 and st["in_use_bytes"] == 0
     finally:
         srv.destroy()
+
+
+@pytest.mark.parametrize("idle_streams", [0, 1, 2, 3])
+def test_slots_run_beside_each_other(ba, idle_streams):
+    """Each slot's batch runs beside the others', whatever other streams the process has: with three large
+    batches in flight, a small request on the fourth slot completes before any of them."""
+    idle = [ba.CudaStream() for _ in range(idle_streams)]
+    srv = ba.serve.Server(ba._test_ctx, 72 << 30, 4)
+    try:
+        ran_apart = False
+        for trial in range(6):  # the first warms up; a trial whose requests shared a batch says nothing
+            log(f"slots side by side: {idle_streams} idle streams, trial {trial}")
+            tickets, at = [], []
+            for log_n, cols, lb in ((22, 128, 2), (22, 128, 2), (22, 128, 2), (12, 8, 1)):
+                at.append(time.perf_counter())
+                tickets.append(srv.submit(log_n, cols, lb, seed=trial))
+                time.sleep(0.003)
+            res = [srv.wait(t) for t in tickets]
+            assert all(r["status"] == 0 for r in res)
+            done = [t + r["latency_ms"] / 1e3 for t, r in zip(at, res)]
+            for t in tickets:
+                srv.release(t)
+            if trial == 0 or len({r["batch"] for r in res}) < 4:
+                continue
+            log(f"completed at {[round((d - at[0]) * 1e3, 2) for d in done]} ms")
+            assert done[3] < min(done[:3])
+            ran_apart = True
+            break
+        assert ran_apart
+    finally:
+        srv.destroy()
+        for s in idle:
+            s.destroy()
