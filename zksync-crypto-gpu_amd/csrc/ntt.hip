@@ -158,10 +158,14 @@ constexpr uint64_t kMaxGrid = 0x7FFFFFFFull;
 //   contiguous, 12 bits:  1792 tiles: 47 (1), 41 (2), 53 (4); 4096: 85, 85, 85, 104 (8); 6400: 127 (1),
 //                         126 (2), 134 (4); 8192: 175, 158, 150 (3), 162 (8); 16384: 459 (1), 358 (2),
 //                         307 (5), 313 (8).  From 14336 tiles on, 8 where that leaves a shorter last
-//                         group (19 columns of 2^22: 340 against 356 by 5) and 5 where it divides
-//                         (16 of 2^22: 287 against 307 by 8): workgroups of one length run in step,
-//                         all loading and all computing at once.  A transform's only pass (short
-//                         columns) takes 8: 16384 columns of 2^12 354 against 360 by 5.
+//                         group (19 columns of 2^22: 340 against 356 by 5) and 5 where 8 divides the
+//                         columns (16 of 2^22: 287 against 307 by 8; 32 of 2^21 282 against 294, inverse 283
+//                         against 301; 240 of 2^18 284 against 296).  Where 5 divides too it is as good or
+//                         better as well, within a run's noise (whole calls, 5 against 8: 80 of 2^20 629
+//                         and 637, inverse 678 and 690; 120 of 2^20 933 and 941, inverse 1019 and 1002; 40
+//                         of 2^21 708 and 709, inverse 738 and 751; 640 of 2^17 605 and 600, inverse 623
+//                         and 633).  A transform's only pass (short columns) takes 8: 16384 columns of
+//                         2^12 354 against 360 by 5.
 //   strided, plain top pass: hardly any set-up (one round without twiddles) and HBM-bound:
 //                         4 bits 2^26 elements: 180 (1), 189 (8); 5 bits 144 (1), 171 (4); 6 bits 184 (1),
 //                         209 (8); 7 bits 204 (1), 199 (2), 213 (8); 8 bits 2^27: 439 (1), 424 (2), 450 (8);
