@@ -326,3 +326,44 @@ def test_traced_lde_runs_the_calls_kernels(ba, log_n, cols, lb, inverse, coset):
     want = [f"void gl::ntt::ntt_pass_{k}({args['cosets' in k]})" for k in inverse + coset * (1 << lb)]
     assert names == want
     assert np.array_equal(got, gl_oracle.lde(ev, log_n, cols, lb, nthreads=8))
+
+
+# LDEs of at most 8 points run a whole transform per thread, all of up to 8 cosets in a launch.
+@pytest.mark.parametrize("log_n", [1, 2, 3])
+@pytest.mark.parametrize("cols,lb", [(1, 1), (7, 2), (255, 3), (257, 4), (2048, 5), (3, 7)])
+@pytest.mark.parametrize("layout", ["column", "coset"])
+def test_tiny_lde_cosets(ba, log_n, cols, lb, layout):
+    n = 1 << log_n
+    log(f"tiny lde log_n={log_n} cols={cols} blowup=2^{lb} {layout}")
+    ev = raw_u64(np.random.default_rng(cols + lb), cols * n)
+    got, ev_after, mono = run_lde(ba, ev, log_n, cols, lb, layout, keep_evals=True)
+    assert np.array_equal(got, gl_oracle.lde(ev, log_n, cols, lb, nthreads=8))
+    assert np.array_equal(mono, gl_oracle.batch_ntt(ev, log_n, cols, n, n, False, True, nthreads=8))
+    assert np.array_equal(ev_after, ev)
+
+
+def test_tiny_lde_takes_few_launches(ba):
+    """At blowup 64 an LDE of 2^3 points is 9 launches, as one of 2^4 is, and not 65, which took 10 times as
+    long as that one (the bound is 3)."""
+    import time
+
+    def best_us(log_n):
+        d_ev, d_out = ba.DeviceAllocation(100 << log_n), ba.DeviceAllocation(6400 << log_n)
+        try:
+            ba.runtime.fill_uniform(d_ev, 1 << log_n, 100, 1)
+            best = float("inf")
+            for _ in range(8):
+                ba.synchronize()
+                t0 = time.perf_counter()
+                for _ in range(20):
+                    ba.lde.lde_batch(ba._test_ctx, d_ev, log_n, 100, 6, d_out)
+                ba.synchronize()
+                best = min(best, (time.perf_counter() - t0) / 20 * 1e6)
+            return best
+        finally:
+            d_ev.free()
+            d_out.free()
+
+    tiny, small = best_us(3), best_us(4)
+    log(f"blowup 64, 100 columns: 2^3 {tiny:.0f} us, 2^4 {small:.0f} us")
+    assert tiny < 3 * small

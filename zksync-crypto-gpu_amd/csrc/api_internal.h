@@ -113,7 +113,9 @@ enum BaLatPolicy { BA_LAT_NEVER = 0, BA_LAT_TUNED = 1, BA_LAT_AUTO = 2 };
 // launches will run beside other streams' work (serve batches), so strided passes whose default
 // build runs four waves per SIMD, filling a CU's LDS, take their three-waves build.  cosets: that
 // many NTTs of the same shape run in each launch (an LDE call's cosets), which the choices that
-// depend on the size of a launch count.
+// depend on the size of a launch count.  in_bitrev_gather (natural -> bit-reversed forward only): the
+// input holds each column in bit-reversed order and the first pass gathers it (by coset_kernel, or grouped),
+// so that bit-reversed monomials feed a coset NTT without a separate permutation.
 int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint32_t log_n,
                  uint32_t num_cols, uint64_t stride_in, uint64_t stride_out, bool bitrev_inputs,
                  bool inverse, uint32_t log_ext, uint32_t coset_idx, bool in_bitrev_gather,
@@ -133,12 +135,6 @@ bool ba_use_latency_passes(const ba_context *ctx, uint32_t log_n, bool n2b, uint
 // Launches them one after another on `stream` (single-batch kernels).
 int ba_run_launches(const std::vector<BaPassLaunch> &launches, hipStream_t stream);
 
-// A pass launch tagged with its dependency level inside a batch plan: every launch at level l
-// only reads what launches at levels < l wrote.
-struct BaLeveledLaunch {
-  uint32_t level;
-  BaPassLaunch launch;
-};
 // A batch plan as data: grouped launches (one per dependency level and pass shape) and the
 // tables they read, laid out for one device allocation of `bytes` bytes.
 struct BaGroup {
@@ -171,11 +167,7 @@ hipError_t ba_plan_launch_group(const BaGroup &g, const void *device, const BaPl
 int ba_validate_lde(uint64_t *evals, uint64_t in_stride, uint64_t *monomials, uint64_t *out,
                     uint64_t out_col_stride, uint64_t out_coset_stride, uint32_t log_n,
                     uint32_t num_cols, uint32_t log_blowup);
-int ba_build_lde(const ba_context *ctx, uint64_t *evals, uint64_t in_stride, uint64_t *monomials,
-                 uint64_t *out, uint64_t out_col_stride, uint64_t out_coset_stride, uint32_t log_n,
-                 uint32_t num_cols, uint32_t log_blowup, std::vector<BaLeveledLaunch> &launches,
-                 uint32_t first_level);
-// Enqueues the coset NTTs of an LDE call (log_n >= 4) from its bit-reversed monomials: each pass as one
+// Enqueues the coset NTTs of an LDE call from its bit-reversed monomials: each pass as one
 // launch over up to 8 cosets, or with `apart` over one, by the same kernels.
 int ba_launch_lde_cosets(const ba_context *ctx, const uint64_t *mono, uint64_t mono_stride, uint64_t *out,
                          uint64_t out_col_stride, uint64_t out_coset_stride, uint32_t log_n, uint32_t num_cols,
@@ -183,13 +175,10 @@ int ba_launch_lde_cosets(const ba_context *ctx, const uint64_t *mono, uint64_t m
 int ba_validate_ntt(uint32_t log_n, uint64_t stride_in, uint64_t stride_out, uint32_t log_ext,
                     uint32_t coset_idx);
 
-// Enqueues one batch NTT (arguments already validated).  in_bitrev_gather (natural -> bitrev
-// forward only): the input holds each column in bit-reversed order and the first pass gathers
-// it, so a bit-reversed monomial vector feeds a coset NTT without a separate permutation.
+// Enqueues one batch NTT (arguments already validated).
 int ba_launch_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint32_t log_n,
                   uint32_t num_cols, uint64_t stride_in, uint64_t stride_out, bool bitrev_inputs,
-                  bool inverse, uint32_t log_ext, uint32_t coset_idx, hipStream_t stream,
-                  bool in_bitrev_gather = false);
+                  bool inverse, uint32_t log_ext, uint32_t coset_idx, hipStream_t stream);
 
 // Launch tracing: when a host thread has called ba_profile_begin, every kernel the library
 // launches from that thread is bracketed by two of the caller's events.

@@ -90,35 +90,6 @@ int ba_validate_lde(uint64_t *evals, uint64_t in_stride, uint64_t *monomials, ui
   return BA_SUCCESS;
 }
 
-int ba_build_lde(const ba_context *ctx, uint64_t *evals, uint64_t in_stride, uint64_t *monomials,
-                 uint64_t *out, uint64_t out_col_stride, uint64_t out_coset_stride, uint32_t log_n,
-                 uint32_t num_cols, uint32_t log_blowup, std::vector<BaLeveledLaunch> &launches,
-                 uint32_t first_level) {
-  if (num_cols == 0) return BA_SUCCESS;
-  const uint64_t n = 1ull << log_n;
-  const uint32_t blowup = 1u << log_blowup;
-  uint64_t *mono = monomials ? monomials : evals;
-  const uint64_t mono_stride = monomials ? n : in_stride;
-  // monomials, bit-reversed: n2b inverse without coset factors
-  std::vector<BaPassLaunch> ls;
-  int rc = ba_build_ntt(ctx, evals, mono, log_n, num_cols, in_stride, mono_stride, false, true, 0, 0, false, ls);
-  if (rc) return rc;
-  uint32_t depth = 0;
-  for (const BaPassLaunch &l : ls) {
-    launches.push_back({first_level + (uint32_t)l.pass, l});
-    depth = std::max<uint32_t>(depth, (uint32_t)l.pass + 1);
-  }
-  for (uint32_t c = 0; c < blowup; c++) {
-    ls.clear();
-    rc = ba_build_ntt(ctx, mono, out + (uint64_t)c * out_coset_stride, log_n, num_cols, mono_stride,
-                      out_col_stride, false, false, log_blowup, bitrev_bits(c, log_blowup),
-                      /*in_bitrev_gather=*/true, ls);
-    if (rc) return rc;
-    for (const BaPassLaunch &l : ls) launches.push_back({first_level + depth + (uint32_t)l.pass, l});
-  }
-  return BA_SUCCESS;
-}
-
 // BOOJUM_AMD_LDE_SERIAL=1 in the environment (read once) launches every coset's passes on their own,
 // in order, so that a profiler's per-kernel figures are one transform's; so does launch tracing.  The
 // kernels and their launch choices are those of the merged launches.
@@ -132,14 +103,17 @@ static bool lde_serial() {
 
 // Each pass of the coset NTTs is merged over the cosets.  A small LDE is a few launches of
 // latency-shaped passes (13 x 2^14 at blowup 4: 29 us, 110 as ten launches of 52 workgroups over four
-// streams); a large one reads the monomials once for 8 cosets.
+// streams); a large one reads the monomials once for 8 cosets; one of at most 2^3 points at blowup 64 is 9
+// launches in place of 65.
 int ba_launch_lde_cosets(const ba_context *ctx, const uint64_t *mono, uint64_t mono_stride, uint64_t *out,
                          uint64_t out_col_stride, uint64_t out_coset_stride, uint32_t log_n, uint32_t num_cols,
                          uint32_t log_blowup, bool apart, hipStream_t stream) {
   std::vector<BaPassLaunch> ls;
   const uint32_t blowup = 1u << log_blowup;
   static_assert(gl::ntt::MAX_COSETS == 8, "cosets of one launch");
-  const uint32_t log_merged = std::min(log_blowup, 3u);
+  uint32_t log_merged = std::min(log_blowup, 3u);
+  // a transform per thread: at most 2^31 threads a launch
+  while (log_n < 4 && log_merged && ((uint64_t)num_cols << log_merged) > (1ull << 31)) log_merged--;
   const uint32_t log_at_once = apart ? 0 : log_merged, at_once = 1u << log_at_once;
   for (uint32_t c0 = 0; c0 < blowup; c0 += at_once) {
     ls.clear();
@@ -188,25 +162,15 @@ static int lde_run(ba_context_t ctx, uint64_t *evals, uint64_t in_stride, uint64
   if (hipGetDevice(&device) != hipSuccess || device != ctx->device) return BA_ERROR_INVALID_VALUE;
   uint64_t *mono = monomials ? monomials : evals;
   const uint64_t mono_stride = monomials ? (1ull << log_n) : in_stride;
-  if (log_n < 4) {  // whole transforms per thread
-    std::vector<BaLeveledLaunch> leveled;
-    rc = ba_build_lde(ctx, evals, in_stride, monomials, out, out_col_stride, out_coset_stride, log_n,
-                      num_cols, log_blowup, leveled, 0);
-    if (rc) return rc;
-    std::vector<BaPassLaunch> flat;
-    for (const BaLeveledLaunch &l : leveled) flat.push_back(l.launch);  // already in dependency order
-    rc = ba_run_launches(flat, (hipStream_t)stream);
-  } else {
-    // The inverse NTT is latency-shaped by size alone: a tile_log of 10 says that plain NTTs of the class
-    // take those passes whatever the batch, which costs a large LDE up to a third of its time (blowup 2,
-    // 128 columns of 2^18: 1000 us against 754; 2048 of 2^14: 753 against 660).
-    std::vector<BaPassLaunch> ls;
-    rc = ba_build_ntt(ctx, evals, mono, log_n, num_cols, in_stride, mono_stride, false, true, 0, 0, false, ls,
-                      ba_small_batch(num_cols, log_n) ? BA_LAT_AUTO : BA_LAT_NEVER);
-    if (rc || (rc = ba_run_launches(ls, (hipStream_t)stream))) return rc;
-    rc = ba_launch_lde_cosets(ctx, mono, mono_stride, out, out_col_stride, out_coset_stride, log_n, num_cols,
-                              log_blowup, ba_trace_active() || lde_serial(), (hipStream_t)stream);
-  }
+  // The inverse NTT is latency-shaped by size alone: a tile_log of 10 says that plain NTTs of the class
+  // take those passes whatever the batch, which costs a large LDE up to a third of its time (blowup 2,
+  // 128 columns of 2^18: 1000 us against 754; 2048 of 2^14: 753 against 660).
+  std::vector<BaPassLaunch> ls;
+  rc = ba_build_ntt(ctx, evals, mono, log_n, num_cols, in_stride, mono_stride, false, true, 0, 0, false, ls,
+                    ba_small_batch(num_cols, log_n) ? BA_LAT_AUTO : BA_LAT_NEVER);
+  if (rc || (rc = ba_run_launches(ls, (hipStream_t)stream))) return rc;
+  rc = ba_launch_lde_cosets(ctx, mono, mono_stride, out, out_col_stride, out_coset_stride, log_n, num_cols,
+                            log_blowup, ba_trace_active() || lde_serial(), (hipStream_t)stream);
   if (rc || !natural_monomials) return rc;
   return ba_bit_reverse_in_place(mono, mono_stride, log_n, num_cols, stream);
 }

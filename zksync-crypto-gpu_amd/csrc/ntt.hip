@@ -142,6 +142,24 @@ struct CosetNames {
     }
   }
 };
+// and for whole transforms per thread
+struct TinyNames {
+  char n[4][2][2][80], cosets[4][80];  // [log_n][n2b][inverse]
+  TinyNames() {
+    static const char *tf[2] = {"false", "true"};
+    for (int k = 0; k < 4; k++) {
+      for (int d = 0; d < 2; d++)
+        for (int i = 0; i < 2; i++)
+          snprintf(n[k][d][i], sizeof(n[k][d][i]), "void gl::ntt::ntt_tiny<%d, %s, %s>(gl::ntt::PassArgs)", k, tf[d], tf[i]);
+      snprintf(cosets[k], sizeof(cosets[k]), "void gl::ntt::ntt_tiny_cosets<%d>(gl::ntt::CosetArgs)", k);
+    }
+  }
+};
+const char *tiny_name(uint32_t log_n, bool n2b, bool inverse, bool cosets) {
+  static const TinyNames names;
+  return cosets ? names.cosets[log_n] : names.n[log_n][n2b][inverse];
+}
+
 const char *coset_name(bool contig, uint32_t S, uint32_t waves) {
   static const CosetNames names;
   return names.n[!contig ? 0 : waves == 4 ? 2 : 1][S];
@@ -286,7 +304,11 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
     l.args.in_bitrev = in_bitrev_gather;
     l.kernels = ba_pick_tiny(log_n, n2b, inverse);
     l.grid = (num_cols + THREADS - 1) / THREADS;
-    l.name = "ntt_tiny";
+    l.name = tiny_name(log_n, n2b, inverse, false);
+    if (in_bitrev_gather) {
+      l.coset_kernel = ba_pick_tiny_cosets(log_n);
+      l.coset_name = tiny_name(log_n, n2b, inverse, true);
+    }
     l.pass = 0;
     l.col0 = 0;
     launches.push_back(l);
@@ -418,7 +440,7 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
       const uint32_t waves = S < 9 ? 3 : tuning.valid && tuning.contig_waves ? tuning.contig_waves : 4;
       l.kernels = pick_kernel(contig, S, n2b, inverse, top, scale, big, gather, waves, shared);
       const bool shared_build =
-          shared && !contig && l.kernels.single != pick_kernel(contig, S, n2b, inverse, top, scale, big, gather, waves, false).single;
+          shared && !contig && l.kernels.group != pick_kernel(contig, S, n2b, inverse, top, scale, big, gather, waves, false).group;
       l.name = kernel_name(contig, S, n2b, inverse, contig ? big : top, scale, gather, waves, shared_build);
       if (a.in_bitrev) {
         l.coset_kernel = !contig      ? ba_pick_strided_cosets(S)
@@ -429,7 +451,7 @@ int ba_build_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint3
       }
       l.pass = p;
       l.col0 = c0;
-      if (!l.kernels.single || (a.in_bitrev && !l.coset_kernel)) return BA_ERROR_INVALID_VALUE;
+      if (!l.kernels.group || (a.in_bitrev && !l.coset_kernel)) return BA_ERROR_INVALID_VALUE;
       launches.push_back(l);
     }
   }
@@ -449,11 +471,10 @@ int ba_run_launches(const std::vector<BaPassLaunch> &launches, hipStream_t strea
 
 int ba_launch_ntt(const ba_context *ctx, const uint64_t *in, uint64_t *out, uint32_t log_n,
                   uint32_t num_cols, uint64_t stride_in, uint64_t stride_out, bool bitrev_inputs,
-                  bool inverse, uint32_t log_ext, uint32_t coset_idx, hipStream_t stream,
-                  bool in_bitrev_gather) {
+                  bool inverse, uint32_t log_ext, uint32_t coset_idx, hipStream_t stream) {
   std::vector<BaPassLaunch> launches;
   const int rc = ba_build_ntt(ctx, in, out, log_n, num_cols, stride_in, stride_out, bitrev_inputs,
-                              inverse, log_ext, coset_idx, in_bitrev_gather, launches, BA_LAT_AUTO);
+                              inverse, log_ext, coset_idx, false, launches, BA_LAT_AUTO);
   if (rc) return rc;
   return ba_run_launches(launches, stream);
 }

@@ -13,8 +13,6 @@ typedef void (*BaCosetKernel)(gl::ntt::CosetArgs);
 struct BaKernels {
   BaPassKernel single;
   BaGroupKernel group;
-  bool operator==(const BaKernels &o) const { return single == o.single; }
-  bool operator<(const BaKernels &o) const { return (void *)single < (void *)o.single; }
 };
 
 // contiguous pass over bits [0, S), 4 <= S <= 8 / 9 <= S <= 12; scale: 0 none, 1 one factor
@@ -38,8 +36,10 @@ const char *ba_lat_cosets_kernel_name(uint32_t S, bool strided);
 const char *ba_lat_wide_kernel_name(uint32_t S, bool n2b, bool inverse, bool scale);
 const char *ba_lat_wide_cosets_kernel_name(uint32_t S);
 
-// the first pass of several coset NTTs of an LDE (gathered, coset-scaled n2b forward): strided over
-// 4..8 bits; contiguous over the whole column of 4..8 / 9..12 bits (waves 4 or 3); latency-shaped
+// the first pass of several coset NTTs of an LDE (gathered, coset-scaled n2b forward): the whole
+// transform of log_n <= 3 per thread; strided over 4..8 bits; contiguous over the whole column of 4..8 /
+// 9..12 bits (waves 4 or 3); latency-shaped
+BaCosetKernel ba_pick_tiny_cosets(uint32_t log_n);
 BaCosetKernel ba_pick_strided_cosets(uint32_t S);
 BaCosetKernel ba_pick_contig_lo_cosets(uint32_t S);
 BaCosetKernel ba_pick_contig_hi_cosets(uint32_t S);

@@ -1074,6 +1074,14 @@ template <int K, bool N2B, bool INV>
 __global__ __launch_bounds__(THREADS) void ntt_tiny(PassArgs a) {
   tiny_body<K, N2B, INV>(a, blockIdx.x);
 }
+// every coset's whole transform of an LDE, several cosets
+template <int K>
+__global__ __launch_bounds__(THREADS) void ntt_tiny_cosets(CosetArgs c) {
+  PassArgs a;
+  u32 tiles;
+  const u32 tile = enter_coset(c, a, tiles);
+  tiny_body<K, true, false>(a, tile);
+}
 template <int K, bool N2B, bool INV>
 __global__ __launch_bounds__(THREADS) void ntt_tiny_group(const PassArgs *jobs, const u32 *wg_start, u32 njobs) {
   const u32 j = group_of(wg_start, njobs, blockIdx.x);

@@ -5,15 +5,24 @@
 using namespace gl::ntt;
 
 // shared: the launch shares the GPU with other streams' work; a four-waves variant then comes in
-// its three-waves build (ntt_pass_strided_shared), the others are the same either way
+// its three-waves build (ntt_pass_strided_shared), the others are the same either way.  The gathered
+// pass's single launches are the coset kernels below.
 template <int S, bool N2B, bool INV, bool TOP, bool SCALE, bool GATHER>
 static BaKernels pair(bool shared) {
-  if constexpr (strided_four_waves<S, TOP, GATHER>()) {
-    if (shared)
-      return {ntt_pass_strided_shared<S, N2B, INV, TOP, SCALE, GATHER>,
-              ntt_pass_strided_shared_group<S, N2B, INV, TOP, SCALE, GATHER>};
+  constexpr bool SHARED_BUILD = strided_four_waves<S, TOP, GATHER>();
+  if constexpr (GATHER) {
+    if constexpr (SHARED_BUILD) {
+      if (shared) return {nullptr, ntt_pass_strided_shared_group<S, N2B, INV, TOP, SCALE, GATHER>};
+    }
+    return {nullptr, ntt_pass_strided_group<S, N2B, INV, TOP, SCALE, GATHER>};
+  } else {
+    if constexpr (SHARED_BUILD) {
+      if (shared)
+        return {ntt_pass_strided_shared<S, N2B, INV, TOP, SCALE, GATHER>,
+                ntt_pass_strided_shared_group<S, N2B, INV, TOP, SCALE, GATHER>};
+    }
+    return {ntt_pass_strided<S, N2B, INV, TOP, SCALE, GATHER>, ntt_pass_strided_group<S, N2B, INV, TOP, SCALE, GATHER>};
   }
-  return {ntt_pass_strided<S, N2B, INV, TOP, SCALE, GATHER>, ntt_pass_strided_group<S, N2B, INV, TOP, SCALE, GATHER>};
 }
 
 // the gathered top pass (LDE coset NTTs) exists for 4..8 bits only
@@ -64,6 +73,10 @@ BaKernels ba_pick_tiny(uint32_t log_n, bool n2b, bool inverse) {
   BA_TINY(3)
 #undef BA_TINY
   return {nullptr, nullptr};
+}
+
+BaCosetKernel ba_pick_tiny_cosets(uint32_t log_n) {
+  return log_n == 1 ? ntt_tiny_cosets<1> : log_n == 2 ? ntt_tiny_cosets<2> : log_n == 3 ? ntt_tiny_cosets<3> : nullptr;
 }
 
 BaCosetKernel ba_pick_strided_cosets(uint32_t S) {

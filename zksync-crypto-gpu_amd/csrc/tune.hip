@@ -106,13 +106,11 @@ int time_entry(ba_context *ctx, const BaTuned &entry, uint32_t log_n, int kind, 
                uint32_t cols, Timer &timer, float &ms, BaLatPolicy lat = BA_LAT_AUTO) {
   ctx->tuned[kind][log_n] = entry;
   const uint64_t n = 1ull << log_n;
-  const bool lde = kind == BA_TUNING_LDE_COSETS;
-  if (lde && log_n >= 4)
+  if (kind == BA_TUNING_LDE_COSETS)
     return timer.time(
         [&] { return ba_launch_lde_cosets(ctx, in, n, out, 2 * n, n, log_n, cols, 1, false, timer.stream); }, ms);
   std::vector<BaPassLaunch> ls;
-  const int rc = lde ? ba_build_ntt(ctx, in, out, log_n, cols, n, n, false, false, 1, 1, true, ls, BA_LAT_NEVER)
-                     : ba_build_ntt(ctx, in, out, log_n, cols, n, n, kind == 0, false, 0, 0, false, ls, lat);
+  const int rc = ba_build_ntt(ctx, in, out, log_n, cols, n, n, kind == 0, false, 0, 0, false, ls, lat);
   if (rc) return rc;
   return timer.time([&] { return ba_run_launches(ls, timer.stream); }, ms);
 }
