@@ -184,12 +184,17 @@ constexpr uint64_t kMaxGrid = 0x7FFFFFFFull;
 //                         of 2^21 708 and 709, inverse 738 and 751; 640 of 2^17 605 and 600, inverse 623
 //                         and 633).  A transform's only pass (short columns) takes 8: 16384 columns of
 //                         2^12 354 against 360 by 5.
+//   contiguous, at most 8 bits: hardly any set-up.  4 bits: 1613 tiles 38 (1), 45 (2); 2100: 42, 47; 2600: 51,
+//                         50; 3200: 64, 68; 4000: 78, 71; 7 bits: 47, 55; 54, 58; 64, 65; 80, 84; 97, 89.  With a
+//                         factor per element the set-up is longer: 4 bits, 2048 tiles 63 (1), 60 (2).
 //   strided, plain top pass: hardly any set-up (one round without twiddles) and HBM-bound:
 //                         4 bits 2^26 elements: 180 (1), 189 (8); 5 bits 144 (1), 171 (4); 6 bits 184 (1),
 //                         209 (8); 7 bits 204 (1), 199 (2), 213 (8); 8 bits 2^27: 439 (1), 424 (2), 450 (8);
 //                         below the top, 6 bits: 198 (1), 181 (3), 191 (8).
 //   strided, one factor for every element (n^-1): 4 bits 185 (1), 204 (8); 5 bits 177 (1), 158 (3), 176 (8);
-//                         8 bits 257 (1), 242 (2..8).
+//                         8 bits 257 (1), 242 (2..8).  Few tiles want all the workgroups (whole calls):
+//                         6 bits, 384 tiles 33 (1), 41 (3); 1024: 48, 53; 1536: 65, 66; 2048: 79, 79; 8 bits,
+//                         768 tiles 43, 50; 1536: 68, 70; 2048: 83, 78.
 //   strided, 9 bits, any factor: 8192 tiles 336 (1), 330 (2), 345 (3), 333 (4), 355 (8); 6656: 274, 277,
 //                         286, 289, 309; 12288: 491 (1), 477 (2), 473 (4), 485 (8); with a coset 532,
 //                         500, 482, 486.
@@ -201,13 +206,14 @@ static uint32_t pick_reps(bool contig, uint32_t S, bool top, int scale, uint64_t
                           bool only_pass) {
   uint32_t reps;
   if (contig) {
-    reps = tiles < 1536 ? 1 : tiles < 7168 ? 2 : tiles < 14336 ? 3 : only_pass || cols % 8 ? 8 : 5;
+    const uint32_t one = S > 8 ? 1536 : scale == 2 ? 2048 : 2560;  // below that many tiles
+    reps = tiles < one ? 1 : tiles < 7168 ? 2 : tiles < 14336 ? 3 : only_pass || cols % 8 ? 8 : 5;
   } else if (scale && S >= 9) {
     reps = tiles <= 8192 ? 2 : 4;
   } else if (scale == 2) {
     reps = std::min<uint32_t>(S == 4 ? 4 : S == 5 ? 5 : 7, (uint32_t)std::min<uint64_t>(8, tiles / 768));
   } else if (scale == 1) {
-    reps = S == 4 ? 1 : 3;
+    reps = S == 4 || tiles < 2048 ? 1 : 3;
   } else {
     reps = !top ? 3 : S <= 6 ? 1 : 2;
   }
