@@ -536,3 +536,34 @@ def test_few_tiles_keep_their_workgroups(ba, log_n, cols, bitrev, inverse):
         ctx.destroy()
     log(f"2^{log_n} x {cols}: built-in {best[0]:.1f} us, 1 column per workgroup {best[1]:.1f} us")
     assert best[0] < 1.1 * best[1]
+
+
+@pytest.mark.parametrize("log_n", [4, 5, 7])
+def test_short_columns_with_coset_factors(ba, log_n):
+    """8192 tiles of short columns scaled by the coset: the built-in columns per workgroup (two) against
+    three, which took 1.05 to 1.18 times as long; results in both against the oracle on sampled columns."""
+    import time
+    n, cols = 1 << log_n, 1 << (25 - log_n)
+    ctx = ba.Context.create(12, 12)
+    d_in, d_out = ba.DeviceAllocation(n * cols), ba.DeviceAllocation(n * cols)
+    ba.runtime.fill_uniform(d_in, n, cols, 1)
+    best = {0: float("inf"), 3: float("inf")}
+    sample = 3 * (4096 // n) + 1
+    try:
+        want = gl_oracle.batch_ntt(d_in.to_host()[:n * sample], log_n, sample, n, n, True, True, 1, 1, nthreads=8)
+        for _ in range(6):
+            for reps in best:
+                ba.tune.set_plan(ctx, log_n, True, [log_n], [reps], tile_log=12)
+                for timed in (False, True):
+                    t0 = time.perf_counter()
+                    for _ in range(10 if timed else 1):
+                        ba.ntt.batch_ntt_ctx(ctx, d_in.ptr, d_out.ptr, log_n, cols, n, n, True, True, 1, 1)
+                    ba.synchronize()
+                best[reps] = min(best[reps], (time.perf_counter() - t0) / 10 * 1e6)
+                assert np.array_equal(d_out.sub(0, n * sample).to_host(), want)
+    finally:
+        d_in.free()
+        d_out.free()
+        ctx.destroy()
+    log(f"2^{log_n} x {cols} with a coset: built-in {best[0]:.0f} us, 3 columns per workgroup {best[3]:.0f} us")
+    assert best[0] < 0.98 * best[3]

@@ -186,7 +186,10 @@ constexpr uint64_t kMaxGrid = 0x7FFFFFFFull;
 //                         2^12 354 against 360 by 5.
 //   contiguous, at most 8 bits: hardly any set-up.  4 bits: 1613 tiles 38 (1), 45 (2); 2100: 42, 47; 2600: 51,
 //                         50; 3200: 64, 68; 4000: 78, 71; 7 bits: 47, 55; 54, 58; 64, 65; 80, 84; 97, 89.  With a
-//                         factor per element the set-up is longer: 4 bits, 2048 tiles 63 (1), 60 (2).
+//                         factor per element the set-up is longer, and half as many workgroups run at once: 4
+//                         bits, 2048 tiles 66 (1), 58 (2); 4096: 124, 109, 119 (3), 110 (8); 8192: 342, 269, 318,
+//                         312; 7 bits, 8192 tiles 394, 330, 355, 337; 11500: 560, 482, 485, 493; 16384: 796, 680,
+//                         680, 668.
 //   strided, plain top pass: hardly any set-up (one round without twiddles) and HBM-bound:
 //                         4 bits 2^26 elements: 180 (1), 189 (8); 5 bits 144 (1), 171 (4); 6 bits 184 (1),
 //                         209 (8); 7 bits 204 (1), 199 (2), 213 (8); 8 bits 2^27: 439 (1), 424 (2), 450 (8);
@@ -207,7 +210,8 @@ static uint32_t pick_reps(bool contig, uint32_t S, bool top, int scale, uint64_t
   uint32_t reps;
   if (contig) {
     const uint32_t one = S > 8 ? 1536 : scale == 2 ? 2048 : 2560;  // below that many tiles
-    reps = tiles < one ? 1 : tiles < 7168 ? 2 : tiles < 14336 ? 3 : only_pass || cols % 8 ? 8 : 5;
+    const uint32_t two = S <= 7 && scale == 2 ? 14336 : 7168;
+    reps = tiles < one ? 1 : tiles < two ? 2 : tiles < 14336 ? 3 : only_pass || cols % 8 ? 8 : 5;
   } else if (scale && S >= 9) {
     reps = tiles <= 8192 ? 2 : 4;
   } else if (scale == 2) {
