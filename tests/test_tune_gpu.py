@@ -567,3 +567,18 @@ def test_short_columns_with_coset_factors(ba, log_n):
         ctx.destroy()
     log(f"2^{log_n} x {cols} with a coset: built-in {best[0]:.0f} us, 3 columns per workgroup {best[3]:.0f} us")
     assert best[0] < 0.98 * best[3]
+
+
+def test_autotune_leaves_the_built_in_columns_open(ba):
+    """The tuner does not pin the columns per workgroup that the built-in rule takes at its trial size (8 for
+    short columns in 2^26 elements), which at other sizes differ."""
+    ctx = ba.Context.create(12, 12)
+    try:
+        ba.tune.autotune(ctx, 9, 12, elems_per_trial=1 << 26)
+        for log_n in range(9, 13):
+            for kind in (False, True, ba.tune.LDE_COSETS):
+                bits, reps = ba.tune.get_plan(ctx, log_n, kind)
+                log(f"tuned over 2^26 elements log_n={log_n} kind={kind}: {reps}")
+                assert bits == [log_n] and reps[0] in (0, 1, 2, 4)
+    finally:
+        ctx.destroy()

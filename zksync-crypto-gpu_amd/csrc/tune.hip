@@ -142,9 +142,18 @@ int tune_class(ba_context *ctx, uint32_t log_n, int kind, const uint64_t *in, ui
     if (rc) return rc;
     if (ms < best_ms) best_ms = ms, best = e;
   }
-  // then the columns per workgroup of each pass in turn (0 = built-in choice, already timed)
+  // then the columns per workgroup of each pass in turn (0 = built-in choice, already timed).  The number
+  // that the built-in rule takes at this size is not timed again: chosen for a difference of clocks, it
+  // would hold at every size, where the rule takes fewer (2^26-element trials pinned 8 for short columns;
+  // 1448 columns of 2^10 then took 88 us instead of 16).
+  ctx->tuned[kind][log_n] = best;
+  std::vector<BaPassLaunch> built;
+  if (const int rc = ba_build_ntt(ctx, in, out, log_n, cols, 1ull << log_n, 1ull << log_n, kind == 0, false, lde, lde,
+                                  lde, built, BA_LAT_AUTO, false, 1u << lde))
+    return rc;
   for (int p = 0; p < best.plan.num_passes; p++) {
     for (uint32_t r : {1u, 2u, 4u, 8u}) {
+      if (r == built[p].args.reps) continue;
       BaTuned e = best;
       e.reps[p] = r;
       float ms = 0;
