@@ -61,8 +61,12 @@ struct ba_context {
   // Streams without work.  HIP opens hardware queues (4 by default) for a process's first streams and then
   // gives each new stream the queue that serves the fewest; only once all are open do the auxiliary
   // streams of a batch plan land on different ones.  In a process without other streams two of them
-  // shared a queue: a plan of 100 groups in 4 levels took 1144 us, with two or more idle streams 703.
-  static constexpr int kIdle = 4;
+  // shared a queue: a plan of 100 groups in 4 levels took 1144 us, and 703 once all were open.  Three,
+  // for with the null stream they are one per queue: the stream that a plan is launched on (the null
+  // stream, or one created before the plan) then shares its queue with the last of the plan's
+  // auxiliary streams, which has the smallest groups (96 uneven jobs: 640 us; with 4, 5 or 6 of them
+  // it is one with larger groups, 672, 710 and 730).
+  static constexpr int kIdle = 3;
   hipStream_t idle[kIdle] = {};
 };
 
