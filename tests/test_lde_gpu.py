@@ -236,6 +236,8 @@ def test_context_outlives_its_users(ba):
         ctx.destroy()
 
 
+# (The cosets no longer fork onto streams of their own: at blowup 4 each pass of the coset NTTs is one
+# launch on the capturing stream, at blowup 16 two.)
 @pytest.mark.parametrize("lb", [2, 4])
 def test_lde_graph_replay(ba, lb):
     """The LDE captured as a hipGraph (as the benchmark runs it) gives the eager result on every

@@ -291,6 +291,8 @@ def test_batch_plan_takes_tuned_tiles(ba):
             ba.tune.set_plan(ba._test_ctx, log_n, br, None)
 
 
+# (The cosets no longer fork onto streams of their own: each pass of the coset NTTs is one launch over
+# all of them, on the caller's stream.)
 @pytest.mark.parametrize("log_n,bits", [(14, [9, 5]), (14, [10, 4]), (17, [9, 8]), (17, [9, 4, 4]), (20, [12, 4, 4]),
                                          (20, [11, 5, 4])])
 def test_lde_coset_plans_bit_exact(ba, log_n, bits):

@@ -29,10 +29,6 @@ namespace {
 using gl::u32;
 using gl::u64;
 
-struct Ext {
-  u64 a, b;
-};
-
 constexpr u32 kThreads = 256;
 constexpr u32 kLogInvBatch = 3;
 
@@ -291,7 +287,7 @@ __global__ __launch_bounds__(kEvalThreads) void partial_kernel(const u64 *ys, co
 }
 
 // evals[col] = sum over chunks of partial[chunk, col], one wave per (column, plane); extension results
-// interleaved (c0, c1).  A lane sums the words of its chunks in 64 bits (at most 2^18 chunks).
+// interleaved (c0, c1).  A lane sums the words of its chunks in 64 bits (2^31 values are 2^19 chunks, 2^13 a lane).
 __global__ __launch_bounds__(64) void final_kernel(const u64 *partial, u32 chunks, u64 *evals) {
   const u64 *p = partial + (u64)blockIdx.x * chunks;
   u64 l = 0, h = 0;

@@ -1,6 +1,7 @@
 // ntt_inst.h -- launch-side handles to the pass kernel instantiations, which are spread over
 // several translation units (ntt_contig_lo.hip, ntt_contig_hi.hip, ntt_strided.hip) so they
-// compile in parallel.  Every pass shape has a single-batch kernel and a grouped kernel.
+// compile in parallel.  Every pass shape has a single-batch kernel and a grouped kernel; the gathered
+// strided pass has its grouped kernel and the coset kernels below.
 #pragma once
 
 #include "ntt_kernels.h"

@@ -1045,11 +1045,11 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 3)))
   const u32 j = group_of(wg_start, njobs, blockIdx.x);
   strided_body<S, N2B, INV, TOP, SCALE, GATHER, true>(jobs[j], blockIdx.x - wg_start[j]);
 }
-// W: waves per SIMD the contiguous pass is compiled for.  4: no prefetch, 128 registers (fastest
-// per launch over many tiles); 3: with the next-tile prefetch (fewer instructions per tile, better
-// when few workgroups run, and it leaves LDS room for a concurrent launch).  The per-element-
-// scaled variants over short columns keep 16 more values per thread and run at 2 either way.
-// The autotuner picks W per size class (ba_tuned_plan.contig_waves).
+// W: waves per SIMD the contiguous pass is compiled for.  4: no prefetch, 128 registers, the built-in
+// choice; 3: with the next-tile prefetch, which takes as long on up to 512 tiles and longer above (34.6
+// against 29.9 us on 1024), and leaves LDS room for a concurrent launch.  The per-element-scaled
+// variants over short columns keep 16 more values per thread and run at 2 either way.  The autotuner may
+// pick either W for a size class (ba_tuned_plan.contig_waves).
 template <int S, bool N2B, bool INV, int SC, bool WHOLE, int W>
 __global__ __launch_bounds__(THREADS, SC == 2 && !WHOLE ? 2 : W) void ntt_pass_contig(PassArgs a) {
   to_slice(a);

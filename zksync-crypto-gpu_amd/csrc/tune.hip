@@ -3,6 +3,7 @@
 // then the tile shape (4096-element tiles of 16 elements per thread against the latency-shaped
 // 1024-element tiles of 4), and keeps the fastest on the context.
 //
+// Plain NTTs of both input orders are timed, and the coset NTTs of an LDE call as the call launches them.
 // No reference counterpart: boojum-cuda's kernel shapes per log_n are fixed tables
 // (crates/boojum-cuda/src/ntt.rs:57-176).  The candidate splits are those the pass kernels
 // cover: one contiguous pass for log_n <= 12; otherwise a contiguous pass over 9..12 low bits
