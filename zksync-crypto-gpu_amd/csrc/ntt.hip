@@ -187,9 +187,10 @@ constexpr uint64_t kMaxGrid = 0x7FFFFFFFull;
 //   contiguous, at most 8 bits: hardly any set-up.  4 bits: 1613 tiles 38 (1), 45 (2); 2100: 42, 47; 2600: 51,
 //                         50; 3200: 64, 68; 4000: 78, 71; 7 bits: 47, 55; 54, 58; 64, 65; 80, 84; 97, 89.  With a
 //                         factor per element the set-up is longer, and half as many workgroups run at once: 4
-//                         bits, 2048 tiles 66 (1), 58 (2); 4096: 124, 109, 119 (3), 110 (8); 8192: 342, 269, 318,
-//                         312; 7 bits, 8192 tiles 394, 330, 355, 337; 11500: 560, 482, 485, 493; 16384: 796, 680,
-//                         680, 668.
+//                         bits, 1536 tiles 50 (1), 55 (2); 1700: 62, 56; 2048: 66, 58; 4096: 124, 109, 119 (3),
+//                         110 (8); 8192: 342, 269, 318, 312; 7 bits, 1536 tiles 59, 66; 1700: 74, 68; 8192: 394,
+//                         330, 355, 337; 11500: 560, 482, 485, 493; 16384: 796, 680, 680, 668; 8 bits, 1536 tiles
+//                         51, 53; 1700: 59, 56.
 //   strided, plain top pass: hardly any set-up (one round without twiddles) and HBM-bound:
 //                         4 bits 2^26 elements: 180 (1), 189 (8); 5 bits 144 (1), 171 (4); 6 bits 184 (1),
 //                         209 (8); 7 bits 204 (1), 199 (2), 213 (8); 8 bits 2^27: 439 (1), 424 (2), 450 (8);
@@ -209,7 +210,7 @@ static uint32_t pick_reps(bool contig, uint32_t S, bool top, int scale, uint64_t
                           bool only_pass) {
   uint32_t reps;
   if (contig) {
-    const uint32_t one = S > 8 ? 1536 : scale == 2 ? 2048 : 2560;  // below that many tiles
+    const uint32_t one = S > 8 ? 1536 : scale == 2 ? 1537 : 2560;  // below that many tiles
     const uint32_t two = S <= 7 && scale == 2 ? 14336 : 7168;
     reps = tiles < one ? 1 : tiles < two ? 2 : tiles < 14336 ? 3 : only_pass || cols % 8 ? 8 : 5;
   } else if (scale && S >= 9) {
