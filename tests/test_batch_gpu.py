@@ -2,6 +2,9 @@
 different sizes, orders, directions and cosets, and coset LDEs -- matches the oracle run on that
 job alone, plan after plan and replay after replay."""
 import ctypes
+import os
+import subprocess
+import sys
 import time
 
 import numpy as np
@@ -226,3 +229,39 @@ def test_groups_of_a_level_run_beside_each_other(ba):
         d_out.free()
     log(f"plan {stats}: {alone:.3f} ms alone, {beside:.3f} ms beside idle streams")
     assert alone < 1.27 * beside
+
+
+def test_context_leaves_queues_unopened():
+    """A context without batch plans opens no hardware queue beside the null stream's: from the second on
+    every kernel costs more (14 columns of 2^16 from bit-reversed order 24.0 us in a process without other
+    streams, 26.3 beside one; the bound is half way)."""
+    child = """
+import time
+import boojum_amd as ba
+ba.set_device(0)
+ctx = ba.Context.create(12, 12)
+n, cols = 1 << 16, 14
+d_in, d_out = ba.DeviceAllocation(n * cols), ba.DeviceAllocation(n * cols)
+ba.runtime.fill_uniform(d_in, n, cols, 1)
+
+def best_us():
+    best = float("inf")
+    for _ in range(12):
+        t0 = time.perf_counter()
+        for _ in range(40):
+            ba.ntt.batch_ntt_ctx(ctx, d_in.ptr, d_out.ptr, 16, cols, n, n, True, False)
+        ba.synchronize()
+        best = min(best, (time.perf_counter() - t0) / 40 * 1e6)
+    return best
+
+best_us()
+alone = best_us()
+s = ba.CudaStream()
+print(alone, best_us(), flush=True)
+"""
+    pkg = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "zksync-crypto-gpu_amd")
+    got = subprocess.run([sys.executable, "-c", child], env={**os.environ, "PYTHONPATH": pkg}, check=True,
+                         capture_output=True, text=True, timeout=100).stdout
+    alone, beside = (float(v) for v in got.split()[-2:])
+    log(f"2^16 x 14 alone {alone:.1f} us, beside a stream {beside:.1f} us")
+    assert alone < 0.96 * beside

@@ -58,15 +58,19 @@ struct ba_context {
   std::atomic<int> users{0};
   // Poseidon2 round constants (30 x 12, device memory), installed by the caller
   uint64_t *p2_round_constants = nullptr;
-  // Streams without work.  HIP opens hardware queues (4 by default) for a process's first streams and then
-  // gives each new stream the queue that serves the fewest; only once all are open do the auxiliary
-  // streams of a batch plan land on different ones.  In a process without other streams two of them
-  // shared a queue: a plan of 100 groups in 4 levels took 1144 us, and 703 once all were open.  Three,
-  // for with the null stream they are one per queue: the stream that a plan is launched on (the null
-  // stream, or one created before the plan) then shares its queue with the last of the plan's
-  // auxiliary streams, which has the smallest groups (96 uneven jobs: 640 us; with 4, 5 or 6 of them
-  // it is one with larger groups, 672, 710 and 730).
+  // Streams without work, made with the context's first batch plan.  HIP opens hardware queues (4 by
+  // default) for a process's first streams and then gives each new stream the queue that serves the
+  // fewest; only once all are open do the auxiliary streams of a batch plan land on different ones.  In a
+  // process without other streams two of them shared a queue: a plan of 100 groups in 4 levels took 1144
+  // us, and 703 once all were open.  Three, for with the null stream they are one per queue: the stream
+  // that a plan is launched on (the null stream, or one created before the plan) then shares its queue
+  // with the last of the plan's auxiliary streams, which has the smallest groups (96 uneven jobs: 640 us;
+  // with 4, 5 or 6 of them it is one with larger groups, 672, 710 and 730).  Not before the first plan:
+  // from the second queue on every kernel of the process costs more, for as long as it runs (14 columns of
+  // 2^16 from bit-reversed order 24.0 -> 26.3 us, a blowup-4 LDE of 181 of 2^12 42.6 -> 44.3, one opening
+  // of 2^22 16.3 -> 16.9).
   static constexpr int kIdle = 3;
+  std::once_flag idle_once;
   hipStream_t idle[kIdle] = {};
 };
 

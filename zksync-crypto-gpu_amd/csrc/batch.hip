@@ -242,6 +242,11 @@ extern "C" int ba_batch_plan_create(ba_context_t ctx, const ba_job *jobs, uint32
       delete p;
       return rc;
     }
+    std::call_once(ctx->idle_once, [ctx] {
+      for (hipStream_t &s : ctx->idle)
+        if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) s = nullptr;
+      (void)hipGetLastError();  // plans work without them
+    });
     hipError_t err = hipEventCreateWithFlags(&p->fork, hipEventDisableTiming);
     for (int i = 0; err == hipSuccess && i < ba_batch_plan::kAux; i++)
       err = hipStreamCreateWithFlags(&p->aux[i], hipStreamNonBlocking);

@@ -103,9 +103,6 @@ extern "C" int ba_context_create(uint32_t w_coarse_log, uint32_t g_coarse_log, b
     ctx->tab.g = {d + off_gf, d + off_gc, gf, (uint32_t)(n_gf - 1)};
     ctx->tab.g_inv = {d + off_if, d + off_ic, gf, (uint32_t)(n_gf - 1)};
     ctx->tab.inv_sizes = d + off_inv;
-    for (hipStream_t &s : ctx->idle)
-      if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) s = nullptr;
-    (void)hipGetLastError();  // the context works without them
     {
       std::lock_guard<std::mutex> lock(g_registry_mutex);
       g_live.push_back(ctx);
