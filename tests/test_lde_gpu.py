@@ -369,3 +369,34 @@ def test_tiny_lde_takes_few_launches(ba):
     tiny, small = best_us(3), best_us(4)
     log(f"blowup 64, 100 columns: 2^3 {tiny:.0f} us, 2^4 {small:.0f} us")
     assert tiny < 3 * small
+
+
+def test_tiny_lde_of_uneven_tiles(ba):
+    """2703 workgroups of columns of 2^1, blowup 2, take as long as 2704, a multiple of the XCDs: with a tile's
+    cosets on different XCDs they took 1.4 times as long (the bound is half way)."""
+    import time
+    most = 692224
+    d_ev, d_mono, d_out = (ba.DeviceAllocation(k * most) for k in (2, 2, 4))
+    best = {691802: float("inf"), most: float("inf")}
+    try:
+        ba.runtime.fill_uniform(d_ev, 2, most, 1)
+        for _ in range(8):
+            for cols in best:
+                for timed in (False, True):
+                    t0 = time.perf_counter()
+                    for _ in range(20 if timed else 2):
+                        ba.lde.lde_batch(ba._test_ctx, d_ev, 1, cols, 1, d_out, monomials=d_mono)
+                    ba.synchronize()
+                best[cols] = min(best[cols], (time.perf_counter() - t0) / 20 * 1e6)
+        ev = d_ev.sub(0, 2 * 691802).to_host()
+        d_out.copy_from_host(np.zeros(4 * most, dtype=np.uint64))
+        ba.lde.lde_batch(ba._test_ctx, d_ev, 1, 691802, 1, d_out, monomials=d_mono)
+        ba.synchronize()
+        got = d_out.to_host()
+    finally:
+        for d in (d_ev, d_mono, d_out):
+            d.free()
+    log(f"2^1 at blowup 2: {best}")
+    assert np.array_equal(got[:4 * 691802], gl_oracle.lde(ev, 1, 691802, 1, nthreads=8))
+    assert not got[4 * 691802:].any()
+    assert best[691802] < 1.2 * best[most]
