@@ -26,7 +26,7 @@ u32 grid_for(u64 count, u32 most = 65536) {
   return (u32)std::max<u64>(1, std::min<u64>((count + kThreads - 1) / kThreads, most));
 }
 // Kernels whose lanes step a power by the grid stride: fewer workgroups spread the first power over
-// more elements.  2^26 elements, omega shift and natural-order powers, us on one box: 65536 workgroups 263 and
+// more elements.  2^26 elements, omega shift and natural-order powers, us on one card: 65536 workgroups 263 and
 // 126, 16384 227 and 100, 4096 237 and 111.
 constexpr u32 kSteppedGrid = 16384;
 
@@ -143,7 +143,7 @@ __global__ __launch_bounds__(kThreads) void powers_ef_kernel(const u64 *base_ptr
 // The exponent (shift (i + offset)) << degree_shift is linear in i modulo 2^30: a lane's elements are a
 // grid stride apart and their factors step by one constant, omega^(+-((shift stride) << degree_shift)).
 // What bounds it: HBM (16 B per element).  A lane loads kShiftBatch elements before it multiplies any,
-// on a grid that fills the chip: 2^26 elements take 205 to 227 us by box (5.2 to 4.7 TB/s, a large copy's
+// on a grid that fills the chip: 2^26 elements take 205 to 227 us by card (5.2 to 4.7 TB/s, a large copy's
 // rate); one load, product and store at a time on four times the workgroups took 263 where it takes 227.
 constexpr u32 kShiftBatch = 4;
 __global__ __launch_bounds__(kThreads) void omega_shift_kernel(gl::Tables tab, const u64 *src, u32 log_degree,
